@@ -1,6 +1,6 @@
-// plane.hip -- matrix-core plane kernels for gfx950: H*X (FP64, FP32 and
-// split-BF16 forms) and the kinetic fast-diagonalisation preconditioner
-// (FP64 and split-BF16 forms).
+// plane.hip -- matrix-core plane kernels for gfx950: the split-BF16 forms of H*X
+// and of the kinetic fast-diagonalisation preconditioner, and the dispatch to
+// the FP64 and FP32 forms (plane_f.hip).
 //
 // Both operators are sums or products of dense 1-D matrices applied along the
 // axes of the x-fastest grid (g = i + nx*(j + ny*k)).  A workgroup (4 waves)
@@ -31,9 +31,7 @@
 //      1, plane (i,k) at j:  W = Qz (S o (Qz^T P)),  S = scale / (lam_x + lam_y + lam_z - shift)
 //      2, plane (i,j) at k:  t = (Qy P) Qx^T                     (W -> t)
 // with |lam_x + lam_y + lam_z - shift| floored at `floor`.
-#include "common.hpp"
-#include "fdm.hpp"
-#include "gmem.hpp"
+#include "plane.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -44,13 +42,6 @@ namespace pisces {
 namespace {
 
 constexpr int kPT = 256;
-
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // ------------------------------------------------------------------ helpers
 __device__ __forceinline__ uint16_t bf16_rne(float x)
@@ -76,136 +67,6 @@ __device__ __forceinline__ f32x4 mma_bf(bf16x8 a, bf16x8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f64x4 mma(double a, double b, f64x4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <typename T> struct Acc;
-template <> struct Acc<double> {
-    typedef f64x4 type;
-    __device__ static inline int row(int lq, int r) { return lq + 4 * r; }
-};
-template <> struct Acc<float> {
-    typedef f32x4 type;
-    __device__ static inline int row(int lq, int r) { return 4 * lq + r; }
-};
-
-// Plane geometry.  kind 0: plane (i,j) at fixed k (rows c = j); kind 1: plane
-// (i,k) at fixed j (rows c = k).
-struct Geo {
-    int ni, nc, npi, npc;
-    long long cs;     // global stride between rows
-    long long vbase;  // offset of (0, 0) within one vector
-    long long base;   // offset of (0, 0) including the vector offset
-    int pl;           // index of the plane along its normal axis
-};
-
-__device__ __forceinline__ bool geo_of(int kind, int nx, int ny, int nz, int nvec, long long ld,
-                                       int npi, int npc, int p, Geo &g)
-{
-    const int nplanes = kind == 0 ? nz : ny;
-    if (p >= nplanes * nvec) return false;
-    const int v = p / nplanes, pl = p - v * nplanes;
-    g.ni = nx;
-    g.npi = npi;
-    g.npc = npc;
-    g.pl = pl;
-    if (kind == 0) {
-        g.nc = ny;
-        g.cs = nx;
-        g.vbase = (long long)nx * ny * pl;
-    } else {
-        g.nc = nz;
-        g.cs = (long long)nx * ny;
-        g.vbase = (long long)nx * pl;
-    }
-    g.base = (long long)v * ld + g.vbase;
-    return true;
-}
-
-// ------------------------------------------------------------------ staging
-// Plane values as FP32 for items of 2 rows x 4 columns.
-template <typename S>
-__device__ __forceinline__ void load_item(const S *src_, const Geo &g, int c, int i, bool vec,
-                                          float (&x)[2][4])
-{
-    const gptr<const S> src = glb(src_) + g.base;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int cc = c + r;
-        const bool okc = cc < g.nc;
-        const gptr<const S> row = src + (okc ? (long long)cc * g.cs : 0);
-        if (vec && i + 4 <= g.ni) {
-            float y[4];
-            if (sizeof(S) == 4) {
-                const f32x4 v = *reinterpret_cast<gptr<const f32x4>>(row + i);
-                y[0] = v[0]; y[1] = v[1]; y[2] = v[2]; y[3] = v[3];
-            } else {
-                const f64x2 a = *reinterpret_cast<gptr<const f64x2>>(row + i);
-                const f64x2 b = *reinterpret_cast<gptr<const f64x2>>(row + i + 2);
-                y[0] = (float)a[0]; y[1] = (float)a[1]; y[2] = (float)b[0]; y[3] = (float)b[1];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) x[r][q] = okc ? y[q] : 0.f;
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const bool ok = okc && i + q < g.ni;
-                const float y = (float)row[ok ? i + q : 0];
-                x[r][q] = ok ? y : 0.f;
-            }
-        }
-    }
-}
-
-// FP32/FP64 plane into LDS, c-major, pitch npi + pad.
-template <typename T, typename S>
-__device__ void stage_f(const S *src, const Geo &g, bool vec, T *P, int pitch)
-{
-    const int nq = g.npi / 4, items = (g.npc / 2) * nq;
-    for (int it = threadIdx.x; it < items; it += kPT) {
-        const int c = 2 * (it / nq), i = 4 * (it - (it / nq) * nq);
-        if (sizeof(S) == 8 && sizeof(T) == 8) {
-            const gptr<const S> sg = glb(src) + g.base;
-            T y[2][4];
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int cc = c + r;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const bool ok = cc < g.nc && i + q < g.ni;
-                    const T v = (T)sg[ok ? (long long)cc * g.cs + i + q : 0];
-                    y[r][q] = ok ? v : T(0);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) P[(c + r) * pitch + i + q] = y[r][q];
-        } else {
-            float x[2][4];
-            load_item(src, g, c, i, vec, x);
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) P[(c + r) * pitch + i + q] = (T)x[r][q];
-        }
-    }
-}
-
-__device__ __forceinline__ bool vec_ok(const void *p, const Geo &g, int elems_per_16b)
-{
-    return ((reinterpret_cast<uintptr_t>(p) & 15) == 0) && (g.ni % 4 == 0) && (g.cs % 4 == 0) &&
-           (g.base % elems_per_16b == 0) && (elems_per_16b == 4 || g.base % 2 == 0);
-}
-
-// f64/f32 pitch: np + 2 doubles (odd number of 16-byte units per row) or np + 4 floats
-template <typename T> __host__ __device__ inline int fpitch(int np) { return sizeof(T) == 8 ? np + 2 : np + 4; }
 
 // ------------------------------------------------------------------ owned tiles (split-BF16 forms)
 // Wave w owns the 16-row tiles tc = w + 4u (u < NCT) of a plane and all of its
@@ -216,12 +77,6 @@ template <typename T> __host__ __device__ inline int fpitch(int np) { return siz
 // move HBM -> registers -> LDS without a layout change.  A workgroup walks the
 // planes p = blockIdx.x, blockIdx.x + gridDim.x, ... of one job; the loads of
 // the next plane are issued before the current one is contracted.
-// The middle pass of H*X (pass B) and of the preconditioner (pass 1) reads
-// what the pass before wrote: it walks its grid in reverse (workgroups are
-// dispatched in order of their linear index), starting on the data the
-// previous pass left last in the L2 and the memory-side cache.
-__device__ __forceinline__ int plane_x(bool rev) { return rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x; }
-__device__ __forceinline__ int plane_y(bool rev) { return rev ? gridDim.y - 1 - blockIdx.y : blockIdx.y; }
 
 template <int NPMAX> struct Own {
     static constexpr int NIT = NPMAX / 16;            // column tiles
@@ -655,364 +510,6 @@ __global__ void __launch_bounds__(kPT) hx_bf2_fused_kernel(const HxJob *__restri
     }
 }
 
-// ------------------------------------------------------------------ H*X, FP64 form
-// Owned tiles as above, in the f64 accumulator layout: lane (l16, lq) holds
-// rows lq + 4 r (r < 4) of column l16 in each of its wave's tiles.  The plane
-// is kept in LDS as FP64, c-major (pitch npi + 2 doubles); the along-c matrix
-// (A operand, rows of the wave's tiles) is held in registers, and in pass B
-// the along-i matrix Tx (B operand) is staged once per workgroup into LDS
-// next to the plane.  Each k-step feeds one A value to the MFMAs of all the
-// wave's column tiles (independent accumulator chains).
-template <int NCT, int NIT>
-__device__ __forceinline__ void own_load64(const double *src_, long long base, const Geo &g,
-                                           double (&x)[NCT][NIT][4])
-{
-    const gptr<const double> src = glb(src_) + base;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c = 16 * (wave + 4 * u) + lq + 4 * r;
-#pragma unroll
-            for (int v = 0; v < NIT; ++v) {
-                const int i = 16 * v + l16;
-                const bool ok = c < g.nc && i < g.ni;
-                const double y = src[ok ? (long long)c * g.cs + i : 0];
-                x[u][v][r] = ok ? y : 0.0;
-            }
-        }
-}
-
-template <int PASS, int NPMAX, bool MULTI>
-__global__ void __launch_bounds__(kPT) hx_f64_kernel(const HxJob *__restrict__ jobs)
-{
-    constexpr int NCT = Own<NPMAX>::NCT, NIT = Own<NPMAX>::NIT, KF = NPMAX / 4;
-    const HxJob &J = jobs[plane_y(PASS == 1)];
-    const AxisMats &Mi = J.ax[0];
-    const AxisMats &Mc = J.ax[PASS == 0 ? 1 : 2];
-    int p = plane_x(PASS == 1);
-    Geo g;
-    if (!geo_of(PASS, J.nx, J.ny, J.nz, J.nvec, J.ld, Mi.np, Mc.np, p, g)) return;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int pitch = g.npi + 2;
-    double *P = reinterpret_cast<double *>(smem);
-    double *Tl = P + g.npc * pitch;  // pass B: Tx, rows k, pitch npi + 2
-    const double *X = static_cast<const double *>(J.X);
-    const double *V = static_cast<const double *>(J.V);
-    const gptr<double> Y = glb(static_cast<double *>(J.Y));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16, ksc = g.npc / 4, ksi = g.npi / 4;
-    // along-c matrix in A form: ac[u][s] = Tc[16 tc + l16][4 s + lq]
-    double ac[NCT][KF];
-    {
-        const gptr<const double> Tc = glb(Mc.t64);
-#pragma unroll
-        for (int u = 0; u < NCT; ++u)
-#pragma unroll
-            for (int s = 0; s < KF; ++s) {
-                const int tc = wave + 4 * u;
-                const bool ok = tc < ntc && s < ksc;
-                const double y = Tc[ok ? (16 * tc + l16) * g.npc + 4 * s + lq : 0];
-                ac[u][s] = ok ? y : 0.0;
-            }
-    }
-    if (PASS == 1) {
-        const gptr<const double> Ti = glb(Mi.t64);
-        for (int e = threadIdx.x; e < g.npi * g.npi; e += kPT) {
-            const int k = e / g.npi, i = e - k * g.npi;
-            Tl[k * pitch + i] = Ti[e];
-        }
-    }
-    double xb[NCT][NIT][4], wb[NCT][NIT][4];  // X; V (pass A) or Y (pass B)
-    own_load64<NCT, NIT>(X, g.base, g, xb);
-    own_load64<NCT, NIT>(PASS == 0 ? V : static_cast<const double *>(J.Y), PASS == 0 ? g.vbase : g.base, g, wb);
-    for (;;) {
-#pragma unroll
-        for (int u = 0; u < NCT; ++u) {
-            const int tc = wave + 4 * u;
-            if (tc >= ntc) break;
-#pragma unroll
-            for (int v = 0; v < NIT; ++v) {
-                if (v >= nti) break;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    P[(16 * tc + lq + 4 * r) * pitch + 16 * v + l16] = xb[u][v][r];
-                    if (PASS == 0) wb[u][v][r] *= xb[u][v][r];
-                }
-            }
-        }
-        __syncthreads();
-        Geo gn;
-        const bool more = MULTI && geo_of(PASS, J.nx, J.ny, J.nz, J.nvec, J.ld, Mi.np, Mc.np, p + gridDim.x, gn);
-        if (more) own_load64<NCT, NIT>(X, gn.base, gn, xb);
-#pragma unroll
-        for (int u = 0; u < NCT; ++u) {
-            const int tc = wave + 4 * u;
-            if (tc >= ntc) break;
-            const int c0 = 16 * tc;
-            f64x4 acc[NIT];
-#pragma unroll
-            for (int v = 0; v < NIT; ++v)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[v][r] = PASS == 0 ? wb[u][v][r] : 0.0;
-            // along c: D(c, i) += sum_k Tc[c][k] P[k][i]
-#pragma unroll
-            for (int s = 0; s < KF; ++s) {
-                if (s >= ksc) break;
-                const double *pr = P + (4 * s + lq) * pitch + l16;
-#pragma unroll
-                for (int v = 0; v < NIT; ++v) {
-                    if (v >= nti) break;
-                    acc[v] = mma(ac[u][s], pr[16 * v], acc[v]);
-                }
-            }
-            // along i: D(c, i) += sum_k P[c][k] Tx[k][i]
-            if (PASS == 1) {
-#pragma unroll
-                for (int s = 0; s < KF; ++s) {
-                    if (s >= ksi) break;
-                    const double a = P[(c0 + l16) * pitch + 4 * s + lq];
-                    const double *tr = Tl + (4 * s + lq) * pitch + l16;
-#pragma unroll
-                    for (int v = 0; v < NIT; ++v) {
-                        if (v >= nti) break;
-                        acc[v] = mma(a, tr[16 * v], acc[v]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int v = 0; v < NIT; ++v) {
-                if (v >= nti) break;
-                const int i = 16 * v + l16;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int c = c0 + lq + 4 * r;
-                    if (c >= g.nc || i >= g.ni) continue;
-                    const long long row = (long long)c * g.cs;
-                    Y[g.base + row + i] = PASS == 0 ? acc[v][r] : wb[u][v][r] + acc[v][r];
-                    if (more) {
-                        const gptr<const double> W =
-                            PASS == 0 ? glb(V) + gn.vbase + row : (gptr<const double>)Y + gn.base + row;
-                        wb[u][v][r] = W[i];
-                    }
-                }
-            }
-        }
-        if (!more) break;
-        __syncthreads();  // every wave is done with this plane's LDS copy
-        g = gn;
-        p += gridDim.x;
-    }
-}
-
-// ------------------------------------------------------------------ H*X, FP32 form
-
-template <typename T> __device__ inline const T *tmat(const AxisMats &m);
-template <> __device__ inline const double *tmat<double>(const AxisMats &m) { return m.t64; }
-template <> __device__ inline const float *tmat<float>(const AxisMats &m) { return m.t32; }
-
-template <typename T, int PASS>
-__global__ void __launch_bounds__(kPT) hx_f_kernel(const HxJob *__restrict__ jobs)
-{
-    typedef typename Acc<T>::type acc_t;
-    const HxJob &J = jobs[blockIdx.y];
-    const AxisMats &Mi = J.ax[0];
-    const AxisMats &Mc = J.ax[PASS == 0 ? 1 : 2];
-    Geo g;
-    if (!geo_of(PASS, J.nx, J.ny, J.nz, J.nvec, J.ld, Mi.np, Mc.np, blockIdx.x, g)) return;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int pitch = fpitch<T>(g.npi);
-    T *P = reinterpret_cast<T *>(smem);
-    const T *X = static_cast<const T *>(J.X);
-    const gptr<T> Y = glb(static_cast<T *>(J.Y));
-    stage_f<T, T>(X, g, vec_ok(X, g, 16 / (int)sizeof(T)), P, pitch);
-    __syncthreads();
-    const gptr<const T> V = glb(static_cast<const T *>(J.V));
-    const gptr<const T> Tc = glb(tmat<T>(Mc)), Ti = glb(tmat<T>(Mi));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16;
-    for (int tc = wave; tc < ntc; tc += 4) {
-        const int c0 = 16 * tc;
-        for (int ti = 0; ti < nti; ti += 2) {
-            const int i0 = 16 * ti, i1 = i0 + 16;
-            acc_t a0 = {}, a1 = {};
-            // along c: A[m][k] = Tc[c0 + m][k], B[k][n] = P[k][i + n]
-            const gptr<const T> tcr = Tc + (c0 + l16) * g.npc + lq;
-#pragma unroll 4
-            for (int k0 = 0; k0 < g.npc; k0 += 4) {
-                const T a = tcr[k0];
-                const T *pr = P + (k0 + lq) * pitch + l16;
-                a0 = mma(a, pr[i0], a0);
-                a1 = mma(a, pr[i1], a1);
-            }
-            if (PASS == 1) {
-                // along i: A[m][k] = P[c0 + m][k], B[k][n] = Ti[k][i + n]
-                const T *prow = P + (c0 + l16) * pitch + lq;
-#pragma unroll 4
-                for (int k0 = 0; k0 < g.npi; k0 += 4) {
-                    const T a = prow[k0];
-                    const gptr<const T> tr = Ti + (k0 + lq) * g.npi + l16;
-                    a0 = mma(a, tr[i0], a0);
-                    a1 = mma(a, tr[i1], a1);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int c = c0 + Acc<T>::row(lq, r);
-                if (c >= g.nc) continue;
-                const long long rowg = g.base + (long long)c * g.cs;
-                const int ia = i0 + l16, ib = i1 + l16;
-                if (PASS == 0) {
-                    const long long rowv = g.vbase + (long long)c * g.cs;
-                    if (ia < g.ni) Y[rowg + ia] = V[rowv + ia] * P[c * pitch + ia] + a0[r];
-                    if (ib < g.ni) Y[rowg + ib] = V[rowv + ib] * P[c * pitch + ib] + a1[r];
-                } else {
-                    if (ia < g.ni) Y[rowg + ia] += a0[r];
-                    if (ib < g.ni) Y[rowg + ib] += a1[r];
-                }
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ preconditioner, FP64
-// Contract the LDS plane P (c-major) into the wave's accumulator tiles:
-// along c with Mc (row-major), or along i with Mi (row-major).
-template <int NCT, int NIT>
-__device__ __forceinline__ void f64_contract(const double *P, int pitch, const Geo &g,
-                                             const double *M_, bool along_c, f64x4 (&acc)[NCT][NIT])
-{
-    const gptr<const double> M = glb(M_);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-        const int c0 = 16 * tc;
-#pragma unroll
-        for (int v = 0; v < NIT; v += 2) {
-            if (v >= nti) break;
-            const int i0 = 16 * v, i1 = i0 + 16;
-            f64x4 a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0};
-            if (along_c) {
-                const gptr<const double> mr = M + (c0 + l16) * g.npc + lq;
-#pragma unroll 4
-                for (int k0 = 0; k0 < g.npc; k0 += 4) {
-                    const double a = mr[k0];
-                    const double *pr = P + (k0 + lq) * pitch + l16;
-                    a0 = mma(a, pr[i0], a0);
-                    a1 = mma(a, pr[i1], a1);
-                }
-            } else {
-                const double *prow = P + (c0 + l16) * pitch + lq;
-#pragma unroll 4
-                for (int k0 = 0; k0 < g.npi; k0 += 4) {
-                    const double a = prow[k0];
-                    const gptr<const double> mr = M + (k0 + lq) * g.npi + l16;
-                    a0 = mma(a, mr[i0], a0);
-                    a1 = mma(a, mr[i1], a1);
-                }
-            }
-            acc[u][v] = a0;
-            acc[u][v + 1] = a1;
-        }
-    }
-}
-
-// Write the wave's tiles back into the LDS plane (c-major), optionally scaled
-// per element by the preconditioner denominators.
-template <int NCT, int NIT>
-__device__ __forceinline__ void f64_store_lds(double *P, int pitch, const Geo &g,
-                                              const f64x4 (&acc)[NCT][NIT], const FdmTask *t)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-#pragma unroll
-        for (int v = 0; v < NIT; ++v) {
-            if (v >= nti) break;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int c = 16 * tc + lq + 4 * r, i = 16 * v + l16;
-                double x = acc[u][v][r];
-                if (t) {
-                    // plane (i = a, c = z index) at fixed j = b
-                    double den = 1.0;
-                    if (i < g.ni && c < g.nc) {
-                        den = t->ax[0].lam[i] + t->ax[1].lam[g.pl] + t->ax[2].lam[c] - t->shift;
-                        if (t->absden) den = fabs(den);
-                        if (fabs(den) < t->floor) den = den < 0 ? -t->floor : t->floor;
-                    }
-                    x *= t->scale / den;
-                }
-                P[c * pitch + i] = x;
-            }
-        }
-    }
-}
-
-template <typename D, int NCT, int NIT>
-__device__ __forceinline__ void f64_store_global(D *dst_, const Geo &g, const f64x4 (&acc)[NCT][NIT])
-{
-    const gptr<D> dst = glb(dst_);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-#pragma unroll
-        for (int v = 0; v < NIT; ++v) {
-            if (v >= nti) break;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int c = 16 * tc + lq + 4 * r, i = 16 * v + l16;
-                if (c < g.nc && i < g.ni) dst[g.base + (long long)c * g.cs + i] = (D)acc[u][v][r];
-            }
-        }
-    }
-}
-
-template <int PASS, int NPMAX>
-__global__ void __launch_bounds__(kPT) fdm_f64_kernel(const FdmTask *__restrict__ tasks)
-{
-    constexpr int NIT = NPMAX / 16, NCT = (NPMAX / 16 + 3) / 4;
-    const FdmTask &t = tasks[blockIdx.y];
-    Geo g;
-    const int kind = PASS == 1 ? 1 : 0;
-    const AxisMats &Mx = t.ax[0], &My = t.ax[1], &Mz = t.ax[2];
-    const AxisMats &Mc = PASS == 1 ? Mz : My;
-    if (!geo_of(kind, Mx.n, My.n, Mz.n, 1, 0, Mx.np, Mc.np, blockIdx.x, g)) return;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int pitch = fpitch<double>(g.npi);
-    double *P = reinterpret_cast<double *>(smem);
-    const double *src = static_cast<const double *>(PASS == 0 ? t.src : t.dst);
-    stage_f<double, double>(src, g, false, P, pitch);
-    __syncthreads();
-    f64x4 acc[NCT][NIT];
-    if (PASS == 0) f64_contract(P, pitch, g, Mx.q64, false, acc);         // P Qx
-    else if (PASS == 1) f64_contract(P, pitch, g, Mz.qt64, true, acc);    // Qz^T P
-    else f64_contract(P, pitch, g, My.q64, true, acc);                    // Qy P
-    __syncthreads();
-    f64_store_lds(P, pitch, g, acc, PASS == 1 ? &t : nullptr);
-    __syncthreads();
-    if (PASS == 0) f64_contract(P, pitch, g, My.qt64, true, acc);         // Qy^T (.)
-    else if (PASS == 1) f64_contract(P, pitch, g, Mz.q64, true, acc);     // Qz (.)
-    else f64_contract(P, pitch, g, Mx.qt64, false, acc);                  // (.) Qx^T
-    f64_store_global(static_cast<double *>(t.dst), g, acc);
-}
-
 // ------------------------------------------------------------------ preconditioner, split-BF16
 // Owned tiles scaled by scale / (lam_x[i] + ly + lam_z[c]), ly = lam_y[j] -
 // shift of plane (i = a, c = z index) at fixed j, then split into the i-major
@@ -1356,18 +853,7 @@ __global__ void __launch_bounds__(kPT) fdm_bf2_fused_kernel(const FdmTask *__res
 }
 
 // ------------------------------------------------------------------ launch helpers
-// Raises a kernel's dynamic LDS limit to `bytes` (the 160 KB of a CU less the
-// kernel's static LDS); a failure is reported, not left behind as the thread's
-// last HIP error.
-template <typename K>
-void allow_lds(K kernel, size_t bytes = 160 * 1024)
-{
-    PC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-}
-
 size_t bf2_lds(int np) { return (size_t)2 * 2 * np * (np + kBf2Pad) * sizeof(uint16_t); }
-template <typename T> size_t f_lds(int np) { return (size_t)np * fpitch<T>(np) * sizeof(T); }
 
 template <int NPMAX>
 void init_np()
@@ -1378,9 +864,6 @@ void init_np()
         allow_lds(hx_bf2_kernel<1, NPMAX, false>);
         allow_lds(hx_bf2_kernel<0, NPMAX, true>);
         allow_lds(hx_bf2_kernel<1, NPMAX, true>);
-        allow_lds(fdm_f64_kernel<0, NPMAX>);
-        allow_lds(fdm_f64_kernel<1, NPMAX>);
-        allow_lds(fdm_f64_kernel<2, NPMAX>);
         allow_lds(fdm_bf2_kernel<0, NPMAX, false>);
         allow_lds(fdm_bf2_kernel<1, NPMAX, false>);
         allow_lds(fdm_bf2_kernel<2, NPMAX, false>);
@@ -1390,21 +873,10 @@ void init_np()
     });
 }
 
-void init_f()
-{
-    static std::once_flag once;
-    std::call_once(once, [] {
-        allow_lds(hx_f_kernel<double, 0>);
-        allow_lds(hx_f_kernel<double, 1>);
-        allow_lds(hx_f_kernel<float, 0>);
-        allow_lds(hx_f_kernel<float, 1>);
-    });
-}
-
 // Planes per workgroup (measured at 64^3 with 8 - 160 vectors): the H*X
 // kernels run fastest with one plane per workgroup, the split-BF16
 // preconditioner with four (one for 32-, 96- and 128-point planes).  PISCES_PPW_HX /
-// PISCES_PPW_F64 / PISCES_PPW_FDM override.
+// PISCES_PPW_FDM override.
 int ppw_of(const char *env, int def)
 {
     const char *e = std::getenv(env);
@@ -1429,52 +901,23 @@ void hx_bf2_launch(const HxJob *d, int n, int pa, int pb, int np, hipStream_t s)
 }
 
 template <int NPMAX>
-void hx_f64_launch(const HxJob *d, int n, int pa, int pb, int np, hipStream_t s)
-{
-    static std::once_flag once;
-    std::call_once(once, [] {
-        allow_lds(hx_f64_kernel<0, NPMAX, false>);
-        allow_lds(hx_f64_kernel<1, NPMAX, false>);
-        allow_lds(hx_f64_kernel<0, NPMAX, true>);
-        allow_lds(hx_f64_kernel<1, NPMAX, true>);
-    });
-    static const int ppw = ppw_of("PISCES_PPW_F64", 1);
-    const dim3 ga((pa + ppw - 1) / ppw, n), gb((pb + ppw - 1) / ppw, n);
-    const size_t la = (size_t)np * (np + 2) * sizeof(double), lb = 2 * la;
-    if (ppw == 1) {
-        hipLaunchKernelGGL((hx_f64_kernel<0, NPMAX, false>), ga, dim3(kPT), la, s, d);
-        hipLaunchKernelGGL((hx_f64_kernel<1, NPMAX, false>), gb, dim3(kPT), lb, s, d);
-    } else {
-        hipLaunchKernelGGL((hx_f64_kernel<0, NPMAX, true>), ga, dim3(kPT), la, s, d);
-        hipLaunchKernelGGL((hx_f64_kernel<1, NPMAX, true>), gb, dim3(kPT), lb, s, d);
-    }
-}
-
-template <int NPMAX>
-void fdm_np_launch(const FdmTask *d, int n, int nplanes, int np, int precision, hipStream_t s)
+void fdm_bf2_launch(const FdmTask *d, int n, int nplanes, int np, hipStream_t s)
 {
     init_np<NPMAX>();
-    if (precision == PISCES_FP64) {
-        const size_t lds = f_lds<double>(np);
-        hipLaunchKernelGGL((fdm_f64_kernel<0, NPMAX>), dim3(nplanes, n), dim3(kPT), lds, s, d);
-        hipLaunchKernelGGL((fdm_f64_kernel<1, NPMAX>), dim3(nplanes, n), dim3(kPT), lds, s, d);
-        hipLaunchKernelGGL((fdm_f64_kernel<2, NPMAX>), dim3(nplanes, n), dim3(kPT), lds, s, d);
+    const size_t lds = bf2_lds(np);
+    // four planes per workgroup for 64-point planes, one otherwise (64
+    // vectors: 96^3 0.64 against 1.13 ms, where the multi-plane form holds
+    // one wave per SIMD; 32^3 0.025 against 0.038 ms)
+    static const int ppw = ppw_of("PISCES_PPW_FDM", NPMAX == 64 ? 4 : 1);
+    const dim3 grid((nplanes + ppw - 1) / ppw, n);
+    if (ppw == 1) {
+        hipLaunchKernelGGL((fdm_bf2_kernel<0, NPMAX, false>), grid, dim3(kPT), lds, s, d);
+        hipLaunchKernelGGL((fdm_bf2_kernel<1, NPMAX, false>), grid, dim3(kPT), lds, s, d);
+        hipLaunchKernelGGL((fdm_bf2_kernel<2, NPMAX, false>), grid, dim3(kPT), lds, s, d);
     } else {
-        const size_t lds = bf2_lds(np);
-        // four planes per workgroup for 64-point planes, one otherwise (64
-        // vectors: 96^3 0.64 against 1.13 ms, where the multi-plane form holds
-        // one wave per SIMD; 32^3 0.025 against 0.038 ms)
-        static const int ppw = ppw_of("PISCES_PPW_FDM", NPMAX == 64 ? 4 : 1);
-        const dim3 grid((nplanes + ppw - 1) / ppw, n);
-        if (ppw == 1) {
-            hipLaunchKernelGGL((fdm_bf2_kernel<0, NPMAX, false>), grid, dim3(kPT), lds, s, d);
-            hipLaunchKernelGGL((fdm_bf2_kernel<1, NPMAX, false>), grid, dim3(kPT), lds, s, d);
-            hipLaunchKernelGGL((fdm_bf2_kernel<2, NPMAX, false>), grid, dim3(kPT), lds, s, d);
-        } else {
-            hipLaunchKernelGGL((fdm_bf2_kernel<0, NPMAX, true>), grid, dim3(kPT), lds, s, d);
-            hipLaunchKernelGGL((fdm_bf2_kernel<1, NPMAX, true>), grid, dim3(kPT), lds, s, d);
-            hipLaunchKernelGGL((fdm_bf2_kernel<2, NPMAX, true>), grid, dim3(kPT), lds, s, d);
-        }
+        hipLaunchKernelGGL((fdm_bf2_kernel<0, NPMAX, true>), grid, dim3(kPT), lds, s, d);
+        hipLaunchKernelGGL((fdm_bf2_kernel<1, NPMAX, true>), grid, dim3(kPT), lds, s, d);
+        hipLaunchKernelGGL((fdm_bf2_kernel<2, NPMAX, true>), grid, dim3(kPT), lds, s, d);
     }
 }
 
@@ -1485,28 +928,15 @@ void hx_mfma_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_pl
 {
     if (njobs <= 0) return;
     PC_REQUIRE(max_n > 0 && max_n <= 128, PISCES_ERR_UNSUPPORTED, "grid dimension above 128");
-    const int np = axis_pad(max_n);
-    if (precision == PISCES_BF16X2) {
-        if (np <= 32) hx_bf2_launch<32>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-        else if (np <= 64) hx_bf2_launch<64>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-        else if (np <= 96) hx_bf2_launch<96>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-        else hx_bf2_launch<128>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    } else if (precision == PISCES_FP32) {
-        init_f();
-        const size_t lds = f_lds<float>(np);
-        hipLaunchKernelGGL((hx_f_kernel<float, 0>), dim3(max_planes_a, njobs), dim3(kPT), lds, s, d_jobs);
-        hipLaunchKernelGGL((hx_f_kernel<float, 1>), dim3(max_planes_b, njobs), dim3(kPT), lds, s, d_jobs);
-    } else if (np <= 32) {
-        hx_f64_launch<32>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    } else if (np <= 64) {
-        hx_f64_launch<64>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    } else {
-        // a 128-wide FP64 plane and Tx do not fit in LDS together
-        init_f();
-        const size_t lds = f_lds<double>(np);
-        hipLaunchKernelGGL((hx_f_kernel<double, 0>), dim3(max_planes_a, njobs), dim3(kPT), lds, s, d_jobs);
-        hipLaunchKernelGGL((hx_f_kernel<double, 1>), dim3(max_planes_b, njobs), dim3(kPT), lds, s, d_jobs);
+    if (precision != PISCES_BF16X2) {
+        hx_f_launch(d_jobs, njobs, max_planes_a, max_planes_b, max_n, precision, s);
+        return;
     }
+    const int np = axis_pad(max_n);
+    if (np <= 32) hx_bf2_launch<32>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
+    else if (np <= 64) hx_bf2_launch<64>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
+    else if (np <= 96) hx_bf2_launch<96>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
+    else hx_bf2_launch<128>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
     PC_HIP(hipGetLastError());
 }
 
@@ -1735,12 +1165,16 @@ void fdm_launch(const FdmTask *d_tasks, int ntasks, int max_n, int precision, hi
 {
     if (ntasks <= 0) return;
     PC_REQUIRE(max_n > 0 && max_n <= 128, PISCES_ERR_UNSUPPORTED, "grid dimension above 128");
+    if (precision == PISCES_FP64) {
+        fdm_f64_launch(d_tasks, ntasks, max_n, s);
+        return;
+    }
     const int np = axis_pad(max_n);
     // planes per pass: the largest of ny (pass 1) and nz (passes 0, 2) <= max_n
-    if (np <= 32) fdm_np_launch<32>(d_tasks, ntasks, max_n, np, precision, s);
-    else if (np <= 64) fdm_np_launch<64>(d_tasks, ntasks, max_n, np, precision, s);
-    else if (np <= 96) fdm_np_launch<96>(d_tasks, ntasks, max_n, np, precision, s);
-    else fdm_np_launch<128>(d_tasks, ntasks, max_n, np, precision, s);
+    if (np <= 32) fdm_bf2_launch<32>(d_tasks, ntasks, max_n, np, s);
+    else if (np <= 64) fdm_bf2_launch<64>(d_tasks, ntasks, max_n, np, s);
+    else if (np <= 96) fdm_bf2_launch<96>(d_tasks, ntasks, max_n, np, s);
+    else fdm_bf2_launch<128>(d_tasks, ntasks, max_n, np, s);
     PC_HIP(hipGetLastError());
 }
 
