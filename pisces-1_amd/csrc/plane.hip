@@ -41,8 +41,6 @@ namespace pisces {
 
 namespace {
 
-constexpr int kPT = 256;
-
 // ------------------------------------------------------------------ helpers
 __device__ __forceinline__ uint16_t bf16_rne(float x)
 {
@@ -50,10 +48,17 @@ __device__ __forceinline__ uint16_t bf16_rne(float x)
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
-__device__ __forceinline__ void split2(float x, uint16_t &h, uint16_t &l)
+// (x0, x1) as packed BF16 pairs hi = bf16(x), lo = bf16(x - hi), rounded to
+// nearest even by the hardware conversion
+__device__ __forceinline__ unsigned pack_bf16(float x0, float x1)
 {
-    h = bf16_rne(x);
-    l = bf16_rne(x - __uint_as_float((unsigned int)h << 16));
+    const f32x2 x = {x0, x1};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(x, bf16x2));
+}
+__device__ __forceinline__ void split2(float x0, float x1, unsigned &h, unsigned &l)
+{
+    h = pack_bf16(x0, x1);
+    l = pack_bf16(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
 }
 __device__ __forceinline__ bf16x8 ld8(const uint16_t *p)
 {
@@ -68,21 +73,60 @@ __device__ __forceinline__ f32x4 mma_bf(bf16x8 a, bf16x8 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// ------------------------------------------------------------------ owned tiles (split-BF16 forms)
-// Wave w owns the 16-row tiles tc = w + 4u (u < NCT) of a plane and all of its
-// 16-column tiles v < NIT; in each, lane (l16, lq) holds rows 4 lq + r (r < 4)
-// of column l16 -- the accumulator layout of the f32-accumulating MFMAs.
-// Global loads, LDS staging and global stores follow this ownership, so a
-// wave combines its results with values it loaded itself, and a plane's rows
-// move HBM -> registers -> LDS without a layout change.  A workgroup walks the
-// planes p = blockIdx.x, blockIdx.x + gridDim.x, ... of one job; the loads of
-// the next plane are issued before the current one is contracted.
-
-template <int NPMAX> struct Own {
-    static constexpr int NIT = NPMAX / 16;            // column tiles
-    static constexpr int NCT = (NPMAX / 16 + 3) / 4;  // row tiles per wave
-    static constexpr int KS = NPMAX / 32;             // k-steps of the bf16 MFMA
+// ------------------------------------------------------------------ owned tiles
+// A workgroup holds one plane.  Its NT x CS waves split the plane's 16 x 16
+// tiles: wave (tc, h) owns row tile tc and the NIT column tiles from h NIT on;
+// in each, lane (l16, lq) holds rows 4 lq + r (r < 4) of column l16 -- the
+// accumulator layout of the f32-accumulating MFMAs.  Global loads, LDS staging
+// and global stores follow this ownership, so a wave combines its results with
+// values it loaded itself, and a plane's rows move HBM -> registers -> LDS
+// without a layout change.  Everything a wave needs from memory is requested
+// before the first wait: at the vector counts of a solve these kernels are
+// bound by the latency of that chain, not by HBM, LDS or the matrix cores.
+// Measured, all passes, us, before (four waves a plane, two row tiles each above
+// 64 points, four planes per preconditioner workgroup at 64) -> now:
+//   H*X 96^3 x 8 70.4 -> 50.0, 128^3 x 8 228 -> 143, 48^3 x 128 98 -> 75,
+//   64^3 x 32 48.6 -> 47.8; preconditioner 64^3 x 1 50.4 -> 18.1, x 32 70.4 ->
+//   61.5, x 128 209 -> 186, 96^3 x 8 104 -> 73.
+// At 64^3 x 128 H*X moves 5.2 MB a vector between its passes and HBM at 4.6
+// TB/s, near the rate of a plain copy.
+template <int NT, int CS> struct Cfg {
+    static constexpr int NIT = NT / CS;     // column tiles per wave
+    static constexpr int THREADS = 64 * NT * CS;
+    static constexpr int KS = NT / 2;       // k-steps of the bf16 MFMA
+    // the along-i matrix as held fragments of the wave's columns, requested with
+    // the plane; for larger planes they do not fit the registers and are read
+    // where they are used
+    static constexpr bool HOLD = NT <= 4 && CS == 2;
 };
+
+template <int NT, int CS> struct Own {
+    static constexpr int NIT = Cfg<NT, CS>::NIT;
+    int tc, v0, l16, lq, ntc, nti, npc, npi;
+    bool active;  // some of the wave's tiles hold points of the plane
+    __device__ __forceinline__ explicit Own(const Geo &g)
+    {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        l16 = lane & 15;
+        lq = lane >> 4;
+        tc = wave % NT;
+        v0 = (wave / NT) * NIT;
+        ntc = (g.nc + 15) / 16;
+        nti = (g.ni + 15) / 16;
+        npc = g.npc / 16;  // staged tiles: the matrix instruction reads 32 k at a time
+        npi = g.npi / 16;
+        active = tc < ntc && v0 < nti;
+    }
+    __device__ __forceinline__ int row(int r) const { return 16 * tc + 4 * lq + r; }
+    __device__ __forceinline__ int col(int v) const { return 16 * (v0 + v) + l16; }
+};
+
+// element `off` (in elements, 32-bit) of a wave-uniform base
+template <typename T> __device__ __forceinline__ T at(gptr<const T> base, unsigned off)
+{
+    return *reinterpret_cast<gptr<const T>>(reinterpret_cast<gptr<const char>>(base) +
+                                            off * (unsigned)sizeof(T));
+}
 
 // Owned plane values as FP32 (zero outside the n_c x n_i plane) from FP64,
 // FP32 or BF16 (uint16_t bit patterns) storage.  Every lane loads
@@ -93,26 +137,23 @@ template <> __device__ __forceinline__ float as_f32<uint16_t>(uint16_t v)
 {
     return __uint_as_float((unsigned int)v << 16);
 }
-template <typename S, int NCT, int NIT>
-__device__ __forceinline__ void own_load(const S *src_, long long base, const Geo &g,
-                                         float (&x)[NCT][NIT][4])
+template <typename S, int NT, int CS>
+__device__ __forceinline__ void own_load(const S *src, long long base, const Geo &g, const Own<NT, CS> &o,
+                                         float (&x)[Own<NT, CS>::NIT][4])
 {
-    const gptr<const S> src = glb(src_) + base;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
+    const gptr<const S> s = glb(src) + base;
 #pragma unroll
-    for (int u = 0; u < NCT; ++u)
+    for (int r = 0; r < 4; ++r) {
+        const int c = o.row(r);
+        const unsigned oc = (unsigned)c * (unsigned)g.cs;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c = 16 * (wave + 4 * u) + 4 * lq + r;
-#pragma unroll
-            for (int v = 0; v < NIT; ++v) {
-                const int i = 16 * v + l16;
-                const bool ok = c < g.nc && i < g.ni;
-                const float y = as_f32(src[ok ? (long long)c * g.cs + i : 0]);
-                x[u][v][r] = ok ? y : 0.f;
-            }
+        for (int v = 0; v < Own<NT, CS>::NIT; ++v) {
+            const int i = o.col(v);
+            const bool ok = c < g.nc && i < g.ni;
+            const float y = as_f32(at<S>(s, ok ? oc + (unsigned)i : 0u));
+            x[v][r] = ok ? y : 0.f;
         }
+    }
 }
 
 // Row padding (BF16 elements) of the split planes in LDS: a row of a 64-point
@@ -133,11 +174,9 @@ __device__ __forceinline__ unsigned swap_adj(unsigned x)
 __device__ __forceinline__ void put_tile(const float (&x)[4], int cb, int i, int pt, int pc,
                                          uint16_t *Pth, uint16_t *Ptl, uint16_t *Pch, uint16_t *Pcl)
 {
-    uint16_t h[4], l[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) split2(x[r], h[r], l[r]);
-    const unsigned h01 = h[0] | ((unsigned)h[1] << 16), h23 = h[2] | ((unsigned)h[3] << 16);
-    const unsigned l01 = l[0] | ((unsigned)l[1] << 16), l23 = l[2] | ((unsigned)l[3] << 16);
+    unsigned h01, h23, l01, l23;
+    split2(x[0], x[1], h01, l01);
+    split2(x[2], x[3], h23, l23);
     if (Pth) {
         u32x2 vh, vl;
         vh[0] = h01; vh[1] = h23;
@@ -159,238 +198,203 @@ __device__ __forceinline__ void put_tile(const float (&x)[4], int cb, int i, int
     }
 }
 
-template <int NCT, int NIT>
-__device__ __forceinline__ void own_stage(const float (&x)[NCT][NIT][4], const Geo &g,
-                                          uint16_t *Pth, uint16_t *Ptl, uint16_t *Pch, uint16_t *Pcl)
+// The owned tiles into LDS, zeros of the padding included (the contractions
+// read whole 32-point k-steps).
+template <int NT, int CS>
+__device__ __forceinline__ void own_put(const float (&x)[Own<NT, CS>::NIT][4], const Geo &g, const Own<NT, CS> &o,
+                                        uint16_t *Pth, uint16_t *Ptl, uint16_t *Pch, uint16_t *Pcl)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16, pt = g.npc + kBf2Pad, pc = g.npi + kBf2Pad;
+    if (o.tc >= o.npc) return;
 #pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-#pragma unroll
-        for (int v = 0; v < NIT; ++v) {
-            if (v >= nti) break;
-            put_tile(x[u][v], 16 * tc + 4 * lq, 16 * v + l16, pt, pc, Pth, Ptl, Pch, Pcl);
-        }
-    }
+    for (int v = 0; v < Own<NT, CS>::NIT; ++v)
+        if (o.v0 + v < o.npi)
+            put_tile(x[v], 16 * o.tc + 4 * o.lq, o.col(v), g.npc + kBf2Pad, g.npi + kBf2Pad, Pth, Ptl,
+                     Pch, Pcl);
 }
 
-__device__ __forceinline__ bf16x8 bf_zero()
-{
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    return __builtin_bit_cast(bf16x8, z);
-}
-
-// A-form fragments of a row-major split matrix (leading dimension ld) for the
-// wave's own tile rows: rows 16 tc + l16, columns 32 s + 8 lq .. + 7.
-template <int NCT, int KS>
-__device__ __forceinline__ void afrag(const uint16_t *Mh, const uint16_t *Ml, int ld, int ntc, int ks,
-                                      bf16x8 (&ah)[NCT][KS], bf16x8 (&al)[NCT][KS])
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u)
+// Fragments of a row-major split matrix (leading dimension np): rows
+// 16 t + l16, columns 32 s + 8 lq .. + 7 -- the A operand of row tile t, or the
+// B operand of column tile t of its transpose.
+template <int KS> struct Frag {
+    bf16x8 h[KS], l[KS];
+    template <typename P> __device__ __forceinline__ void load(P Mh, P Ml, int ld, int t, int l16, int lq, int ks)
+    {
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            const int tc = wave + 4 * u;
-            if (tc < ntc && s < ks) {
-                ah[u][s] = ld8(glb(Mh) + (16 * tc + l16) * ld + 32 * s + 8 * lq);
-                al[u][s] = ld8(glb(Ml) + (16 * tc + l16) * ld + 32 * s + 8 * lq);
-            } else {
-                ah[u][s] = bf_zero();
-                al[u][s] = bf_zero();
-            }
+            const int e = s < ks ? (16 * t + l16) * ld + 32 * s + 8 * lq : 0;
+            h[s] = ld8(Mh + e);
+            l[s] = ld8(Ml + e);
         }
-}
+    }
+};
 
-// D(c, i) += sum_k A(c, k) B(k, i) on the column-tile pair (i0, i0 + 16) of
-// one row tile, split-BF16 (hi*hi + hi*lo + lo*hi).  A: held fragments.
-// B(k, i) = Bm[i][k] with Bm row-major of pitch ld: the i-major LDS plane for
-// a contraction along c, or the B-form matrix for one along i.
-template <int KS, typename BP>
-__device__ __forceinline__ void mm_pair(const bf16x8 (&ah)[KS], const bf16x8 (&al)[KS], BP Bh, BP Bl,
-                                        int ld, int ks, int i0, f32x4 &a0, f32x4 &a1)
+// acc += A B over ks k-steps, split-BF16: hi*hi + hi*lo + lo*hi
+template <int KS>
+__device__ __forceinline__ void mm(const Frag<KS> &a, const Frag<KS> &b, int ks, f32x4 &acc)
 {
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
-    const int o0 = (i0 + l16) * ld + 8 * lq, o1 = o0 + 16 * ld;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
         if (s >= ks) break;
-        const bf16x8 b0h = ld8(Bh + o0 + 32 * s), b0l = ld8(Bl + o0 + 32 * s);
-        const bf16x8 b1h = ld8(Bh + o1 + 32 * s), b1l = ld8(Bl + o1 + 32 * s);
-        a0 = mma_bf(ah[s], b0h, a0);
-        a1 = mma_bf(ah[s], b1h, a1);
-        a0 = mma_bf(ah[s], b0l, a0);
-        a1 = mma_bf(ah[s], b1l, a1);
-        a0 = mma_bf(al[s], b0h, a0);
-        a1 = mma_bf(al[s], b1h, a1);
+        acc = mma_bf(a.h[s], b.h[s], acc);
+        acc = mma_bf(a.h[s], b.l[s], acc);
+        acc = mma_bf(a.l[s], b.h[s], acc);
     }
 }
 
-// B-form fragments of a row-major split matrix (leading dimension ld) for all
-// column tiles: rows 16 v + l16, columns 32 s + 8 lq .. + 7.  Held in
-// registers for a workgroup's lifetime where they fit (grids up to 64).
-template <int NIT, int KS>
-__device__ __forceinline__ void bfrag(const uint16_t *Mh, const uint16_t *Ml, int ld, int nti, int ks,
-                                      bf16x8 (&bh)[NIT][KS], bf16x8 (&bl)[NIT][KS])
+// acc(c, i) += sum_k M[c][k] P[k][i]: A = held fragments of the wave's row
+// tile of M, B = the i-major plane
+template <int NT, int CS>
+__device__ __forceinline__ void mul_c(const Frag<Cfg<NT, CS>::KS> &a, const uint16_t *Pth, const uint16_t *Ptl,
+                                      const Geo &g, const Own<NT, CS> &o, f32x4 (&acc)[Own<NT, CS>::NIT])
 {
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+    const int pt = g.npc + kBf2Pad, ks = g.npc / 32;
+    // column tiles in pairs: two independent accumulator chains per k-step
 #pragma unroll
-    for (int v = 0; v < NIT; ++v)
+    for (int v = 0; v < Own<NT, CS>::NIT; v += 2) {
+        if (o.v0 + v >= o.nti) break;
+        const bool two = v + 1 < Own<NT, CS>::NIT;
+        const int e0 = o.col(v) * pt + 8 * o.lq, e1 = e0 + 16 * pt;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if (v < nti && s < ks) {
-                bh[v][s] = ld8(glb(Mh) + (16 * v + l16) * ld + 32 * s + 8 * lq);
-                bl[v][s] = ld8(glb(Ml) + (16 * v + l16) * ld + 32 * s + 8 * lq);
+        for (int s = 0; s < Cfg<NT, CS>::KS; ++s) {
+            if (s >= ks) break;
+            const bf16x8 b0h = ld8(Pth + e0 + 32 * s), b0l = ld8(Ptl + e0 + 32 * s);
+            if (two) {
+                const bf16x8 b1h = ld8(Pth + e1 + 32 * s), b1l = ld8(Ptl + e1 + 32 * s);
+                acc[v] = mma_bf(a.h[s], b0h, acc[v]);
+                acc[v + two] = mma_bf(a.h[s], b1h, acc[v + two]);
+                acc[v] = mma_bf(a.h[s], b0l, acc[v]);
+                acc[v + two] = mma_bf(a.h[s], b1l, acc[v + two]);
+                acc[v] = mma_bf(a.l[s], b0h, acc[v]);
+                acc[v + two] = mma_bf(a.l[s], b1h, acc[v + two]);
             } else {
-                bh[v][s] = bf_zero();
-                bl[v][s] = bf_zero();
+                acc[v] = mma_bf(a.h[s], b0h, acc[v]);
+                acc[v] = mma_bf(a.h[s], b0l, acc[v]);
+                acc[v] = mma_bf(a.l[s], b0h, acc[v]);
             }
         }
-}
-
-// mm_pair with both operands held in registers.
-template <int KS>
-__device__ __forceinline__ void mm_pair_held(const bf16x8 (&ah)[KS], const bf16x8 (&al)[KS],
-                                             const bf16x8 (&b0h)[KS], const bf16x8 (&b0l)[KS],
-                                             const bf16x8 (&b1h)[KS], const bf16x8 (&b1l)[KS], int ks,
-                                             f32x4 &a0, f32x4 &a1)
-{
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        if (s >= ks) break;
-        a0 = mma_bf(ah[s], b0h[s], a0);
-        a1 = mma_bf(ah[s], b1h[s], a1);
-        a0 = mma_bf(ah[s], b0l[s], a0);
-        a1 = mma_bf(ah[s], b1l[s], a1);
-        a0 = mma_bf(al[s], b0h[s], a0);
-        a1 = mma_bf(al[s], b1h[s], a1);
     }
 }
 
-// A-form fragments of the wave's own rows of the c-major LDS plane.
-template <int KS>
-__device__ __forceinline__ void afrag_lds(const uint16_t *Pch, const uint16_t *Pcl, int pc, int c0, int ks,
-                                          bf16x8 (&ah)[KS], bf16x8 (&al)[KS])
-{
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+// The along-i matrix of a contraction, B(k, i) = M[i][k] with M row-major:
+// held fragments of the wave's column tiles, or the matrix itself.
+template <int NT, int CS> struct MatI {
+    const uint16_t *h, *l;
+    Frag<Cfg<NT, CS>::HOLD ? Cfg<NT, CS>::KS : 1> f[Cfg<NT, CS>::HOLD ? Own<NT, CS>::NIT : 1];
+    __device__ __forceinline__ MatI(const uint16_t *Mh, const uint16_t *Ml) : h(Mh), l(Ml) {}
+    __device__ __forceinline__ void load(const Geo &g, const Own<NT, CS> &o)
+    {
+        if constexpr (Cfg<NT, CS>::HOLD) {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        if (s >= ks) break;
-        ah[s] = ld8(Pch + (c0 + l16) * pc + 32 * s + 8 * lq);
-        al[s] = ld8(Pcl + (c0 + l16) * pc + 32 * s + 8 * lq);
+            for (int v = 0; v < Own<NT, CS>::NIT; ++v)
+                f[v].load(glb(h), glb(l), g.npi, o.v0 + v < o.nti ? o.v0 + v : 0, o.l16, o.lq, g.npi / 32);
+        }
+    }
+};
+
+// acc(c, i) += sum_k P[c][k] M[k][i]: A = the wave's rows of the c-major plane
+template <int NT, int CS>
+__device__ __forceinline__ void mul_i(const uint16_t *Pch, const uint16_t *Pcl, const MatI<NT, CS> &m,
+                                      const Geo &g, const Own<NT, CS> &o, f32x4 (&acc)[Own<NT, CS>::NIT])
+{
+    constexpr int KS = Cfg<NT, CS>::KS;
+    const int ks = g.npi / 32;
+    Frag<KS> a;
+    a.load(Pch, Pcl, g.npi + kBf2Pad, o.tc, o.l16, o.lq, ks);
+#pragma unroll
+    for (int v = 0; v < Own<NT, CS>::NIT; ++v) {
+        if (o.v0 + v >= o.nti) break;
+        if constexpr (Cfg<NT, CS>::HOLD) {
+            mm(a, m.f[v], ks, acc[v]);
+        } else {
+            Frag<KS> b;
+            b.load(glb(m.h), glb(m.l), g.npi, o.v0 + v, o.l16, o.lq, ks);
+            mm(a, b, ks, acc[v]);
+        }
+    }
+}
+
+template <int N> __device__ __forceinline__ void zero(f32x4 (&acc)[N])
+{
+#pragma unroll
+    for (int v = 0; v < N; ++v) acc[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+template <typename D> __device__ __forceinline__ D of_f32(float v) { return (D)v; }
+template <> __device__ __forceinline__ uint16_t of_f32<uint16_t>(float v) { return bf16_rne(v); }
+
+// Stores the owned tiles to FP64, FP32 or BF16 (uint16_t bit patterns, rounded
+// to nearest even) storage.
+template <typename D, int NT, int CS>
+__device__ __forceinline__ void own_store(D *dst, const Geo &g, const Own<NT, CS> &o,
+                                          const f32x4 (&acc)[Own<NT, CS>::NIT])
+{
+    const gptr<D> d = glb(dst) + g.base;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int c = o.row(r);
+        const unsigned oc = (unsigned)c * (unsigned)g.cs;
+#pragma unroll
+        for (int v = 0; v < Own<NT, CS>::NIT; ++v)
+            if (c < g.nc && o.col(v) < g.ni)
+                *reinterpret_cast<gptr<D>>(reinterpret_cast<gptr<char>>(d) +
+                                           (oc + (unsigned)o.col(v)) * (unsigned)sizeof(D)) = of_f32<D>(acc[v][r]);
     }
 }
 
 // ------------------------------------------------------------------ H*X, split-BF16 form
 // Pass A (plane (i,j) at k): Y = V o X + Ty X along c = j; the accumulators
 // start from V o X.  Pass B (plane (i,k) at j): Y += Tz X along c = k + X Tx
-// along i; the wave's Y values of the next plane are loaded as soon as those
-// of the current plane have been used.  LDS: the i-major plane (pass A), plus
-// the c-major plane (pass B).
-// Planes p, p + pstride, ... (MULTI) or plane p alone of job J; returns at
-// once where p is past the job's planes.
-template <int PASS, int NPMAX, bool MULTI>
-__device__ __forceinline__ void hx_bf2_planes(const HxJob &J, int p, int pstride, unsigned char *smem)
+// along i.  LDS: the i-major plane (pass A), plus the c-major plane (pass B).
+// Plane p of job J; returns at once where p is past the job's planes.
+template <int PASS, int NT, int CS>
+__device__ __forceinline__ void hx_bf2_plane(const HxJob &J, int p, unsigned char *smem)
 {
-    constexpr int NCT = Own<NPMAX>::NCT, NIT = Own<NPMAX>::NIT, KS = Own<NPMAX>::KS;
+    constexpr int NIT = Own<NT, CS>::NIT;
     const AxisMats &Mi = J.ax[0];
     const AxisMats &Mc = J.ax[PASS == 0 ? 1 : 2];
     Geo g;
     if (!geo_of(PASS, J.nx, J.ny, J.nz, J.nvec, J.ld, Mi.np, Mc.np, p, g)) return;
+    const Own<NT, CS> o(g);
     const int pt = g.npc + kBf2Pad, pc = g.npi + kBf2Pad;
     uint16_t *Pth = reinterpret_cast<uint16_t *>(smem);
     uint16_t *Ptl = Pth + g.npi * pt;
     uint16_t *Pch = Ptl + g.npi * pt;
     uint16_t *Pcl = Pch + g.npc * pc;
-    const float *X = static_cast<const float *>(J.X);
-    const float *V = static_cast<const float *>(J.V);
-    const gptr<float> Y = glb(static_cast<float *>(J.Y));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16, ksc = g.npc / 32, ksi = g.npi / 32;
-    bf16x8 ach[NCT][KS], acl[NCT][KS];
-    afrag(Mc.th, Mc.tl, g.npc, ntc, ksc, ach, acl);
-    // pass B, grids up to 64, several planes per workgroup: Tx in B form held
-    // for the workgroup's lifetime (with one plane it is loaded where used:
-    // the same loads, 64 fewer live registers)
-    constexpr bool HOLD = PASS == 1 && NPMAX <= 64 && MULTI;
-    constexpr int NB = HOLD ? NIT : 1, KB = HOLD ? KS : 1;
-    bf16x8 bth[NB][KB], btl[NB][KB];
-    if constexpr (HOLD) bfrag(Mi.th, Mi.tl, g.npi, nti, ksi, bth, btl);
-    float xb[NCT][NIT][4], wb[NCT][NIT][4];  // X; V (pass A) or Y (pass B)
-    own_load(X, g.base, g, xb);
-    own_load(PASS == 0 ? V : static_cast<const float *>(J.Y), PASS == 0 ? g.vbase : g.base, g, wb);
-    for (;;) {
-        own_stage(xb, g, Pth, Ptl, PASS == 1 ? Pch : nullptr, Pcl);
-        if (PASS == 0) {
-#pragma unroll
-            for (int u = 0; u < NCT; ++u)
-#pragma unroll
-                for (int v = 0; v < NIT; ++v)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) wb[u][v][r] *= xb[u][v][r];
-        }
-        __syncthreads();
-        Geo gn;
-        const bool more = MULTI && geo_of(PASS, J.nx, J.ny, J.nz, J.nvec, J.ld, Mi.np, Mc.np, p + pstride, gn);
-        if (more) own_load(X, gn.base, gn, xb);
-#pragma unroll
-        for (int u = 0; u < NCT; ++u) {
-            const int tc = wave + 4 * u;
-            if (tc >= ntc) break;
-            const int c0 = 16 * tc;
-            bf16x8 aih[KS], ail[KS];
-            if (PASS == 1) afrag_lds(Pch, Pcl, pc, c0, ksi, aih, ail);
-#pragma unroll
-            for (int v = 0; v < NIT; v += 2) {
-                if (v >= nti) break;
-                f32x4 a0, a1;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    a0[r] = PASS == 0 ? wb[u][v][r] : 0.f;
-                    a1[r] = PASS == 0 ? wb[u][v + 1][r] : 0.f;
-                }
-                mm_pair(ach[u], acl[u], Pth, Ptl, pt, ksc, 16 * v, a0, a1);
-                // B(k, i) = Tx[k][i] = Tx[i][k] (symmetric)
-                if constexpr (HOLD)
-                    mm_pair_held(aih, ail, bth[v], btl[v], bth[v + 1], btl[v + 1], ksi, a0, a1);
-                else if (PASS == 1)
-                    mm_pair(aih, ail, glb(Mi.th), glb(Mi.tl), g.npi, ksi, 16 * v, a0, a1);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int c = c0 + 4 * lq + r;
-                    if (c >= g.nc) continue;
-                    const long long row = (long long)c * g.cs;
-                    const int ia = 16 * v + l16, ib = ia + 16;
-                    if (ia < g.ni) Y[g.base + row + ia] = PASS == 0 ? a0[r] : wb[u][v][r] + a0[r];
-                    if (ib < g.ni) Y[g.base + row + ib] = PASS == 0 ? a1[r] : wb[u][v + 1][r] + a1[r];
-                    if (more) {
-                        const gptr<const float> W =
-                            PASS == 0 ? glb(V) + gn.vbase + row : (gptr<const float>)Y + gn.base + row;
-                        const float wa = W[ia < g.ni ? ia : 0], wv = W[ib < g.ni ? ib : 0];
-                        wb[u][v][r] = ia < g.ni ? wa : 0.f;
-                        wb[u][v + 1][r] = ib < g.ni ? wv : 0.f;
-                    }
-                }
-            }
-        }
-        if (!more) break;
-        __syncthreads();  // every wave is done with this plane's LDS copy
-        g = gn;
-        p += pstride;
+    float *Y = static_cast<float *>(J.Y);
+    const float *W = PASS == 0 ? static_cast<const float *>(J.V) : Y;  // V (pass A) or Y (pass B)
+    float xb[NIT][4], wb[NIT][4];
+    Frag<Cfg<NT, CS>::KS> a;
+    MatI<NT, CS> ti(Mi.th, Mi.tl);  // B(k, i) = Tx[k][i] = Tx[i][k] (symmetric)
+    own_load<float, NT, CS>(static_cast<const float *>(J.X), g.base, g, o, xb);
+    if (o.active) {
+        a.load(glb(Mc.th), glb(Mc.tl), g.npc, o.tc, o.l16, o.lq, g.npc / 32);
+        if (PASS == 1) ti.load(g, o);
+        own_load<float, NT, CS>(W, PASS == 0 ? g.vbase : g.base, g, o, wb);
     }
+    own_put<NT, CS>(xb, g, o, Pth, Ptl, PASS == 1 ? Pch : nullptr, Pcl);
+    __syncthreads();
+    if (!o.active) return;
+    f32x4 acc[NIT];
+#pragma unroll
+    for (int v = 0; v < NIT; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[v][r] = PASS == 0 ? wb[v][r] * xb[v][r] : 0.f;
+    mul_c<NT, CS>(a, Pth, Ptl, g, o, acc);
+    if (PASS == 1) {
+        mul_i<NT, CS>(Pch, Pcl, ti, g, o, acc);
+#pragma unroll
+        for (int v = 0; v < NIT; ++v)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[v][r] = wb[v][r] + acc[v][r];
+    }
+    own_store<float, NT, CS>(Y, g, o, acc);
 }
 
-template <int PASS, int NPMAX, bool MULTI>
-__global__ void __launch_bounds__(kPT) hx_bf2_kernel(const HxJob *__restrict__ jobs)
+template <int PASS, int NT, int CS>
+__global__ void __launch_bounds__((Cfg<NT, CS>::THREADS), (CS == 1 ? 4 : 1)) hx_bf2_kernel(const HxJob *__restrict__ jobs)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    hx_bf2_planes<PASS, NPMAX, MULTI>(jobs[plane_y(PASS == 1)], plane_x(PASS == 1), gridDim.x, smem);
+    hx_bf2_plane<PASS, NT, CS>(jobs[plane_y(PASS == 1)], plane_x(PASS == 1), smem);
 }
 
 // ------------------------------------------------------------------ H*X, split-BF16, one launch
@@ -445,8 +449,8 @@ __device__ __forceinline__ int xcd_read(int *p)
     return seen;
 }
 
-template <int NPMAX>
-__global__ void __launch_bounds__(kPT) hx_bf2_fused_kernel(const HxJob *__restrict__ jobs,
+template <int NT>
+__global__ void __launch_bounds__((Cfg<NT, 2>::THREADS)) hx_bf2_fused_kernel(const HxJob *__restrict__ jobs,
                                                            int *__restrict__ plan, int batch)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -495,8 +499,8 @@ __global__ void __launch_bounds__(kPT) hx_bf2_fused_kernel(const HxJob *__restri
         const HxJob &J = jobs[job];
         const int pass = s_task[2];
         // plane index within the job: vector-major, as the two-launch kernels count
-        if (pass == 0) hx_bf2_planes<0, NPMAX, false>(J, s_task[1] * J.nz + s_task[3], 1, smem);
-        else hx_bf2_planes<1, NPMAX, false>(J, s_task[1] * J.ny + s_task[3], 1, smem);
+        if (pass == 0) hx_bf2_plane<0, NT, 2>(J, s_task[1] * J.nz + s_task[3], smem);
+        else hx_bf2_plane<1, NT, 2>(J, s_task[1] * J.ny + s_task[3], smem);
         if (pass == 0) {
             // this plane's Y stores have reached the L2 before it is counted
             __builtin_amdgcn_s_waitcnt(0);
@@ -511,254 +515,101 @@ __global__ void __launch_bounds__(kPT) hx_bf2_fused_kernel(const HxJob *__restri
 }
 
 // ------------------------------------------------------------------ preconditioner, split-BF16
-// Owned tiles scaled by scale / (lam_x[i] + ly + lam_z[c]), ly = lam_y[j] -
-// shift of plane (i = a, c = z index) at fixed j, then split into the i-major
-// plane.  lx[v] = lam_x[16 v + l16] and lz[u][r] = lam_z[c] are held per
-// workgroup; the factor is formed in FP32 (the scaled values are FP32 and go
-// on as split BF16).
-template <int NCT, int NIT>
-__device__ __forceinline__ void put_scaled(const f32x4 (&acc)[NCT][NIT], const Geo &g, float ly,
-                                           const float (&lx)[NIT], const float (&lz)[NCT][4],
-                                           float scale, float floor, bool absden, uint16_t *Pth,
-                                           uint16_t *Ptl)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16, pt = g.npc + kBf2Pad;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-#pragma unroll
-        for (int v = 0; v < NIT; ++v) {
-            if (v >= nti) break;
-            const int i = 16 * v + l16, cb = 16 * tc + 4 * lq;
-            float x[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float den = lx[v] + ly + lz[u][r];
-                if (absden) den = fabsf(den);
-                if (fabsf(den) < floor) den = den < 0.f ? -floor : floor;
-                x[r] = acc[u][v][r] * (scale / den);
-            }
-            put_tile(x, cb, i, pt, 0, Pth, Ptl, nullptr, nullptr);
-        }
-    }
-}
-
-template <int NCT, int NIT>
-__device__ __forceinline__ void put_acc(const f32x4 (&acc)[NCT][NIT], const Geo &g, uint16_t *Pth,
-                                        uint16_t *Ptl, uint16_t *Pch, uint16_t *Pcl)
-{
-    float x[NCT][NIT][4];
-#pragma unroll
-    for (int u = 0; u < NCT; ++u)
-#pragma unroll
-        for (int v = 0; v < NIT; ++v)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[u][v][r] = acc[u][v][r];
-    own_stage(x, g, Pth, Ptl, Pch, Pcl);
-}
-
-template <typename D> __device__ __forceinline__ D of_f32(float v) { return (D)v; }
-template <> __device__ __forceinline__ uint16_t of_f32<uint16_t>(float v) { return bf16_rne(v); }
-
-// Stores the owned tiles to FP64, FP32 or BF16 (uint16_t bit patterns, rounded
-// to nearest even) storage.
-template <typename D, int NCT, int NIT>
-__device__ __forceinline__ void bf2_store_global(D *dst_, const Geo &g, const f32x4 (&acc)[NCT][NIT])
-{
-    const gptr<D> dst = glb(dst_);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int ntc = g.npc / 16, nti = g.npi / 16;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-#pragma unroll
-        for (int v = 0; v < NIT; ++v) {
-            if (v >= nti) break;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int c = 16 * tc + 4 * lq + r, i = 16 * v + l16;
-                if (c < g.nc && i < g.ni) dst[g.base + (long long)c * g.cs + i] = of_f32<D>(acc[u][v][r]);
-            }
-        }
-    }
-}
-
-// All owned tiles of one contraction: along c (A = held fragments of the
-// along-c matrix, B = i-major plane) or along i (A = own rows of the c-major
-// plane, B = B-form matrix from global memory).
-template <int NCT, int NIT, int KS>
-__device__ __forceinline__ void mm_c_all(const bf16x8 (&ah)[NCT][KS], const bf16x8 (&al)[NCT][KS],
-                                         const uint16_t *Pth, const uint16_t *Ptl, const Geo &g,
-                                         f32x4 (&acc)[NCT][NIT])
-{
-    const int wave = threadIdx.x >> 6;
-    const int ntc = g.npc / 16, nti = g.npi / 16, ksc = g.npc / 32, pt = g.npc + kBf2Pad;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        if (wave + 4 * u >= ntc) break;
-#pragma unroll
-        for (int v = 0; v < NIT; v += 2) {
-            if (v >= nti) break;
-            f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
-            mm_pair(ah[u], al[u], Pth, Ptl, pt, ksc, 16 * v, a0, a1);
-            acc[u][v] = a0;
-            acc[u][v + 1] = a1;
-        }
-    }
-}
-
-template <int NCT, int NIT, int KS>
-__device__ __forceinline__ void mm_i_held(const uint16_t *Pch, const uint16_t *Pcl,
-                                          const bf16x8 (&bh)[NIT][KS], const bf16x8 (&bl)[NIT][KS],
-                                          const Geo &g, f32x4 (&acc)[NCT][NIT])
-{
-    const int wave = threadIdx.x >> 6;
-    const int ntc = g.npc / 16, nti = g.npi / 16, ksi = g.npi / 32, pc = g.npi + kBf2Pad;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-        bf16x8 ah[KS], al[KS];
-        afrag_lds(Pch, Pcl, pc, 16 * tc, ksi, ah, al);
-#pragma unroll
-        for (int v = 0; v < NIT; v += 2) {
-            if (v >= nti) break;
-            f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
-            mm_pair_held(ah, al, bh[v], bl[v], bh[v + 1], bl[v + 1], ksi, a0, a1);
-            acc[u][v] = a0;
-            acc[u][v + 1] = a1;
-        }
-    }
-}
-
-template <int NCT, int NIT, int KS>
-__device__ __forceinline__ void mm_i_all(const uint16_t *Pch, const uint16_t *Pcl, const uint16_t *Mh,
-                                         const uint16_t *Ml, const Geo &g, f32x4 (&acc)[NCT][NIT])
-{
-    const int wave = threadIdx.x >> 6;
-    const int ntc = g.npc / 16, nti = g.npi / 16, ksi = g.npi / 32, pc = g.npi + kBf2Pad;
-#pragma unroll
-    for (int u = 0; u < NCT; ++u) {
-        const int tc = wave + 4 * u;
-        if (tc >= ntc) break;
-        bf16x8 ah[KS], al[KS];
-        afrag_lds(Pch, Pcl, pc, 16 * tc, ksi, ah, al);
-#pragma unroll
-        for (int v = 0; v < NIT; v += 2) {
-            if (v >= nti) break;
-            f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
-            mm_pair(ah, al, glb(Mh), glb(Ml), g.npi, ksi, 16 * v, a0, a1);
-            acc[u][v] = a0;
-            acc[u][v + 1] = a1;
-        }
-    }
-}
-
-// Three passes, each walking planes like the H*X kernels:
+// Three passes, one plane per workgroup as H*X:
 //   0, plane (i,j) at k: r -> c-major plane; X Qx along i -> i-major plane;
 //      Qy^T (.) along c -> work
-//   1, plane (i,k) at j: work -> i-major plane A; Qz^T (.) along c, scaled ->
-//      i-major plane B; Qz (.) along c -> work
+//   1, plane (i,k) at j: work -> i-major plane A; Qz^T (.) along c, scaled by
+//      scale / (lam_x[i] + lam_y[j] - shift + lam_z[c]) (formed in FP32: the
+//      scaled values are FP32 and go on as split BF16) -> i-major plane B;
+//      Qz (.) along c -> work
 //   2, plane (i,j) at k: work -> i-major plane; Qy (.) along c -> c-major
 //      plane; (.) Qx^T along i -> t
-// The c-major plane is only read by the wave that wrote its rows.
-// Planes p, p + pstride, ... (MULTI) or plane p alone of one pass of task t.
-template <int PASS, int NPMAX, bool MULTI>
-__device__ __forceinline__ void fdm_bf2_planes(const FdmTask &t, int p, int pstride, unsigned char *smem)
+// Plane p, or with MULTI the planes p, p + pstride, ... of one pass of task t:
+// the matrix fragments are then fetched once for several planes and the next
+// plane is requested before the current one is contracted.
+template <int PASS, int NT, int CS, bool MULTI>
+__device__ __forceinline__ void fdm_bf2_plane(const FdmTask &t, int p, int pstride, unsigned char *smem)
 {
-    constexpr int NCT = Own<NPMAX>::NCT, NIT = Own<NPMAX>::NIT, KS = Own<NPMAX>::KS;
-    const int kind = PASS == 1 ? 1 : 0;
+    constexpr int NIT = Own<NT, CS>::NIT, KS = Cfg<NT, CS>::KS;
     const AxisMats &Mx = t.ax[0], &My = t.ax[1], &Mz = t.ax[2];
     const AxisMats &Mc = PASS == 1 ? Mz : My;
     Geo g;
-    if (!geo_of(kind, Mx.n, My.n, Mz.n, 1, 0, Mx.np, Mc.np, p, g)) return;
-    const int pt = g.npc + kBf2Pad, pc = g.npi + kBf2Pad;
+    if (!geo_of(PASS == 1 ? 1 : 0, Mx.n, My.n, Mz.n, 1, 0, Mx.np, Mc.np, p, g)) return;
+    const Own<NT, CS> o(g);
+    const int pt = g.npc + kBf2Pad, pc = g.npi + kBf2Pad, ksc = g.npc / 32;
     uint16_t *Pth = reinterpret_cast<uint16_t *>(smem);
     uint16_t *Ptl = Pth + g.npi * pt;
     uint16_t *P2h = Ptl + g.npi * pt;  // c-major plane (passes 0, 2) or i-major plane B (pass 1)
     uint16_t *P2l = P2h + (PASS == 1 ? g.npi * pt : g.npc * pc);
-    const int ntc = g.npc / 16, ksc = g.npc / 32;
-    bf16x8 ah[NCT][KS], al[NCT][KS], bh[NCT][KS], bl[NCT][KS];
-    if (PASS == 0) afrag(My.qth, My.qtl, g.npc, ntc, ksc, ah, al);       // Qy^T
-    if (PASS == 1) {
-        afrag(Mz.qth, Mz.qtl, g.npc, ntc, ksc, ah, al);                  // Qz^T
-        afrag(Mz.qh, Mz.ql, g.npc, ntc, ksc, bh, bl);                    // Qz
-    }
-    if (PASS == 2) afrag(My.qh, My.ql, g.npc, ntc, ksc, ah, al);         // Qy
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int nti = g.npi / 16, ksi = g.npi / 32;
-    // passes 0 and 2, grids up to 64, several planes per workgroup: Qx in B form
-    // held for the workgroup's lifetime (with one plane it is loaded where used)
-    constexpr bool HOLD = PASS != 1 && NPMAX <= 64 && MULTI;
-    constexpr int NB = HOLD ? NIT : 1, KB = HOLD ? KS : 1;
-    bf16x8 qbh[NB][KB], qbl[NB][KB];
-    if constexpr (HOLD) {
-        if (PASS == 0) bfrag(Mx.qth, Mx.qtl, g.npi, nti, ksi, qbh, qbl);  // B form of Qx
-        else bfrag(Mx.qh, Mx.ql, g.npi, nti, ksi, qbh, qbl);              // B form of Qx^T
-    }
-    // pass 1: eigenvalues of the owned rows and columns
-    float lx[NIT], lz[NCT][4];
-    if (PASS == 1) {
-        const gptr<const double> Lx = glb(Mx.lam), Lz = glb(Mz.lam);
-#pragma unroll
-        for (int v = 0; v < NIT; ++v) {
-            const int i = 16 * v + l16;
-            const double y = Lx[i < g.ni ? i : 0];
-            lx[v] = i < g.ni ? (float)y : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < NCT; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int c = 16 * (wave + 4 * u) + 4 * lq + r;
-                const double y = Lz[c < g.nc ? c : 0];
-                lz[u][r] = c < g.nc ? (float)y : 0.f;
-            }
-    }
+    float xb[NIT][4], lx[NIT], lz[4];
+    Frag<KS> a, b;
+    // B form of Qx (pass 0) and of Qx^T (pass 2)
+    MatI<NT, CS> mi(PASS == 0 ? Mx.qth : Mx.qh, PASS == 0 ? Mx.qtl : Mx.ql);
     // pass 0 reads r (FP64 or FP32); passes 1 and 2 the BF16 intermediate
-    float xb[NCT][NIT][4];
     auto load = [&](const Geo &gg) {
-        if constexpr (PASS != 0) own_load(static_cast<const uint16_t *>(t.work), gg.base, gg, xb);
-        else if (t.src32) own_load(static_cast<const float *>(t.src), gg.base, gg, xb);
-        else own_load(static_cast<const double *>(t.src), gg.base, gg, xb);
+        if constexpr (PASS != 0) own_load<uint16_t, NT, CS>(static_cast<const uint16_t *>(t.work), gg.base, gg, o, xb);
+        else if (t.src32) own_load<float, NT, CS>(static_cast<const float *>(t.src), gg.base, gg, o, xb);
+        else own_load<double, NT, CS>(static_cast<const double *>(t.src), gg.base, gg, o, xb);
     };
     load(g);
-    f32x4 acc[NCT][NIT];
+    if (o.active) {
+        // along c: Qy^T (pass 0), Qz^T then Qz (pass 1), Qy (pass 2)
+        a.load(glb(PASS == 2 ? My.qh : Mc.qth), glb(PASS == 2 ? My.ql : Mc.qtl), g.npc, o.tc, o.l16, o.lq, ksc);
+        if (PASS == 1) {
+            if (NT < 8) b.load(glb(Mz.qh), glb(Mz.ql), g.npc, o.tc, o.l16, o.lq, ksc);
+#pragma unroll
+            for (int v = 0; v < NIT; ++v) lx[v] = (float)at<double>(glb(Mx.lam), o.col(v) < g.ni ? o.col(v) : 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) lz[r] = (float)at<double>(glb(Mz.lam), o.row(r) < g.nc ? o.row(r) : 0);
+        } else {
+            mi.load(g, o);
+        }
+    }
+    const float scale = (float)t.scale, floor = (float)t.floor;
     for (;;) {
-        own_stage(xb, g, PASS == 0 ? nullptr : Pth, Ptl, PASS == 0 ? P2h : nullptr, P2l);
+        const double ly = PASS == 1 ? glb(My.lam)[g.pl] : 0.0;
+        own_put<NT, CS>(xb, g, o, PASS == 0 ? nullptr : Pth, Ptl, PASS == 0 ? P2h : nullptr, P2l);
         __syncthreads();
         Geo gn;
-        const bool more = MULTI && geo_of(kind, Mx.n, My.n, Mz.n, 1, 0, Mx.np, Mc.np, p + pstride, gn);
+        const bool more = MULTI && geo_of(PASS == 1 ? 1 : 0, Mx.n, My.n, Mz.n, 1, 0, Mx.np, Mc.np, p + pstride, gn);
         if (more) load(gn);
-        if (PASS == 0) {
-            if constexpr (HOLD) mm_i_held<NCT, NIT, KS>(P2h, P2l, qbh, qbl, g, acc);  // X Qx
-            else mm_i_all<NCT, NIT, KS>(P2h, P2l, Mx.qth, Mx.qtl, g, acc);
-            put_acc(acc, g, Pth, Ptl, nullptr, nullptr);
-            __syncthreads();
-            mm_c_all(ah, al, Pth, Ptl, g, acc);                            // Qy^T (.)
-            bf2_store_global(t.work, g, acc);
-        } else if (PASS == 1) {
-            mm_c_all(ah, al, Pth, Ptl, g, acc);                            // Qz^T X
-            // rows of the scaled plane: i = a, c = z index, at j = g.pl
-            put_scaled(acc, g, (float)(glb(My.lam)[g.pl] - t.shift), lx, lz, (float)t.scale,
-                       (float)t.floor, t.absden != 0, P2h, P2l);
-            __syncthreads();
-            mm_c_all(bh, bl, P2h, P2l, g, acc);                            // Qz (.)
-            bf2_store_global(t.work, g, acc);
-        } else {
-            mm_c_all(ah, al, Pth, Ptl, g, acc);                            // Qy X
-            put_acc(acc, g, nullptr, nullptr, P2h, P2l);
-            __syncthreads();
-            if constexpr (HOLD) mm_i_held<NCT, NIT, KS>(P2h, P2l, qbh, qbl, g, acc);  // (.) Qx^T
-            else mm_i_all<NCT, NIT, KS>(P2h, P2l, Mx.qh, Mx.ql, g, acc);
-            if (t.dst32) bf2_store_global(static_cast<float *>(t.dst), g, acc);
-            else bf2_store_global(static_cast<double *>(t.dst), g, acc);
+        f32x4 acc[NIT];
+        zero(acc);
+        if (o.active) {
+            if (PASS == 0) mul_i<NT, CS>(P2h, P2l, mi, g, o, acc);  // X Qx
+            else mul_c<NT, CS>(a, Pth, Ptl, g, o, acc);             // Qz^T X, Qy X
+            // both matrices at once exceed the registers of 16 waves
+            if (PASS == 1 && NT == 8) b.load(glb(Mz.qh), glb(Mz.ql), g.npc, o.tc, o.l16, o.lq, ksc);
+        }
+        const float fly = (float)(ly - t.shift);
+        float y[NIT][4];
+#pragma unroll
+        for (int v = 0; v < NIT; ++v)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (PASS == 1) {
+                    // outside the plane the accumulators are 0
+                    float den = o.active && o.col(v) < g.ni && o.row(r) < g.nc ? lx[v] + fly + lz[r] : 1.f;
+                    if (t.absden) den = fabsf(den);
+                    if (fabsf(den) < floor) den = den < 0.f ? -floor : floor;
+                    y[v][r] = acc[v][r] * (scale / den);
+                } else {
+                    y[v][r] = acc[v][r];
+                }
+            }
+        // the other plane's LDS: its last readers are past the barrier above
+        if (PASS == 0) own_put<NT, CS>(y, g, o, Pth, Ptl, nullptr, nullptr);
+        else if (PASS == 1) own_put<NT, CS>(y, g, o, P2h, P2l, nullptr, nullptr);
+        else own_put<NT, CS>(y, g, o, nullptr, nullptr, P2h, P2l);
+        __syncthreads();
+        if (o.active) {
+            zero(acc);
+            if (PASS == 0) mul_c<NT, CS>(a, Pth, Ptl, g, o, acc);        // Qy^T (.)
+            else if (PASS == 1) mul_c<NT, CS>(b, P2h, P2l, g, o, acc);   // Qz (.)
+            else mul_i<NT, CS>(P2h, P2l, mi, g, o, acc);                 // (.) Qx^T
+            if (PASS != 2) own_store<uint16_t, NT, CS>(t.work, g, o, acc);
+            else if (t.dst32) own_store<float, NT, CS>(static_cast<float *>(t.dst), g, o, acc);
+            else own_store<double, NT, CS>(static_cast<double *>(t.dst), g, o, acc);
         }
         if (!more) break;
         g = gn;
@@ -766,11 +617,11 @@ __device__ __forceinline__ void fdm_bf2_planes(const FdmTask &t, int p, int pstr
     }
 }
 
-template <int PASS, int NPMAX, bool MULTI>
-__global__ void __launch_bounds__(kPT) fdm_bf2_kernel(const FdmTask *__restrict__ tasks)
+template <int PASS, int NT, int CS, bool MULTI>
+__global__ void __launch_bounds__((Cfg<NT, CS>::THREADS)) fdm_bf2_kernel(const FdmTask *__restrict__ tasks)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    fdm_bf2_planes<PASS, NPMAX, MULTI>(tasks[plane_y(PASS == 1)], plane_x(PASS == 1), gridDim.x, smem);
+    fdm_bf2_plane<PASS, NT, CS, MULTI>(tasks[plane_y(PASS == 1)], plane_x(PASS == 1), gridDim.x, smem);
 }
 
 // ------------------------------------------------------------------ preconditioner, one launch
@@ -787,8 +638,8 @@ __global__ void __launch_bounds__(kPT) fdm_bf2_kernel(const FdmTask *__restrict_
 // [16, 25) first segment of each XCD, [25] vectors, then per vector the
 // completion counts of pass 0 and of pass 1, then the segments (task, 0,
 // pass, first ticket, planes, vector slot).
-template <int NPMAX>
-__global__ void __launch_bounds__(kPT) fdm_bf2_fused_kernel(const FdmTask *__restrict__ tasks,
+template <int NT>
+__global__ void __launch_bounds__((Cfg<NT, 2>::THREADS)) fdm_bf2_fused_kernel(const FdmTask *__restrict__ tasks,
                                                             int *__restrict__ plan, int batch)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -836,9 +687,9 @@ __global__ void __launch_bounds__(kPT) fdm_bf2_fused_kernel(const FdmTask *__res
         if (task < 0) break;
         const FdmTask &T = tasks[task];
         const int pass = s_task[1];
-        if (pass == 0) fdm_bf2_planes<0, NPMAX, false>(T, s_task[2], 1, smem);
-        else if (pass == 1) fdm_bf2_planes<1, NPMAX, false>(T, s_task[2], 1, smem);
-        else fdm_bf2_planes<2, NPMAX, false>(T, s_task[2], 1, smem);
+        if (pass == 0) fdm_bf2_plane<0, NT, 2, false>(T, s_task[2], 1, smem);
+        else if (pass == 1) fdm_bf2_plane<1, NT, 2, false>(T, s_task[2], 1, smem);
+        else fdm_bf2_plane<2, NT, 2, false>(T, s_task[2], 1, smem);
         if (pass < 2) {
             // this plane's stores have reached the L2 before it is counted
             __builtin_amdgcn_s_waitcnt(0);
@@ -855,70 +706,43 @@ __global__ void __launch_bounds__(kPT) fdm_bf2_fused_kernel(const FdmTask *__res
 // ------------------------------------------------------------------ launch helpers
 size_t bf2_lds(int np) { return (size_t)2 * 2 * np * (np + kBf2Pad) * sizeof(uint16_t); }
 
-template <int NPMAX>
-void init_np()
-{
-    static std::once_flag once;
-    std::call_once(once, [] {
-        allow_lds(hx_bf2_kernel<0, NPMAX, false>);
-        allow_lds(hx_bf2_kernel<1, NPMAX, false>);
-        allow_lds(hx_bf2_kernel<0, NPMAX, true>);
-        allow_lds(hx_bf2_kernel<1, NPMAX, true>);
-        allow_lds(fdm_bf2_kernel<0, NPMAX, false>);
-        allow_lds(fdm_bf2_kernel<1, NPMAX, false>);
-        allow_lds(fdm_bf2_kernel<2, NPMAX, false>);
-        allow_lds(fdm_bf2_kernel<0, NPMAX, true>);
-        allow_lds(fdm_bf2_kernel<1, NPMAX, true>);
-        allow_lds(fdm_bf2_kernel<2, NPMAX, true>);
-    });
-}
-
-// Planes per workgroup (measured at 64^3 with 8 - 160 vectors): the H*X
-// kernels run fastest with one plane per workgroup, the split-BF16
-// preconditioner with four (one for 32-, 96- and 128-point planes).  PISCES_PPW_HX /
-// PISCES_PPW_FDM override.
-int ppw_of(const char *env, int def)
+// a positive integer from the environment, else def
+int env_or(const char *env, int def)
 {
     const char *e = std::getenv(env);
     const int v = e ? std::atoi(e) : 0;
     return v > 0 ? v : def;
 }
 
-template <int NPMAX>
-void hx_bf2_launch(const HxJob *d, int n, int pa, int pb, int np, hipStream_t s)
+template <int NT, int CS>
+void hx_bf2_launch(const HxJob *d, int n, int pa, int pb, hipStream_t s)
 {
-    init_np<NPMAX>();
-    static const int ppw = ppw_of("PISCES_PPW_HX", 1);
-    const dim3 ga((pa + ppw - 1) / ppw, n), gb((pb + ppw - 1) / ppw, n);
+    static std::once_flag once;
+    std::call_once(once, [] {
+        allow_lds(hx_bf2_kernel<0, NT, CS>);
+        allow_lds(hx_bf2_kernel<1, NT, CS>);
+    });
+    const size_t lds = bf2_lds(16 * NT);
+    const dim3 blk(Cfg<NT, CS>::THREADS);
     // pass A uses only the i-major plane (first half of the layout)
-    if (ppw == 1) {
-        hipLaunchKernelGGL((hx_bf2_kernel<0, NPMAX, false>), ga, dim3(kPT), bf2_lds(np) / 2, s, d);
-        hipLaunchKernelGGL((hx_bf2_kernel<1, NPMAX, false>), gb, dim3(kPT), bf2_lds(np), s, d);
-    } else {
-        hipLaunchKernelGGL((hx_bf2_kernel<0, NPMAX, true>), ga, dim3(kPT), bf2_lds(np) / 2, s, d);
-        hipLaunchKernelGGL((hx_bf2_kernel<1, NPMAX, true>), gb, dim3(kPT), bf2_lds(np), s, d);
-    }
+    hipLaunchKernelGGL((hx_bf2_kernel<0, NT, CS>), dim3(pa, n), blk, lds / 2, s, d);
+    hipLaunchKernelGGL((hx_bf2_kernel<1, NT, CS>), dim3(pb, n), blk, lds, s, d);
 }
 
-template <int NPMAX>
-void fdm_bf2_launch(const FdmTask *d, int n, int nplanes, int np, hipStream_t s)
+template <int NT, int CS, bool MULTI>
+void fdm_bf2_launch(const FdmTask *d, int n, int nplanes, hipStream_t s, int ppw = 1)
 {
-    init_np<NPMAX>();
-    const size_t lds = bf2_lds(np);
-    // four planes per workgroup for 64-point planes, one otherwise (64
-    // vectors: 96^3 0.64 against 1.13 ms, where the multi-plane form holds
-    // one wave per SIMD; 32^3 0.025 against 0.038 ms)
-    static const int ppw = ppw_of("PISCES_PPW_FDM", NPMAX == 64 ? 4 : 1);
-    const dim3 grid((nplanes + ppw - 1) / ppw, n);
-    if (ppw == 1) {
-        hipLaunchKernelGGL((fdm_bf2_kernel<0, NPMAX, false>), grid, dim3(kPT), lds, s, d);
-        hipLaunchKernelGGL((fdm_bf2_kernel<1, NPMAX, false>), grid, dim3(kPT), lds, s, d);
-        hipLaunchKernelGGL((fdm_bf2_kernel<2, NPMAX, false>), grid, dim3(kPT), lds, s, d);
-    } else {
-        hipLaunchKernelGGL((fdm_bf2_kernel<0, NPMAX, true>), grid, dim3(kPT), lds, s, d);
-        hipLaunchKernelGGL((fdm_bf2_kernel<1, NPMAX, true>), grid, dim3(kPT), lds, s, d);
-        hipLaunchKernelGGL((fdm_bf2_kernel<2, NPMAX, true>), grid, dim3(kPT), lds, s, d);
-    }
+    static std::once_flag once;
+    std::call_once(once, [] {
+        allow_lds(fdm_bf2_kernel<0, NT, CS, MULTI>);
+        allow_lds(fdm_bf2_kernel<1, NT, CS, MULTI>);
+        allow_lds(fdm_bf2_kernel<2, NT, CS, MULTI>);
+    });
+    const size_t lds = bf2_lds(16 * NT);
+    const dim3 grid((nplanes + ppw - 1) / ppw, n), blk(Cfg<NT, CS>::THREADS);
+    hipLaunchKernelGGL((fdm_bf2_kernel<0, NT, CS, MULTI>), grid, blk, lds, s, d);
+    hipLaunchKernelGGL((fdm_bf2_kernel<1, NT, CS, MULTI>), grid, blk, lds, s, d);
+    hipLaunchKernelGGL((fdm_bf2_kernel<2, NT, CS, MULTI>), grid, blk, lds, s, d);
 }
 
 }  // namespace
@@ -933,10 +757,20 @@ void hx_mfma_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_pl
         return;
     }
     const int np = axis_pad(max_n);
-    if (np <= 32) hx_bf2_launch<32>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    else if (np <= 64) hx_bf2_launch<64>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    else if (np <= 96) hx_bf2_launch<96>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    else hx_bf2_launch<128>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
+    if (np <= 32) hx_bf2_launch<2, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+    else if (np <= 64) {
+        // Few planes: eight waves each, for the latency of a plane; more than
+        // about 1.5 a CU: four waves and fewer registers, so that four planes
+        // are in flight on a CU instead of two.  us at 64^3, eight / four waves:
+        // 4 vectors 14.4 / 15.2, 8 20.8 / 20.1, 32 49.9 / 47.8, 128 161 / 147;
+        // at 48^3 128 vectors 102 / 75.
+        if ((long long)njobs * max_planes_a < 384)
+            hx_bf2_launch<4, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+        else
+            hx_bf2_launch<4, 1>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+    }
+    else if (np <= 96) hx_bf2_launch<6, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+    else hx_bf2_launch<8, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
     PC_HIP(hipGetLastError());
 }
 
@@ -1001,16 +835,16 @@ void hx_fused_plan(const HxJob *h_jobs, int njobs, int *plan)
 }
 
 namespace {
-template <int NPMAX>
-void hx_fused_np_launch(const HxJob *d_jobs, int *d_plan, int np, int max_tickets, hipStream_t s)
+template <int NT>
+void hx_fused_nt_launch(const HxJob *d_jobs, int *d_plan, int max_tickets, hipStream_t s)
 {
     static std::once_flag once;
-    std::call_once(once, [] { allow_lds(hx_bf2_fused_kernel<NPMAX>, bf2_lds(NPMAX)); });
+    std::call_once(once, [] { allow_lds(hx_bf2_fused_kernel<NT>, bf2_lds(16 * NT)); });
     // workgroups per XCD: two per CU (32 CUs) unless an XCD has fewer planes
-    static const int wpx = ppw_of("PISCES_HXF_WG", 64);
-    static const int batch = ppw_of("PISCES_HXF_BATCH", 4);
+    static const int wpx = env_or("PISCES_HXF_WG", 64);
+    static const int batch = env_or("PISCES_HXF_BATCH", 4);
     const int w = std::max(1, std::min(wpx, max_tickets));
-    hipLaunchKernelGGL((hx_bf2_fused_kernel<NPMAX>), dim3(kXcds * w), dim3(kPT), bf2_lds(np), s,
+    hipLaunchKernelGGL((hx_bf2_fused_kernel<NT>), dim3(kXcds * w), dim3(Cfg<NT, 2>::THREADS), bf2_lds(16 * NT), s,
                        d_jobs, d_plan, batch);
 }
 }  // namespace
@@ -1023,9 +857,9 @@ void hx_fused_launch(const HxJob *h_jobs, const HxJob *d_jobs, int njobs, const 
     int mt = 0;
     for (int x = 0; x < kXcds; ++x) mt = std::max(mt, h_plan[8 + x]);
     const int np = axis_pad(max_n);
-    if (np <= 32) hx_fused_np_launch<32>(d_jobs, d_plan, np, mt, s);
-    else if (np <= 64) hx_fused_np_launch<64>(d_jobs, d_plan, np, mt, s);
-    else hx_fused_np_launch<128>(d_jobs, d_plan, np, mt, s);
+    if (np <= 32) hx_fused_nt_launch<2>(d_jobs, d_plan, mt, s);
+    else if (np <= 64) hx_fused_nt_launch<4>(d_jobs, d_plan, mt, s);
+    else hx_fused_nt_launch<8>(d_jobs, d_plan, mt, s);
     PC_HIP(hipGetLastError());
 }
 
@@ -1125,15 +959,15 @@ void fdm_fused_plan(const FdmTask *h_tasks, int ntasks, int *plan)
 }
 
 namespace {
-template <int NPMAX>
-void fdm_fused_np_launch(const FdmTask *d_tasks, int *d_plan, int np, int max_tickets, hipStream_t s)
+template <int NT>
+void fdm_fused_nt_launch(const FdmTask *d_tasks, int *d_plan, int max_tickets, hipStream_t s)
 {
     static std::once_flag once;
-    std::call_once(once, [] { allow_lds(fdm_bf2_fused_kernel<NPMAX>, bf2_lds(NPMAX)); });
-    static const int wpx = ppw_of("PISCES_FDMF_WG", 64);
-    static const int batch = ppw_of("PISCES_FDMF_BATCH", 4);
+    std::call_once(once, [] { allow_lds(fdm_bf2_fused_kernel<NT>, bf2_lds(16 * NT)); });
+    static const int wpx = env_or("PISCES_FDMF_WG", 64);
+    static const int batch = env_or("PISCES_FDMF_BATCH", 4);
     const int w = std::max(1, std::min(wpx, max_tickets));
-    hipLaunchKernelGGL((fdm_bf2_fused_kernel<NPMAX>), dim3(kXcds * w), dim3(kPT), bf2_lds(np), s,
+    hipLaunchKernelGGL((fdm_bf2_fused_kernel<NT>), dim3(kXcds * w), dim3(Cfg<NT, 2>::THREADS), bf2_lds(16 * NT), s,
                        d_tasks, d_plan, batch);
 }
 }  // namespace
@@ -1146,9 +980,9 @@ void fdm_fused_launch(const FdmTask *d_tasks, int *d_plan, const int *h_plan, in
     for (int x = 0; x < kXcds; ++x) mt = std::max(mt, h_plan[8 + x]);
     if (mt == 0) return;
     const int np = axis_pad(max_n);
-    if (np <= 32) fdm_fused_np_launch<32>(d_tasks, d_plan, np, mt, s);
-    else if (np <= 64) fdm_fused_np_launch<64>(d_tasks, d_plan, np, mt, s);
-    else fdm_fused_np_launch<128>(d_tasks, d_plan, np, mt, s);
+    if (np <= 32) fdm_fused_nt_launch<2>(d_tasks, d_plan, mt, s);
+    else if (np <= 64) fdm_fused_nt_launch<4>(d_tasks, d_plan, mt, s);
+    else fdm_fused_nt_launch<8>(d_tasks, d_plan, mt, s);
     PC_HIP(hipGetLastError());
 }
 
@@ -1171,10 +1005,24 @@ void fdm_launch(const FdmTask *d_tasks, int ntasks, int max_n, int precision, hi
     }
     const int np = axis_pad(max_n);
     // planes per pass: the largest of ny (pass 1) and nz (passes 0, 2) <= max_n
-    if (np <= 32) fdm_bf2_launch<32>(d_tasks, ntasks, max_n, np, s);
-    else if (np <= 64) fdm_bf2_launch<64>(d_tasks, ntasks, max_n, np, s);
-    else if (np <= 96) fdm_bf2_launch<96>(d_tasks, ntasks, max_n, np, s);
-    else fdm_bf2_launch<128>(d_tasks, ntasks, max_n, np, s);
+    if (np <= 32) {
+        fdm_bf2_launch<2, 2, false>(d_tasks, ntasks, max_n, s);
+    } else if (np <= 64) {
+        // Planes per workgroup by the number of planes: a plane's three matrix
+        // fragments are as many bytes from the L2 as six planes, so workgroups
+        // keep them for several planes as soon as that leaves every CU busy.  us
+        // at 64^3 with 1 / 2 / 4 / 8 planes: 4 vectors 20 / 26 / 38 / 62, 16
+        // 54 / 45 / 46 / 70, 32 91 / 71 / 62 / 70, 128 327 / 241 / 203 / 186.
+        // (32-point planes: one is best or the same up to 128 vectors; 96 and
+        // 128 points do not hold the along-i matrix.)  PISCES_PPW_FDM overrides.
+        const long long planes = (long long)ntasks * max_n;
+        static const int ppw_env = env_or("PISCES_PPW_FDM", 0);
+        const int ppw = ppw_env ? ppw_env : planes < 600 ? 1 : planes < 1800 ? 2 : planes < 4096 ? 4 : 8;
+        if (ppw == 1) fdm_bf2_launch<4, 2, false>(d_tasks, ntasks, max_n, s);
+        else fdm_bf2_launch<4, 2, true>(d_tasks, ntasks, max_n, s, ppw);
+    }
+    else if (np <= 96) fdm_bf2_launch<6, 2, false>(d_tasks, ntasks, max_n, s);
+    else fdm_bf2_launch<8, 2, false>(d_tasks, ntasks, max_n, s);
     PC_HIP(hipGetLastError());
 }
 

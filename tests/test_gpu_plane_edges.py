@@ -40,3 +40,24 @@ def test_precond_fp64_tile_edges(pisces, oracle_mod, n):
         t = ctx.kinetic_precond(r, shift=-0.05, scale=-1.0, floor=1e-3)
     lhs = g.apply_h(np.zeros(g.ngp), t) + 0.05 * t
     np.testing.assert_allclose(lhs, -r, rtol=0, atol=1e-10)
+
+
+@pytest.mark.parametrize("n", [(33, 40, 35), (64, 9, 50)])
+@pytest.mark.parametrize("nvec", [5, 13, 30, 70])
+def test_bf16x2_launch_shapes_agree(pisces, n, nvec):
+    """The split-BF16 kernels choose waves and planes per workgroup by the
+    number of planes; a plane's arithmetic is the same in every form, so each
+    vector comes out bit for bit as it does alone."""
+    print("bf16x2 shapes", n, nvec, flush=True)
+    L = tuple(0.6 * (v + 1) for v in n)
+    rng = np.random.default_rng(nvec)
+    ngp = int(np.prod(n))
+    X = rng.uniform(-1, 1, (nvec, ngp))
+    with pisces.Context(n, L) as ctx:
+        ctx.set_potential(rng.uniform(-1.0, 0.5, ngp))
+        Y = ctx.apply_h_ex(X, pisces.BF16X2)
+        T = ctx.kinetic_precond(X, shift=-0.05, precision=pisces.BF16X2)
+        for v in (0, nvec // 2, nvec - 1):
+            np.testing.assert_array_equal(Y[v], ctx.apply_h_ex(X[v], pisces.BF16X2))
+            np.testing.assert_array_equal(T[v], ctx.kinetic_precond(X[v], shift=-0.05,
+                                                                    precision=pisces.BF16X2)[0])
