@@ -407,14 +407,14 @@ int pisces_build_cluster_potential(pisces_ctx *c, int nw, const double *xyz_ang,
         PC_REQUIRE(water_sites_host(nw, xyz_ang, sites.data()), PISCES_ERR_NUMERIC,
                    "water projection produced non-finite coordinates");
         const int ns = 3 * nw;
-        dbuf dsites, dmu, depc, dtens, dinfo;
+        dbuf dsites, dmu, depc, dwork, dinfo;
         upload(dsites, sites.data(), sizeof(double) * sites.size(), c->stream);
         dmu.alloc(sizeof(double) * 3 * ns);
         depc.alloc(sizeof(double) * 3 * ns);
-        dtens.alloc(sizeof(double) * 6 * (size_t)ns * ns);
+        dwork.alloc(water_scf_work_bytes(nw));
         dinfo.alloc(sizeof(int) * 2);
         water_scf_launch(nw, dsites.as<double>(), dmu.as<double>(), depc.as<double>(),
-                         dtens.as<double>(), dinfo.as<int>(), c->stream);
+                         dwork.as<double>(), dinfo.as<int>(), c->stream);
         int info[2] = {0, 0};
         PC_HIP(hipMemcpyAsync(info, dinfo.p, sizeof(info), hipMemcpyDeviceToHost, c->stream));
         std::vector<double> mu((size_t)3 * ns);

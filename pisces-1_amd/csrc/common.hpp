@@ -194,14 +194,16 @@ void pol3_grid_launch(const Pol3Dev &D, int nx, int ny, int nz, const double *d_
 bool water_sites_host(int nw, const double *xyz_ang, double *sites);
 // Device: induced-dipole SCF; d_sites 12*nw, outputs d_mu/d_epc 9*nw.
 void water_scf_launch(int nw, const double *d_sites, double *d_mu, double *d_epc,
-                      double *d_tensor, int *d_info, hipStream_t s);
+                      double *d_work, int *d_info, hipStream_t s);
 struct ScfTask {
     int nw;
     const double *sites;
-    double *mu, *epc, *tens;
+    double *mu, *epc, *work;
     int *info;
 };
-void water_scf_batched_launch(const ScfTask *d_tasks, int ntasks, hipStream_t s);
+void water_scf_batched_launch(const ScfTask *d_tasks, int ntasks, int max_waters, hipStream_t s);
+// bytes of ScfTask::work (d_work) that a cluster of nw waters needs (0 for small ones)
+size_t water_scf_work_bytes(int nw);
 int water_scf_max_waters();
 // Host: energy of the neutral cluster (E0, electrostatic, polarization,
 // dispersion) from the sites (12*nw, bohr) and the induced dipoles (9*nw).

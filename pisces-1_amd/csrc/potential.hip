@@ -17,6 +17,9 @@
 #include "common.hpp"
 #include "gmem.hpp"
 
+#include <algorithm>
+#include <mutex>
+
 namespace pisces {
 
 namespace {
@@ -41,7 +44,7 @@ __device__ inline double reff(double r, double r0)
 // |r| from r^2 and 1/|r| (0 at r = 0, where 1/|r| is infinite)
 __device__ __forceinline__ double norm_of(double r2, double ri) { return r2 > 0.0 ? r2 * ri : 0.0; }
 
-__device__ void potential_point(const PotParams &P, const PotDev &D, const SiteLds *__restrict__ S,
+__device__ __forceinline__ void potential_point(const PotParams &P, const PotDev &D, const SiteLds *__restrict__ S,
                                 int nx, int ny, int nz, const double *__restrict__ gx,
                                 const double *__restrict__ gy, const double *__restrict__ gz,
                                 double *__restrict__ v, float *__restrict__ v32, long long g)
@@ -169,228 +172,250 @@ potential_grid_batched_kernel(PotParams P, const PotTask *__restrict__ tasks)
 }
 
 // --------------------------------------------------------------------------
-// Induced dipoles of the rigid DPP waters, FP64, one workgroup.
+// Induced dipoles of the rigid DPP waters, FP64, one workgroup per cluster.
 // WaterCluster::CalcInducedDipoles (src/DPP.cpp:760-1065): field of the
 // permanent charges of the other waters at the polarizable sites (O, H1, H2),
 // then the 0.5-mixed fixed-point iteration mu <- 0.5 mu + 0.5 alpha (E_pc +
-// T mu) until the mean change drops below 1e-12.  The damped dipole tensors
-// T_ij (src/DPP.cpp:2377-2410) do not change during the iteration and are
-// computed once into d_tensor (6 doubles per ordered pair).
-constexpr int kScfThreads = 256;
-constexpr int kScfSharedSites = kScfThreads / 2;  // clusters solved with the dipoles in LDS
+// T mu) until the mean change drops below 1e-12.  The damped dipole tensor of a
+// pair (src/DPP.cpp:2377-2410) is T = a r r^T - b, a = 3 d1 / r^5, b = d2 / r^3,
+// and does not change during the iteration: each thread computes a and b of its
+// pairs once and keeps them in registers.
+//
+// The iteration is a serial chain of some fifty small steps on one CU, so its
+// cost is the length of a step.  The threads are split evenly over
+// the sites, 2^lg lanes of one wave per site; a lane sums its partners j = part,
+// part + 2^lg, ..., the lanes' sums meet by lane permutes, dipoles and the
+// waves' shares of the change are double-buffered in LDS, and every thread adds
+// those shares itself: one barrier per step.  A thread's first HELD pairs (all of
+// them up to 24 waters) stay in registers, as sqrt(a) r and b, which
+// leaves only the partner's dipole to read; of the rest, (a, b) of as many as
+// fit are kept in LDS and the remainder in `work`, laid out so that a wave reads
+// it contiguously.  us a launch, before (6-element tensors from global memory,
+// 256 threads, ten barriers a step) -> now: 24 waters 427 -> 91, 45 waters
+// 1834 -> 313.
+//
+// Two forms: 640 threads (three waves a SIMD, so that 12 pairs fit the registers)
+// up to 640 sites, 1024 threads beyond.
+template <int NT> struct Scf {
+    static constexpr int HELD = NT == 640 ? 9 : 6;      // pairs of a thread in registers
+    static constexpr int SLOT_BYTES = NT * 2 * (int)sizeof(double);
+    static constexpr int LDS = 152 * 1024;
+    // lanes per site, as a power of two: the most that fit
+    __host__ __device__ static int lg(int ns)
+    {
+        int l = 6;
+        while (l > 0 && (ns << l) > NT) --l;
+        return l;
+    }
+    __host__ __device__ static int pairs(int ns) { return (ns + (1 << lg(ns)) - 1) >> lg(ns); }
+    // pairs of a thread in LDS, beside the 9 ns doubles of positions and dipoles
+    __host__ __device__ static int slots(int ns)
+    {
+        const int left = (LDS - 8 * (9 * ns + 1)) / SLOT_BYTES, want = pairs(ns) - HELD;
+        return want < 0 ? 0 : want < left ? want : left;
+    }
+};
+constexpr int kScfSmall = 640, kScfLarge = 1024;
 constexpr double kA2B = 1.0 / 0.52917720859;
+constexpr double kPolO = 1.22 * kA2B * kA2B * kA2B, kPolH = 0.28 * kA2B * kA2B * kA2B;
 
-__device__ inline void site_params(int s, double &q, double &sig, double &alpha)
+// Sums over groups of 2^to lanes whose sub-groups of 2^from lanes hold equal
+// values: xor 1, 2 by DPP quad permutes, then (equal groups of 4 and 8) the half
+// row and row mirrors, then shuffles.
+template <int CTRL> __device__ __forceinline__ double dpp_add(double x)
 {
-    // src/Water.cpp:233-236 (chargeselector 2) with src/ttm_data.h:14-15, 51-52
-    const double a3 = kA2B * kA2B * kA2B;
-    const double polO = 1.22 * a3, polH = 0.28 * a3;
-    const double qH = 0.5742185854046506;
-    if (s == 0) { q = 0.0; sig = 0.0; alpha = polO; }
-    else if (s < 3) { q = qH; sig = polH; alpha = polH; }
-    else { q = -2.0 * qH; sig = polO; alpha = 0.0; }
+    const long long v = __builtin_bit_cast(long long, x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xF, 0xF, false);
+    return x + __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double scf_lanes(double x, int from, int to)
+{
+    if (from <= 0 && to > 0) x = dpp_add<0xB1>(x);
+    if (from <= 1 && to > 1) x = dpp_add<0x4E>(x);
+    if (from <= 2 && to > 2) x = dpp_add<0x141>(x);
+    if (from <= 3 && to > 3) x = dpp_add<0x140>(x);
+    if (from <= 4 && to > 4) x += __shfl_xor(x, 16, 64);
+    if (from <= 5 && to > 5) x += __shfl_xor(x, 32, 64);
+    return x;
 }
 
-__device__ inline double damp_cd(double r, double ai, double aj, double a)
+// polarizabilities (O, H1, H2), charges (H1, H2, M) and the charges' damping
+// polarizabilities: src/Water.cpp:233-236 (chargeselector 2) with
+// src/ttm_data.h:14-15, 51-52
+__device__ __forceinline__ double scf_alpha(int i) { return i % 3 == 0 ? kPolO : kPolH; }
+// 1 / sqrt(alpha alpha') of two sites by how many of them are oxygens (or M for
+// a charge): sqrt(1.22 * 0.28)
+constexpr double kSqrtOH = 0.58446556784809830;
+__device__ __forceinline__ double scf_damp_scale(int oxygens)
 {
-    const double A = pow(ai * aj, 1.0 / 6.0);
-    const double x = a * pow(r / A, 3);
-    return 1.0 - exp(-x);
-}
-__device__ inline double damp_dd(double r, double ai, double aj, double a)
-{
-    const double A = pow(ai * aj, 1.0 / 6.0);
-    const double x = a * pow(r / A, 3);
-    return 1.0 - (1 + x) * exp(-x);
+    constexpr double a3 = kA2B * kA2B * kA2B;
+    return oxygens == 2 ? 1.0 / kPolO : oxygens == 1 ? 1.0 / (kSqrtOH * a3) : 1.0 / kPolH;
 }
 
-__device__ void water_scf_body(int nw, const double *__restrict__ sites, double *__restrict__ mu_out,
-                               double *__restrict__ epc_out, double *__restrict__ tens,
+template <int NT>
+__device__ __forceinline__ void water_scf_body(int nw, const double *__restrict__ sites, double *__restrict__ mu_out,
+                               double *__restrict__ epc_out, double *__restrict__ work,
                                int *__restrict__ info)
 {
-    const int ns = 3 * nw;
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
     const double dampCD = 0.21, dampDD = 0.3;  // src/Water.cpp:243
-    __shared__ double red[kScfThreads];
-    __shared__ int s_done;
-    // tensors of every ordered pair (i at row, dipole j)
-    for (long long p = threadIdx.x; p < (long long)ns * ns; p += blockDim.x) {
-        const int i = (int)(p / ns), j = (int)(p % ns);
-        double *t = tens + 6 * p;
-        if (i == j) { for (int c = 0; c < 6; ++c) t[c] = 0.0; continue; }
-        double q, sg, ai, aj;
-        site_params(i % 3, q, sg, ai);
-        site_params(j % 3, q, sg, aj);
-        const double *xi = sites + 12 * (i / 3) + 3 * (i % 3);
-        const double *xj = sites + 12 * (j / 3) + 3 * (j % 3);
-        const double rx = xi[0] - xj[0], ry = xi[1] - xj[1], rz = xi[2] - xj[2];
-        const double r2 = rx * rx + ry * ry + rz * rz;
-        const double r5 = pow(r2, -2.5);
-        const double d1 = damp_dd(sqrt(r2), ai, aj, dampDD);
-        const double d2 = damp_cd(sqrt(r2), ai, aj, dampDD);
-        t[0] = (d1 * 3. * rx * rx - d2 * r2) * r5;
-        t[1] = (d1 * 3. * ry * ry - d2 * r2) * r5;
-        t[2] = (d1 * 3. * rz * rz - d2 * r2) * r5;
-        t[3] = d1 * 3. * rx * ry * r5;
-        t[4] = d1 * 3. * rx * rz * r5;
-        t[5] = d1 * 3. * ry * rz * r5;
+    const double qH = 0.5742185854046506;
+    constexpr int HELD = Scf<NT>::HELD;
+    const int ns = 3 * nw, lg = Scf<NT>::lg(ns), nu = Scf<NT>::pairs(ns);
+    // positions, two sets of dipoles (3 ns each), then the LDS pairs
+    extern __shared__ __align__(16) double scf_lds[];
+    __shared__ double red[2][NT / 64];
+    double *px = scf_lds, *m0 = scf_lds + 3 * ns;
+    f64x2 *slot = reinterpret_cast<f64x2 *>(scf_lds + 9 * ns + (ns & 1));
+    const int nslot = Scf<NT>::slots(ns), first = HELD + nslot;  // first pair in `work`
+    const int tid = threadIdx.x;
+    const int i = tid >> lg, part = tid & ((1 << lg) - 1);
+    const bool own = i < ns;
+    for (int k = tid; k < 3 * ns; k += NT) {
+        const int s = k / 3;
+        px[k] = sites[12 * (s / 3) + 3 * (s % 3) + k % 3];
     }
-    // permanent-charge field (src/DPP.cpp:830-865); each thread owns sites i
-    for (int i = threadIdx.x; i < ns; i += blockDim.x) {
-        double q, sg, ai;
-        site_params(i % 3, q, sg, ai);
-        const double *xi = sites + 12 * (i / 3) + 3 * (i % 3);
-        double f0 = 0, f1 = 0, f2 = 0;
-        for (int w = 0; w < nw; ++w)
-            for (int s = 0; s < 4; ++s) {
-                double qq, sig, a;
-                site_params(s, qq, sig, a);
-                if (qq == 0 || i / 3 == w) continue;
-                const double *pc = sites + 12 * w + 3 * s;
-                const double rx = xi[0] - pc[0], ry = xi[1] - pc[1], rz = xi[2] - pc[2];
-                const double t = qq * pow(rx * rx + ry * ry + rz * rz, -1.5);
-                const double dist = sqrt(rx * rx + ry * ry + rz * rz);
-                const double dmp = damp_cd(dist, ai, sig, dampCD);
-                f0 += t * rx * dmp;
-                f1 += t * ry * dmp;
-                f2 += t * rz * dmp;
-            }
+    __syncthreads();
+    const double ai = own ? scf_alpha(i) : 0.0;
+    const double xi = own ? px[3 * i] : 0.0, yi = own ? px[3 * i + 1] : 0.0, zi = own ? px[3 * i + 2] : 0.0;
+    // pair coefficients
+    auto pair = [&](int j) {
+        f64x2 c = {0.0, 0.0};
+        if (own && j < ns && j != i) {
+            const double rx = xi - px[3 * j], ry = yi - px[3 * j + 1], rz = zi - px[3 * j + 2];
+            const double r2 = rx * rx + ry * ry + rz * rz, ri = rsq64(r2), ri3 = ri * ri * ri;
+            const double x = dampDD * (r2 * r2 * ri) * scf_damp_scale((i % 3 == 0) + (j % 3 == 0)), ex = exp(-x);
+            c[0] = 3.0 * (1.0 - (1.0 + x) * ex) * ri3 * ri * ri;
+            c[1] = (1.0 - ex) * ri3;
+        }
+        return c;
+    };
+    double sx[HELD], sy[HELD], sz[HELD], sb[HELD];
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) {
+        const int j = part + (u << lg), jj = j < ns ? j : 0;
+        const f64x2 c = pair(j);
+        const double sa = sqrt(c[0]);
+        sx[u] = sa * (xi - px[3 * jj]);
+        sy[u] = sa * (yi - px[3 * jj + 1]);
+        sz[u] = sa * (zi - px[3 * jj + 2]);
+        sb[u] = c[1];
+        __builtin_amdgcn_sched_barrier(0);  // one pair's temporaries at a time
+    }
+    f64x2 *rest = reinterpret_cast<f64x2 *>(work) + tid;
+    for (int u = 0; u < nslot; ++u) slot[u * NT + tid] = pair(part + ((HELD + u) << lg));
+    for (int u = first; u < nu; ++u) rest[(size_t)(u - first) * NT] = pair(part + (u << lg));
+    // permanent-charge field (src/DPP.cpp:830-865)
+    double f0 = 0.0, f1 = 0.0, f2 = 0.0;
+    for (int q = part; q < 3 * nw; q += 1 << lg) {
+        const int w = q / 3, s = 1 + q % 3;  // H1, H2, M of water w
+        if (!own || i / 3 == w) continue;
+        const double *pc = sites + 12 * w + 3 * s;
+        const double rx = xi - pc[0], ry = yi - pc[1], rz = zi - pc[2];
+        const double r2 = rx * rx + ry * ry + rz * rz, ri = rsq64(r2);
+        const double x = dampCD * (r2 * r2 * ri) * scf_damp_scale((i % 3 == 0) + (s == 3));
+        const double t = (s == 3 ? -2.0 * qH : qH) * ri * ri * ri * (1.0 - exp(-x));
+        f0 += t * rx;
+        f1 += t * ry;
+        f2 += t * rz;
+    }
+    f0 = scf_lanes(f0, 0, lg);
+    f1 = scf_lanes(f1, 0, lg);
+    f2 = scf_lanes(f2, 0, lg);
+    double o0 = 0.5 * ai * f0, o1 = 0.5 * ai * f1, o2 = 0.5 * ai * f2;
+    if (own && part == 0) {
         epc_out[3 * i] = f0;
         epc_out[3 * i + 1] = f1;
         epc_out[3 * i + 2] = f2;
-        mu_out[3 * i] = 0.5 * ai * f0;
-        mu_out[3 * i + 1] = 0.5 * ai * f1;
-        mu_out[3 * i + 2] = 0.5 * ai * f2;
+        m0[3 * i] = o0;
+        m0[3 * i + 1] = o1;
+        m0[3 * i + 2] = o2;
     }
     __syncthreads();
     const int maxit = 5 * (ns + 10);
+    const double tol2 = (3e-12 * ns) * (3e-12 * ns);  // |change| / 3 / ns < 1e-12
     int it = 0, conv = 0;
-    if (ns <= kScfSharedSites) {
-        // ns <= 128: tps = floor(256 / ns) >= 2 threads per site, each summing
-        // the partners j = part, part + tps, ...; the dipoles live in LDS and
-        // the tps partial fields of a site are added there
-        __shared__ double smu[3 * kScfSharedSites];
-        __shared__ double pe[kScfThreads][3];
-        const int tps = kScfThreads / ns;
-        const int i = threadIdx.x / tps, part = threadIdx.x - i * tps;
-        const bool own = i < ns;
-        for (int idx = threadIdx.x; idx < 3 * ns; idx += blockDim.x) smu[idx] = mu_out[idx];
-        double q, sg, ai = 0.0;
-        if (own) site_params(i % 3, q, sg, ai);
-        __syncthreads();
-        for (it = 0; it < maxit; ++it) {
-            double e0 = 0, e1 = 0, e2 = 0;
-            if (own) {
-                const double *t = tens + 6LL * i * ns;
-                for (int j = part; j < ns; j += tps) {
-                    if (j == i) continue;
-                    const double m0 = smu[3 * j], m1 = smu[3 * j + 1], m2 = smu[3 * j + 2];
-                    const double *tj = t + 6 * j;
-                    e0 += tj[0] * m0 + tj[3] * m1 + tj[4] * m2;
-                    e1 += tj[3] * m0 + tj[1] * m1 + tj[5] * m2;
-                    e2 += tj[4] * m0 + tj[5] * m1 + tj[2] * m2;
-                }
-            }
-            pe[threadIdx.x][0] = e0;
-            pe[threadIdx.x][1] = e1;
-            pe[threadIdx.x][2] = e2;
-            __syncthreads();  // partial fields written, old dipoles read
-            double part_d = 0.0, n0 = 0, n1 = 0, n2 = 0;
-            if (own && part == 0) {
-                for (int p2 = 1; p2 < tps; ++p2) {
-                    e0 += pe[threadIdx.x + p2][0];
-                    e1 += pe[threadIdx.x + p2][1];
-                    e2 += pe[threadIdx.x + p2][2];
-                }
-                const double o0 = smu[3 * i], o1 = smu[3 * i + 1], o2 = smu[3 * i + 2];
-                n0 = 0.5 * o0 + 0.5 * ai * (epc_out[3 * i] + e0);
-                n1 = 0.5 * o1 + 0.5 * ai * (epc_out[3 * i + 1] + e1);
-                n2 = 0.5 * o2 + 0.5 * ai * (epc_out[3 * i + 2] + e2);
-                const double d0 = o0 - n0, d1 = o1 - n1, d2 = o2 - n2;
-                part_d = d0 * d0 + d1 * d1 + d2 * d2;
-            }
-            red[threadIdx.x] = part_d;
-            __syncthreads();  // every owner has read its old dipole
-            if (own && part == 0) {
-                smu[3 * i] = n0;
-                smu[3 * i + 1] = n1;
-                smu[3 * i + 2] = n2;
-            }
-            for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-                __syncthreads();
-                if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-            }
-            if (threadIdx.x == 0) s_done = (sqrt(red[0]) / 3 / ns < 1e-12) ? 1 : 0;
-            __syncthreads();
-            if (s_done) { conv = 1; break; }
-        }
-        for (int idx = threadIdx.x; idx < 3 * ns; idx += blockDim.x) mu_out[idx] = smu[idx];
-        if (threadIdx.x == 0) {
-            info[0] = conv;
-            info[1] = conv ? it + 1 : it;
-        }
-        return;
-    }
-    // larger clusters: mu_out holds the current dipoles; a private next value
-    // per owned site is kept in registers (at most ceil(ns/256) sites per thread)
-    constexpr int kPer = 4;
     for (it = 0; it < maxit; ++it) {
-        double nxt[kPer][3];
-        double part = 0.0;
-        int slot = 0;
-        for (int i = threadIdx.x; i < ns; i += blockDim.x, ++slot) {
-            double q, sg, ai;
-            site_params(i % 3, q, sg, ai);
-            double e0 = 0, e1 = 0, e2 = 0;
-            const double *t = tens + 6LL * i * ns;
-            for (int j = 0; j < ns; ++j) {
-                if (j == i) continue;
-                const double m0 = mu_out[3 * j], m1 = mu_out[3 * j + 1], m2 = mu_out[3 * j + 2];
-                const double *tj = t + 6 * j;
-                e0 += tj[0] * m0 + tj[3] * m1 + tj[4] * m2;
-                e1 += tj[3] * m0 + tj[1] * m1 + tj[5] * m2;
-                e2 += tj[4] * m0 + tj[5] * m1 + tj[2] * m2;
-            }
-            const double o0 = mu_out[3 * i], o1 = mu_out[3 * i + 1], o2 = mu_out[3 * i + 2];
-            nxt[slot][0] = 0.5 * o0 + 0.5 * ai * (epc_out[3 * i] + e0);
-            nxt[slot][1] = 0.5 * o1 + 0.5 * ai * (epc_out[3 * i + 1] + e1);
-            nxt[slot][2] = 0.5 * o2 + 0.5 * ai * (epc_out[3 * i + 2] + e2);
-            const double d0 = o0 - nxt[slot][0], d1 = o1 - nxt[slot][1], d2 = o2 - nxt[slot][2];
-            part += d0 * d0 + d1 * d1 + d2 * d2;
+        const double *cur = m0 + 3 * ns * (it & 1);
+        double *nxt = m0 + 3 * ns * ((it & 1) ^ 1);
+        double e0 = 0.0, e1 = 0.0, e2 = 0.0;
+        auto add = [&](int j, f64x2 c) {
+            const int jj = j < ns ? j : 0;  // c = 0 past the last site
+            const double u0 = cur[3 * jj], u1 = cur[3 * jj + 1], u2 = cur[3 * jj + 2];
+            const double rx = xi - px[3 * jj], ry = yi - px[3 * jj + 1], rz = zi - px[3 * jj + 2];
+            const double d = c[0] * (rx * u0 + ry * u1 + rz * u2);
+            e0 += d * rx - c[1] * u0;
+            e1 += d * ry - c[1] * u1;
+            e2 += d * rz - c[1] * u2;
+        };
+        if (own) {
+#pragma unroll
+            for (int u = 0; u < HELD; ++u)
+                if (u < nu) {
+                    const int j = part + (u << lg), jj = j < ns ? j : 0;
+                    const double u0 = cur[3 * jj], u1 = cur[3 * jj + 1], u2 = cur[3 * jj + 2];
+                    const double d = sx[u] * u0 + sy[u] * u1 + sz[u] * u2;
+                    e0 += d * sx[u] - sb[u] * u0;
+                    e1 += d * sy[u] - sb[u] * u1;
+                    e2 += d * sz[u] - sb[u] * u2;
+                }
+            for (int u = 0; u < nslot; ++u) add(part + ((HELD + u) << lg), slot[u * NT + tid]);
+#pragma unroll 4
+            for (int u = first; u < nu; ++u) add(part + (u << lg), rest[(size_t)(u - first) * NT]);
         }
-        red[threadIdx.x] = part;
-        __syncthreads();  // every thread has read the old dipoles
-        slot = 0;
-        for (int i = threadIdx.x; i < ns; i += blockDim.x, ++slot) {
-            mu_out[3 * i] = nxt[slot][0];
-            mu_out[3 * i + 1] = nxt[slot][1];
-            mu_out[3 * i + 2] = nxt[slot][2];
+        e0 = scf_lanes(e0, 0, lg);
+        e1 = scf_lanes(e1, 0, lg);
+        e2 = scf_lanes(e2, 0, lg);
+        const double n0 = 0.5 * o0 + 0.5 * ai * (f0 + e0);
+        const double n1 = 0.5 * o1 + 0.5 * ai * (f1 + e1);
+        const double n2 = 0.5 * o2 + 0.5 * ai * (f2 + e2);
+        // the lanes of a site hold the same change: sum over the wave's sites
+        double d = (o0 - n0) * (o0 - n0) + (o1 - n1) * (o1 - n1) + (o2 - n2) * (o2 - n2);
+        d = scf_lanes(own ? d : 0.0, lg, 6);
+        if (own && part == 0) {
+            nxt[3 * i] = n0;
+            nxt[3 * i + 1] = n1;
+            nxt[3 * i + 2] = n2;
         }
-        for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-            __syncthreads();
-            if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        o0 = n0;
+        o1 = n1;
+        o2 = n2;
+        if ((tid & 63) == 0) red[it & 1][tid >> 6] = d;
+        __syncthreads();  // the new dipoles and every wave's share are in LDS
+        double s2[2] = {0.0, 0.0};
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) s2[w & 1] += red[it & 1][w];
+        if (s2[0] + s2[1] < tol2) {
+            conv = 1;
+            break;
         }
-        if (threadIdx.x == 0) s_done = (sqrt(red[0]) / 3 / ns < 1e-12) ? 1 : 0;
-        __syncthreads();
-        if (s_done) { conv = 1; break; }
     }
-    if (threadIdx.x == 0) {
+    if (own && part == 0) {
+        mu_out[3 * i] = o0;
+        mu_out[3 * i + 1] = o1;
+        mu_out[3 * i + 2] = o2;
+    }
+    if (tid == 0) {
         info[0] = conv;
         info[1] = conv ? it + 1 : it;
     }
 }
 
-__global__ void __launch_bounds__(kScfThreads)
+template <int NT>
+__global__ void __launch_bounds__(NT)
 water_scf_kernel(int nw, const double *__restrict__ sites, double *__restrict__ mu_out,
-                 double *__restrict__ epc_out, double *__restrict__ tens, int *__restrict__ info)
+                 double *__restrict__ epc_out, double *__restrict__ work, int *__restrict__ info)
 {
-    water_scf_body(nw, sites, mu_out, epc_out, tens, info);
+    water_scf_body<NT>(nw, sites, mu_out, epc_out, work, info);
 }
 
 // one cluster per workgroup
-__global__ void __launch_bounds__(kScfThreads) water_scf_batched_kernel(const ScfTask *__restrict__ tasks)
+template <int NT>
+__global__ void __launch_bounds__(NT) water_scf_batched_kernel(const ScfTask *__restrict__ tasks)
 {
     const ScfTask &t = tasks[blockIdx.x];
-    water_scf_body(t.nw, t.sites, t.mu, t.epc, t.tens, t.info);
+    water_scf_body<NT>(t.nw, t.sites, t.mu, t.epc, t.work, t.info);
 }
 
 }  // namespace
@@ -417,23 +442,63 @@ void potential_grid_batched_launch(const PotParams &P, const PotTask *d_tasks, i
     PC_HIP(hipGetLastError());
 }
 
-void water_scf_batched_launch(const ScfTask *d_tasks, int ntasks, hipStream_t s)
+namespace {
+// Dynamic LDS of a launch whose largest cluster has ns sites: all of it once
+// the pairs of some cluster size up to that overflow the registers.
+template <int NT> size_t scf_lds_bytes(int ns)
+{
+    static std::once_flag once;
+    std::call_once(once, [] {
+        for (const void *k : {reinterpret_cast<const void *>(water_scf_kernel<NT>),
+                              reinterpret_cast<const void *>(water_scf_batched_kernel<NT>)})
+            PC_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, Scf<NT>::LDS));
+    });
+    for (int m = 1; m <= ns; ++m)
+        if (Scf<NT>::slots(m) > 0) return Scf<NT>::LDS;
+    return (size_t)9 * ns * sizeof(double);
+}
+template <int NT> size_t scf_work_bytes(int ns)
+{
+    const int n = Scf<NT>::pairs(ns) - Scf<NT>::HELD - Scf<NT>::slots(ns);
+    return n > 0 ? (size_t)n * Scf<NT>::SLOT_BYTES : 0;
+}
+}  // namespace
+
+int water_scf_max_waters() { return kScfLarge / 3; }
+int potential_max_sites() { return kMaxSites; }
+
+// for either form: a batch takes the one its largest cluster needs
+size_t water_scf_work_bytes(int nw)
+{
+    const size_t l = scf_work_bytes<kScfLarge>(3 * nw);
+    return 3 * nw > kScfSmall ? l : std::max(l, scf_work_bytes<kScfSmall>(3 * nw));
+}
+
+void water_scf_batched_launch(const ScfTask *d_tasks, int ntasks, int max_waters, hipStream_t s)
 {
     if (ntasks <= 0) return;
-    hipLaunchKernelGGL(water_scf_batched_kernel, dim3(ntasks), dim3(kScfThreads), 0, s, d_tasks);
+    const int ns = 3 * max_waters;
+    if (ns <= kScfSmall)
+        hipLaunchKernelGGL((water_scf_batched_kernel<kScfSmall>), dim3(ntasks), dim3(kScfSmall),
+                           scf_lds_bytes<kScfSmall>(ns), s, d_tasks);
+    else
+        hipLaunchKernelGGL((water_scf_batched_kernel<kScfLarge>), dim3(ntasks), dim3(kScfLarge),
+                           scf_lds_bytes<kScfLarge>(ns), s, d_tasks);
     PC_HIP(hipGetLastError());
 }
 
-int water_scf_max_waters() { return 4 * kScfThreads / 3; }
-int potential_max_sites() { return kMaxSites; }
-
-void water_scf_launch(int nw, const double *d_sites, double *d_mu, double *d_epc,
-                      double *d_tensor, int *d_info, hipStream_t s)
+void water_scf_launch(int nw, const double *d_sites, double *d_mu, double *d_epc, double *d_work,
+                      int *d_info, hipStream_t s)
 {
-    PC_REQUIRE(nw > 0 && 3 * nw <= 4 * kScfThreads, PISCES_ERR_UNSUPPORTED,
+    PC_REQUIRE(nw > 0 && nw <= water_scf_max_waters(), PISCES_ERR_UNSUPPORTED,
                "too many waters for the dipole solve");
-    hipLaunchKernelGGL(water_scf_kernel, dim3(1), dim3(kScfThreads), 0, s, nw, d_sites, d_mu,
-                       d_epc, d_tensor, d_info);
+    const int ns = 3 * nw;
+    if (ns <= kScfSmall)
+        hipLaunchKernelGGL((water_scf_kernel<kScfSmall>), dim3(1), dim3(kScfSmall),
+                           scf_lds_bytes<kScfSmall>(ns), s, nw, d_sites, d_mu, d_epc, d_work, d_info);
+    else
+        hipLaunchKernelGGL((water_scf_kernel<kScfLarge>), dim3(1), dim3(kScfLarge),
+                           scf_lds_bytes<kScfLarge>(ns), s, nw, d_sites, d_mu, d_epc, d_work, d_info);
     PC_HIP(hipGetLastError());
 }
 

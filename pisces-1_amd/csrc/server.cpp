@@ -232,7 +232,7 @@ struct Prep {
     std::vector<double> sites, q, rep;
     std::vector<int> iq, id, irep, ipps;
     size_t o_sites, o_q, o_iq, o_id, o_rep, o_irep, o_ipps, o_ion, o_ionq;  // upload offsets
-    size_t o_mu, o_epc, o_tens, o_info;                                   // work offsets
+    size_t o_mu, o_epc, o_work, o_info;                                   // work offsets
 };
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -275,7 +275,7 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
         auto wput = [&](size_t bytes) { const size_t o = wk; wk += align256(bytes); return o; };
         r.o_mu = wput(sizeof(double) * 3 * ns);
         r.o_epc = wput(sizeof(double) * 3 * ns);
-        r.o_tens = wput(sizeof(double) * 6 * (size_t)ns * ns);
+        r.o_work = wput(water_scf_work_bytes(nw));
         r.o_info = wput(sizeof(int) * 2);
     }
     P.ion_r = 2.9;  // Bloomfield r_Na, src/NaCl.cpp:95
@@ -292,12 +292,14 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
     ScfTask *scf = reinterpret_cast<ScfTask *>(h);
     PotTask *pot = reinterpret_cast<PotTask *>(h + align256(sizeof(ScfTask) * nb));
     long long max_ng = 0;
+    int max_nw = 0;
     for (int i = 0; i < nb; ++i) {
         Prep &r = batch[i];
         auto cp = [&](size_t off, const void *src, size_t bytes) {
             if (bytes) std::memcpy(h + off, src, bytes);
         };
         const int nw = r.p->req.nw, nion = r.p->req.nion;
+        max_nw = std::max(max_nw, nw);
         cp(r.o_sites, r.sites.data(), sizeof(double) * r.sites.size());
         cp(r.o_q, r.q.data(), sizeof(double) * r.q.size());
         cp(r.o_iq, r.iq.data(), sizeof(int) * r.iq.size());
@@ -310,7 +312,7 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
         double *mu = reinterpret_cast<double *>(w + r.o_mu);
         scf[i] = ScfTask{nw, reinterpret_cast<const double *>(d + r.o_sites), mu,
                          reinterpret_cast<double *>(w + r.o_epc),
-                         reinterpret_cast<double *>(w + r.o_tens),
+                         reinterpret_cast<double *>(w + r.o_work),
                          reinterpret_cast<int *>(w + r.o_info)};
         const GridShape &g = *r.res->shape;
         PotTask t{};
@@ -338,7 +340,7 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
     PC_HIP(hipMemcpyAsync(d, h, up, hipMemcpyHostToDevice, sv->stream));
     {
         ProfScope ps(PK_SCF, sv->stream, 0.0);
-        water_scf_batched_launch(reinterpret_cast<const ScfTask *>(d), nb, sv->stream);
+        water_scf_batched_launch(reinterpret_cast<const ScfTask *>(d), nb, max_nw, sv->stream);
     }
     {
         double bytes = 0;  // V written in FP64 and FP32, read once more with diag H written
