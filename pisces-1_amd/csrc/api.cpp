@@ -277,25 +277,42 @@ int build_potential_impl(pisces_ctx *c, const int flags[6], const double *potpar
                  ds.as<double>(), dq.as<double>(), diq.as<int>(), dd.as<double>(), did.as<int>(),
                  drep.as<double>(), direp.as<int>(), dipps.as<int>(), dix.as<double>(),
                  diq2.as<double>()};
-        potential_grid_launch(P, D, c->n[0], c->n[1], c->n[2], c->dx[0].as<double>(),
-                              c->dx[1].as<double>(), c->dx[2].as<double>(), c->dV64.as<double>(),
-                              nullptr, c->stream);
+        const int n3p = np > 0 ? pol3_padded(np) : 0;
+        PC_REQUIRE(n3p <= kPol3MaxN, PISCES_ERR_UNSUPPORTED, "too many polarizable sites");
+        std::vector<double> rp((size_t)3 * np), ep((size_t)n3p, 0.0);
+        int *flag = reinterpret_cast<int *>(c->hsmall);
+        dbuf dalpha, dtmp, dflag;
         if (np > 0) {
             // SetupDPPGTOP case 3 (src/Potential.cpp:387-432): InvA of the
-            // polarizable sites on the host, the grid sum on the matrix cores
-            const int n3p = pol3_padded(np);
-            PC_REQUIRE(n3p <= kPol3MaxN, PISCES_ERR_UNSUPPORTED, "too many polarizable sites");
-            std::vector<double> rp((size_t)3 * np), ep((size_t)n3p, 0.0), inv((size_t)n3p * n3p);
+            // polarizable sites, inverted before the grid pass so that the host
+            // learns during that pass whether it was positive definite
             for (int i = 0; i < np; ++i)
                 for (int k = 0; k < 3; ++k) {
                     rp[3 * i + k] = sites[3 * ip[i] + k];
                     ep[3 * i + k] = epc[3 * i + k];
                 }
-            PC_REQUIRE(pol3_inva_host(np, rp.data(), alpha, n3p, inv.data()), PISCES_ERR_NUMERIC,
-                       "singular polarization matrix");
             upload(drp, rp.data(), sizeof(double) * rp.size(), c->stream);
             upload(depc, ep.data(), sizeof(double) * ep.size(), c->stream);
-            upload(dinv, inv.data(), sizeof(double) * inv.size(), c->stream);
+            upload(dalpha, alpha, sizeof(double) * np, c->stream);
+            dinv.alloc(sizeof(double) * (size_t)n3p * n3p);
+            dtmp.alloc(sizeof(double) * 2 * (size_t)n3p * n3p);
+            dflag.alloc(sizeof(int));
+            pol3_inva_launch(np, drp.as<double>(), dalpha.as<double>(), n3p, dtmp.as<double>(),
+                             dinv.as<double>(), dflag.as<int>(), c->stream);
+            PC_HIP(hipMemcpyAsync(flag, dflag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        }
+        potential_grid_launch(P, D, c->n[0], c->n[1], c->n[2], c->dx[0].as<double>(),
+                              c->dx[1].as<double>(), c->dx[2].as<double>(), c->dV64.as<double>(),
+                              nullptr, c->stream);
+        if (np > 0) {
+            c->sync();
+            if (*flag) {
+                std::vector<double> inv((size_t)n3p * n3p);
+                PC_REQUIRE(pol3_inva_host(np, rp.data(), alpha, n3p, inv.data()), PISCES_ERR_NUMERIC,
+                           "singular polarization matrix");
+                upload(dinv, inv.data(), sizeof(double) * inv.size(), c->stream);
+                c->sync();  // inv goes out of scope
+            }
             Pol3Dev Q{np, n3p, P.damp_type, 0, P.pdamp, vpol_ww, drp.as<double>(),
                       depc.as<double>(), dinv.as<double>()};
             {

@@ -184,6 +184,11 @@ inline int pol3_padded(int np) { return (3 * np + 15) / 16 * 16; }
 // matrix is singular.
 bool pol3_inva_host(int np, const double *rpol, const double *alpha, int n3p, double *inva);
 bool sym_inverse(int n, std::vector<double> &A, int n3p, double *inva, int method);
+// Device: the same InvA into d_inva (n3p x n3p; d_tmp: two such matrices).
+// *d_flag is 0 where the matrix was positive definite and the inverse finite;
+// otherwise d_inva holds no result (pol3_inva_host decides).
+void pol3_inva_launch(int np, const double *d_rpol, const double *d_alpha, int n3p, double *d_tmp,
+                      double *d_inva, int *d_flag, hipStream_t s);
 // Device: d_v[g] += -E^T InvA E / 2 - vpolww at every grid point, E the
 // electron's damped field at the sites plus epc.
 void pol3_grid_launch(const Pol3Dev &D, int nx, int ny, int nz, const double *d_x,
