@@ -62,4 +62,21 @@ __device__ __forceinline__ double rsq64(double x)
     return y;
 }
 
+// x plus x of the lane that a DPP control names, and sums over groups of lanes
+// by them (the LDS stays out of it): quad permutes 1,0,3,2 (0xB1) and 2,3,0,1
+// (0x4E), then, on equal quads and equal groups of 8, the half-row (0x141) and
+// row (0x140) mirrors.
+template <int CTRL> __device__ __forceinline__ double dpp_add(double x)
+{
+    const long long v = __builtin_bit_cast(long long, x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xF, 0xF, false);
+    return x + __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+// the sum of the 16 lanes of a row, in all of them
+__device__ __forceinline__ double row_sum(double x)
+{
+    return dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(x))));
+}
+
 }  // namespace pisces

@@ -5,15 +5,18 @@
 // r - site i, g the damped R^-3), mu = InvA E, Vpol = -E.mu / 2 -
 // VpolWaterWater.  Over a tile of grid points that is the product E InvA (points
 // x 3np times 3np x 3np) followed by a row-wise dot with E: FP64 matrix-core
-// work of 2 (3np)^2 flops per point.  A workgroup takes 16 RB points (RB = 1
-// by default): it builds their E rows in LDS (odd pitch: the 16 rows that one
-// matrix-core operand reads fall on distinct banks), then each of its 8 or 16
-// waves takes 16-column blocks of InvA, streams them from L2 (InvA is shared by all
-// workgroups: at most 2.6 MB) as the B operand of v_mfma_f64_16x16x4 against
-// the 16-point row blocks of E, and folds each 16 x 16 result into the
-// per-point dot at once.
-// InvA is symmetric, so only its upper block triangle is multiplied: (3np)^2
-// (1 + 16 / 3np) flops per point.
+// work of 2 (3np)^2 flops per point.  InvA is symmetric, so only its upper block
+// triangle is multiplied: (3np)^2 (1 + 16 / 3np) flops per point.  A workgroup
+// takes 16 RB points (RB = 2 by default): it builds their E rows in LDS (odd
+// pitch: the 16 rows that one matrix-core operand reads fall on distinct banks),
+// then its waves split the list of 16 x 16 InvA tiles evenly, stream them from
+// L2 (InvA is shared by all workgroups: at most 2.6 MB) one tile ahead as the B
+// operand of v_mfma_f64_16x16x4 against the row blocks of E, and fold each column
+// block's sum into the per-point dot.  us at 216 / 405 dimensions, before (16
+// points, whole column blocks per wave, 64-bit divisions for every E value) ->
+// now: 423 / 4360 -> 341 / 3311, which is 0.57 / 0.64 of the 72.7 TFLOP/s that a
+// large FP64 matrix product reaches; the E rows and the ends of a workgroup are
+// the rest.
 #include "common.hpp"
 #include "gmem.hpp"
 
@@ -24,7 +27,7 @@ namespace pisces {
 
 namespace {
 
-constexpr int kLdsMax = 160 * 1024 - 16 * 64 * (int)sizeof(double);  // E rows + red (16 waves)
+constexpr int kLdsMax = 160 * 1024 - (16 + 3) * 64 * (int)sizeof(double);  // E rows, red (16 waves), pt
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -48,6 +51,7 @@ pol3_grid_kernel(Pol3Dev D, int nx, int ny, int nz, const double *__restrict__ g
     constexpr int kP3Pts = 16 * RB, kP3Threads = NT, NW = NT / 64;
     extern __shared__ double Es[];  // kP3Pts rows of n3p (+1) values
     __shared__ double red[kP3Threads / 64][kP3Pts];
+    __shared__ double pt[kP3Pts][3];  // the points' coordinates
     const int n3p = D.n3p, ldE = n3p + 1, np = D.np, n3 = 3 * np;
     const long long ng = (long long)nx * ny * nz;
     const long long g0 = (long long)blockIdx.x * kP3Pts;
@@ -55,99 +59,105 @@ pol3_grid_kernel(Pol3Dev D, int nx, int ny, int nz, const double *__restrict__ g
 
     // E rows: the electron's field at the sites (src/Potential.cpp:1531-1562,
     // DampType 1: R^-3 (1 - exp(-p R^3)); 2: Reff^-3 inside the damping radius)
-    // plus the permanent-charge field; rows past the grid stay 0
-    for (int idx = threadIdx.x; idx < kP3Pts * np; idx += kP3Threads) {
-        const int p = idx / np, i = idx - p * np;
-        const long long g = g0 + p;
-        double e0 = 0.0, e1 = 0.0, e2 = 0.0;
-        if (g < ng) {
-            const int ix = (int)(g % nx), iy = (int)((g / nx) % ny);
-            const int iz = (int)(g / ((long long)nx * ny));
-            const double rx = gx[ix] - rp[3 * i], ry = gy[iy] - rp[3 * i + 1],
-                         rz = gz[iz] - rp[3 * i + 2];
-            const double R2 = rx * rx + ry * ry + rz * rz;
-            double gij = 0.0;  // R = 0: the field's limit, 0
-            if (R2 > 0.0) {
-                const double ri = rsq64(R2), R = R2 * ri;
-                if (D.damp_type == 1) {
-                    gij = ri * ri * ri * (1.0 - exp(-D.pdamp * R * R2));
-                } else if (R < D.pdamp) {
-                    const double re = reff3(R, D.pdamp);
-                    gij = 1.0 / (re * re * re);
-                } else {
-                    gij = ri * ri * ri;
-                }
-            }
-            e0 = gij * rx + ep[3 * i];
-            e1 = gij * ry + ep[3 * i + 1];
-            e2 = gij * rz + ep[3 * i + 2];
-        }
-        double *row = Es + p * ldE + 3 * i;
-        row[0] = e0;
-        row[1] = e1;
-        row[2] = e2;
-    }
-    const int padw = n3p - n3;
-    for (int idx = threadIdx.x; idx < kP3Pts * padw; idx += kP3Threads) {
-        const int p = idx / padw;
-        Es[p * ldE + n3 + (idx - p * padw)] = 0.0;
+    // plus the permanent-charge field; rows past the grid repeat its last point
+    if (threadIdx.x < kP3Pts) {
+        const unsigned g = (unsigned)(g0 + threadIdx.x < ng ? g0 + threadIdx.x : ng - 1);
+        const unsigned iy = g / (unsigned)nx, iz = iy / (unsigned)ny;
+        pt[threadIdx.x][0] = gx[g - iy * nx];
+        pt[threadIdx.x][1] = gy[iy - iz * ny];
+        pt[threadIdx.x][2] = gz[iz];
     }
     __syncthreads();
+    for (int idx = threadIdx.x; idx < kP3Pts * np; idx += kP3Threads) {
+        const int p = idx % kP3Pts, i = idx / kP3Pts;
+        const double rx = pt[p][0] - rp[3 * i], ry = pt[p][1] - rp[3 * i + 1], rz = pt[p][2] - rp[3 * i + 2];
+        const double R2 = rx * rx + ry * ry + rz * rz;
+        double gij = 0.0;  // R = 0: the field's limit, 0
+        if (R2 > 0.0) {
+            const double ri = rsq64(R2), R = R2 * ri;
+            if (D.damp_type == 1) {
+                gij = ri * ri * ri * (1.0 - exp(-D.pdamp * R * R2));
+            } else if (R < D.pdamp) {
+                const double re = reff3(R, D.pdamp);
+                gij = rcp64(re * re * re);
+            } else {
+                gij = ri * ri * ri;
+            }
+        }
+        double *row = Es + p * ldE + 3 * i;
+        row[0] = gij * rx + ep[3 * i];
+        row[1] = gij * ry + ep[3 * i + 1];
+        row[2] = gij * rz + ep[3 * i + 2];
+    }
+    for (int idx = threadIdx.x; idx < kP3Pts * (n3p - n3); idx += kP3Threads)
+        Es[(idx % kP3Pts) * ldE + n3 + idx / kP3Pts] = 0.0;
+    __syncthreads();
 
-    // E^T InvA E over the upper block triangle of the symmetric InvA: column
-    // block cb takes rows k < 16 cb twice and its diagonal 16 x 16 tile once.
-    // Block cb costs cb + 1 row blocks, so the waves take the blocks of each
-    // group of four in alternating order to even out their work.
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // E^T InvA E over the upper block triangle of the symmetric InvA: 16 x 16
+    // tiles above the diagonal count twice, those on it once.  The tiles, column
+    // by column, are one list that the waves split evenly; a wave folds its sum
+    // over the rows k of a column block into the per-point dot when it leaves
+    // the column.  The next tile's InvA values are requested before the current
+    // ones are used.
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, lq = lane >> 4;
-    const gptr<const double> A = glb(D.inva);
+    const gptr<const double> A = glb(D.inva) + (lq * n3p + l16);
     double sr[RB][4];
+    f64x4 o[RB];
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
+    for (int b = 0; b < RB; ++b) {
+        o[b] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int r = 0; r < 4; ++r) sr[b][r] = 0.0;
+    }
     const double *ea = Es + l16 * ldE + lq;  // row block b: + 16 b ldE
-    const int ncb = n3p / 16;
-    for (int j = 0; NW * j < ncb; ++j) {
-        const int cb = (j & 1) ? NW * j + NW - 1 - wave : NW * j + wave;
-        if (cb >= ncb) continue;
-        f64x4 o[RB], d[RB];
+    const int ncb = n3p / 16, ntile = ncb * (ncb + 1) / 2;
+    const int t0 = ntile * wave / NW, t1 = ntile * (wave + 1) / NW;
+    // tile t0: column block cb, row block kb <= cb
+    int cb = 0, kb = t0;
+    while (kb > cb) {
+        kb -= cb + 1;
+        ++cb;
+    }
+    double nv[4];
+    if (t0 < t1)
 #pragma unroll
-        for (int b = 0; b < RB; ++b) {
-            o[b] = f64x4{0.0, 0.0, 0.0, 0.0};
-            d[b] = f64x4{0.0, 0.0, 0.0, 0.0};
-        }
-        const gptr<const double> bc = A + (long long)lq * n3p + 16 * cb + l16;
-        const int kd = 16 * cb;
-#pragma unroll 8
-        for (int k0 = 0; k0 < kd; k0 += 4) {
-            const double bv = bc[(long long)k0 * n3p];  // InvA[k0 + lq][16 cb + l16]
-#pragma unroll
-            for (int b = 0; b < RB; ++b)
-                o[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ea[16 * b * ldE + k0], bv, o[b], 0, 0, 0);
-        }
-#pragma unroll
-        for (int k0 = kd; k0 < kd + 16; k0 += 4) {
-            const double bv = bc[(long long)k0 * n3p];
-#pragma unroll
-            for (int b = 0; b < RB; ++b)
-                d[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ea[16 * b * ldE + k0], bv, d[b], 0, 0, 0);
-        }
-        // o[b][r], d[b][r]: point 16 b + lq + 4 r, column 16 cb + l16
+        for (int q = 0; q < 4; ++q) nv[q] = A[(16 * kb + 4 * q) * n3p + 16 * cb];
+    auto fold = [&](double w) {
         const int c = 16 * cb + l16;
 #pragma unroll
         for (int b = 0; b < RB; ++b)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                sr[b][r] += (2.0 * o[b][r] + d[b][r]) * Es[(16 * b + lq + 4 * r) * ldE + c];
+            for (int r = 0; r < 4; ++r) {
+                sr[b][r] += (w * o[b][r]) * Es[(16 * b + lq + 4 * r) * ldE + c];
+                o[b][r] = 0.0;
+            }
+    };
+    for (int t = t0; t < t1; ++t) {
+        const bool diag = kb == cb;
+        const int nk = diag ? 0 : kb + 1, nc = diag ? cb + 1 : cb;  // the next tile
+        double bv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) bv[q] = nv[q];
+        if (t + 1 < t1)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) nv[q] = A[(16 * nk + 4 * q) * n3p + 16 * nc];
+        if (diag) fold(2.0);  // the tiles above the diagonal so far
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+                o[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ea[16 * b * ldE + 16 * kb + 4 * q], bv[q], o[b], 0, 0, 0);
+        if (diag) fold(1.0);
+        if (t + 1 == t1 && !diag) fold(2.0);
+        kb = nk;
+        cb = nc;
     }
     // sum over the 16 columns a lane group holds, then over the waves
 #pragma unroll
-    for (int off = 1; off < 16; off <<= 1)
+    for (int b = 0; b < RB; ++b)
 #pragma unroll
-        for (int b = 0; b < RB; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sr[b][r] += __shfl_xor(sr[b][r], off, 64);
+        for (int r = 0; r < 4; ++r) sr[b][r] = row_sum(sr[b][r]);
     if (l16 == 0)
 #pragma unroll
         for (int b = 0; b < RB; ++b)
@@ -179,47 +189,40 @@ void pol3_grid_launch(const Pol3Dev &D, int nx, int ny, int nz, const double *d_
                             reinterpret_cast<const void *>(pol3_grid_kernel<2, 256>),
                             reinterpret_cast<const void *>(pol3_grid_kernel<4, 256>),
                             reinterpret_cast<const void *>(pol3_grid_kernel<1, 512>),
-                            reinterpret_cast<const void *>(pol3_grid_kernel<1, 1024>)};
+                            reinterpret_cast<const void *>(pol3_grid_kernel<2, 512>),
+                            reinterpret_cast<const void *>(pol3_grid_kernel<4, 512>),
+                            reinterpret_cast<const void *>(pol3_grid_kernel<1, 1024>),
+                            reinterpret_cast<const void *>(pol3_grid_kernel<2, 1024>),
+                            reinterpret_cast<const void *>(pol3_grid_kernel<4, 1024>)};
         for (const void *k : ks)
             PC_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax));
     });
-    // RB 16-point row blocks per workgroup (PISCES_POL3_RB = 1, 2 or 4).  The E
-    // rows in LDS bound how many workgroups a CU holds, and that decides the
-    // speed: 16-point tiles (1) measured 1.27x / 1.16x faster than 32-point
-    // ones at 216 / 405 polarizable dimensions, 64-point tiles slower still,
-    // although each InvA fragment then feeds fewer matrix-core products.
+    // RB 16-point row blocks per workgroup (PISCES_POL3_RB = 1, 2 or 4): each
+    // InvA fragment from the L2 feeds RB products, the E rows in LDS bound the
+    // workgroups per CU.  us at 216 (64^3) / 405 dimensions (96^3), RB 1, 2, 4
+    // with the threads below: 359 / 3377, 341 / 3311, 381 / 3325.
     const char *rb_e = std::getenv("PISCES_POL3_RB");  // read per build: not a hot path
     const int rb_env = rb_e ? std::atoi(rb_e) : 0;
-    // threads per workgroup (PISCES_POL3_NT = 256, 512 or 1024): the waves of a
-    // workgroup share its column blocks, and more resident waves hide the L2
-    // latency of the InvA operand.  Measured at 16-point tiles: 256 / 512 /
-    // 1024 threads 0.578 / 0.419 / 0.487 ms at 216 dimensions (14 blocks),
-    // 8.74 / 4.66 / 4.44 ms at 405 (26 blocks): 1024 from 24 blocks on.
+    // threads per workgroup (PISCES_POL3_NT = 256, 512 or 1024): with 32-point
+    // tiles 512 / 1024 threads take 341 / 400 us at 216 dimensions (two
+    // workgroups a CU fit) and 3655 / 3311 us at 405 (one does): 1024 from 24
+    // column blocks on.
     const char *nt_e = std::getenv("PISCES_POL3_NT");
     const int nt_v = nt_e ? std::atoi(nt_e) : (D.n3p / 16 >= 24 ? 1024 : 512);
     const int nt = (nt_v == 256 || nt_v == 1024) ? nt_v : 512;
     const size_t row = (size_t)(D.n3p + 1) * sizeof(double);
-    int rb = (rb_env == 1 || rb_env == 2 || rb_env == 4) ? rb_env : 1;
+    int rb = (rb_env == 1 || rb_env == 2 || rb_env == 4) ? rb_env : 2;
     while (rb > 1 && 16 * rb * row > (size_t)kLdsMax) rb /= 2;
     const long long ng = (long long)nx * ny * nz;
     const int pts = 16 * rb;
     const unsigned blocks = (unsigned)((ng + pts - 1) / pts);
     const size_t lds = (size_t)pts * row;
-    if (rb == 1 && nt == 1024)
-        hipLaunchKernelGGL((pol3_grid_kernel<1, 1024>), dim3(blocks), dim3(1024), lds, s, D, nx, ny,
-                           nz, d_x, d_y, d_z, d_v);
-    else if (rb == 1 && nt == 512)
-        hipLaunchKernelGGL((pol3_grid_kernel<1, 512>), dim3(blocks), dim3(512), lds, s, D, nx, ny,
-                           nz, d_x, d_y, d_z, d_v);
-    else if (rb == 4)
-        hipLaunchKernelGGL((pol3_grid_kernel<4, 256>), dim3(blocks), dim3(256), lds, s, D, nx, ny,
-                           nz, d_x, d_y, d_z, d_v);
-    else if (rb == 2)
-        hipLaunchKernelGGL((pol3_grid_kernel<2, 256>), dim3(blocks), dim3(256), lds, s, D, nx, ny,
-                           nz, d_x, d_y, d_z, d_v);
-    else
-        hipLaunchKernelGGL((pol3_grid_kernel<1, 256>), dim3(blocks), dim3(256), lds, s, D, nx, ny,
-                           nz, d_x, d_y, d_z, d_v);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(nt), lds, s, D, nx, ny, nz, d_x, d_y, d_z, d_v);
+    };
+    if (nt == 1024) go(rb == 1 ? pol3_grid_kernel<1, 1024> : rb == 2 ? pol3_grid_kernel<2, 1024> : pol3_grid_kernel<4, 1024>);
+    else if (nt == 512) go(rb == 1 ? pol3_grid_kernel<1, 512> : rb == 2 ? pol3_grid_kernel<2, 512> : pol3_grid_kernel<4, 512>);
+    else go(rb == 1 ? pol3_grid_kernel<1, 256> : rb == 2 ? pol3_grid_kernel<2, 256> : pol3_grid_kernel<4, 256>);
     PC_HIP(hipGetLastError());
 }
 

@@ -222,13 +222,6 @@ constexpr double kPolO = 1.22 * kA2B * kA2B * kA2B, kPolH = 0.28 * kA2B * kA2B *
 // Sums over groups of 2^to lanes whose sub-groups of 2^from lanes hold equal
 // values: xor 1, 2 by DPP quad permutes, then (equal groups of 4 and 8) the half
 // row and row mirrors, then shuffles.
-template <int CTRL> __device__ __forceinline__ double dpp_add(double x)
-{
-    const long long v = __builtin_bit_cast(long long, x);
-    const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xF, 0xF, false);
-    return x + __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
-}
 __device__ __forceinline__ double scf_lanes(double x, int from, int to)
 {
     if (from <= 0 && to > 0) x = dpp_add<0xB1>(x);
