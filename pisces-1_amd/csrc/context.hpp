@@ -46,6 +46,7 @@ struct pisces_ctx {
     // solver workspace (grown on demand)
     pisces::dbuf wB, wZ, wU, wZV, wR, wC, wJ, wdiag, wpart, wsmall, winfo, wX, wY;
     pisces::dbuf wB32, wZ32, wC32;
+    pisces::dbuf wgrad;  // gradient workspace
     double *hsmall = nullptr;  // pinned, kSmall doubles
     static constexpr int kSmall = 1 << 16;
 
