@@ -50,10 +50,10 @@ void pisces_ctx::hx(const void *X, void *Y, long long ld, int nvec, int precisio
     for (int a = 0; a < 3; ++a) j.ax[a] = ax[a].m;
     j.V = f64 ? dV64.p : dV32.p;
     j.X = X; j.Y = Y; j.ld = ld;
-    const HxJob *d = push_job(j);
     if (precision == PISCES_BF16X2 && (hx_variant == 3 || (hx_variant == 1 && hx_fused_enabled()))) {
         // the one-launch form: its plan (with zeroed counters) is uploaded from
         // pageable memory, which the copy has consumed when it returns
+        const HxJob *d = push_job(j);
         std::vector<int> plan(hx_fused_plan_ints(&j, 1));
         hx_fused_plan(&j, 1, plan.data());
         dplan.ensure(sizeof(int) * plan.size());
@@ -62,7 +62,10 @@ void pisces_ctx::hx(const void *X, void *Y, long long ld, int nvec, int precisio
         hx_fused_launch(&j, d, 1, plan.data(), dplan.as<int>(), maxn, stream);
         return;
     }
-    hx_launch(d, 1, n[2] * nvec, n[1] * nvec, maxn, precision, stream, hx_variant);
+    if (hx_variant == 0 && precision != PISCES_BF16X2)
+        hx_launch(push_job(j), 1, n[2] * nvec, n[1] * nvec, maxn, precision, stream, hx_variant);
+    else
+        hx_launch_one(j, precision, stream);
 }
 
 void pisces_ctx::sync() { PC_HIP(hipStreamSynchronize(stream)); }

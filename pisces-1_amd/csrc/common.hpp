@@ -109,6 +109,9 @@ struct HxJob {
 // of the matrix-core kernels, which every other value selects)
 void hx_launch(const HxJob *d_jobs, int njobs, int max_planes_x, int max_planes_z,
                int max_n, int precision, hipStream_t s, int variant = 1);
+// One job passed by value (the matrix-core kernels take it from their kernel
+// arguments: no descriptor in memory, no copy before the launch).
+void hx_launch_one(const HxJob &job, int precision, hipStream_t s);
 // Split-BF16 H*X with both passes in one launch, ordered per XCD so that
 // pass B reads X and Y from the L2 that pass A left them in.  The plan (ints,
 // hx_fused_plan_ints of them) is built on the host from the host copy of the

@@ -25,6 +25,14 @@ struct FdmTask {
 // precision: PISCES_FP64 (FP64 matrix cores) or PISCES_BF16X2 (split BF16)
 void fdm_launch(const FdmTask *d_tasks, int ntasks, int max_n, int precision, hipStream_t s);
 
+// nvec vectors of one grid, passed by value: vector v at t.src / dst / work + v
+// ngp elements.  Same kernels, no descriptors in memory.
+struct FdmOne {
+    FdmTask t;
+    long long ngp;
+};
+void fdm_launch_one(const FdmOne &one, int nvec, int precision, hipStream_t s);
+
 // The split-BF16 form with its three passes in one XCD-ordered launch (each
 // pass reads the intermediate the previous one left in the L2).  The plan
 // (fdm_fused_plan_ints ints, built on the host from the host copy of the

@@ -1,13 +1,14 @@
 // noalloc.hip -- the kinetic preconditioner without device allocation.
 //
 // pisces_kinetic_precond allocates its device buffers per call: the residual
-// and result copies, the task descriptors and the FP32 intermediate between the
+// and result copies, the task descriptors and the BF16 intermediate between the
 // three plane passes of the split-BF16 form.  Callers that cannot allocate
 // (code under stream capture, tight serving loops) pass device residuals and
-// results instead and the descriptors and intermediate live in `scratch`, a
-// fixed-size array in the library's code object.  Every GPU holds its own copy
-// of the array until the process ends; its address on each device is looked up
-// once, when the first context is created on that device.
+// results instead; the description of the vectors is a kernel argument and the
+// intermediate lives in `scratch`, a fixed-size array in the library's code
+// object.  Every GPU holds its own copy of the array until the process ends; its
+// address on each device is looked up once, when the first context is created on
+// that device.
 #include <mutex>
 
 #include "context.hpp"
@@ -27,30 +28,6 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 std::mutex g_scratch_mu;
 void *g_scratch_ptr[kMaxDevices];
-
-// One descriptor per vector: the same fields pisces_kinetic_precond fills on
-// the host, written on the device so that no host-to-device copy is needed.
-__global__ void fdm_tasks_kernel(FdmTask *tasks, int nvec, AxisMats ax0, AxisMats ax1,
-                                 AxisMats ax2, const double *r, double *t, uint16_t *work,
-                                 long long ngp, double shift, double scale, double floor)
-{
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nvec) return;
-    FdmTask f;
-    f.ax[0] = ax0;
-    f.ax[1] = ax1;
-    f.ax[2] = ax2;
-    f.src = r + ngp * v;
-    f.dst = t + ngp * v;
-    f.work = work ? work + ngp * v : nullptr;
-    f.shift = shift;
-    f.scale = scale;
-    f.floor = floor;
-    f.src32 = 0;
-    f.dst32 = 0;
-    f.absden = 0;
-    tasks[v] = f;
-}
 
 inline size_t round256(size_t b) { return (b + 255) & ~size_t(255); }
 
@@ -93,6 +70,7 @@ int pisces_kinetic_precond_noalloc(pisces_ctx *c, int nvec, const double *d_r, d
         set_last_error("pisces_kinetic_precond_noalloc: no scratch address for this context");
         return PISCES_ERR_STATE;
     }
+    // the documented limit counts a descriptor per vector
     const size_t task_bytes = round256(sizeof(FdmTask) * (size_t)nvec);
     const size_t work_bytes =
         precision == PISCES_BF16X2 ? sizeof(uint16_t) * (size_t)c->ngp * (size_t)nvec : 0;
@@ -106,13 +84,16 @@ int pisces_kinetic_precond_noalloc(pisces_ctx *c, int nvec, const double *d_r, d
     return guarded_call([&] {
         PC_HIP(hipSetDevice(c->device));
         unsigned char *base = static_cast<unsigned char *>(c->scratch);
-        FdmTask *tasks = reinterpret_cast<FdmTask *>(base);
-        uint16_t *work = work_bytes ? reinterpret_cast<uint16_t *>(base + task_bytes) : nullptr;
-        hipLaunchKernelGGL(fdm_tasks_kernel, dim3((nvec + 63) / 64), dim3(64), 0, c->stream,
-                           tasks, nvec, c->ax[0].m, c->ax[1].m, c->ax[2].m, d_r, d_t, work,
-                           c->ngp, shift, scale, floor);
-        PC_HIP(hipGetLastError());
-        fdm_launch(tasks, nvec, c->maxn, precision, c->stream);
+        FdmOne one{};
+        for (int a = 0; a < 3; ++a) one.t.ax[a] = c->ax[a].m;
+        one.t.src = d_r;
+        one.t.dst = d_t;
+        one.t.work = work_bytes ? reinterpret_cast<uint16_t *>(base + task_bytes) : nullptr;
+        one.t.shift = shift;
+        one.t.scale = scale;
+        one.t.floor = floor;
+        one.ngp = c->ngp;
+        fdm_launch_one(one, nvec, precision, c->stream);
         c->sync();
         return 0;
     });

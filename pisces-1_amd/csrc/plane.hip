@@ -397,6 +397,13 @@ __global__ void __launch_bounds__((Cfg<NT, CS>::THREADS), (CS == 1 ? 4 : 1)) hx_
     hx_bf2_plane<PASS, NT, CS>(jobs[plane_y(PASS == 1)], plane_x(PASS == 1), smem);
 }
 
+template <int PASS, int NT, int CS>
+__global__ void __launch_bounds__((Cfg<NT, CS>::THREADS), (CS == 1 ? 4 : 1)) hx_bf2_one_kernel(HxJob J)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    hx_bf2_plane<PASS, NT, CS>(J, plane_x(PASS == 1), smem);
+}
+
 // ------------------------------------------------------------------ H*X, split-BF16, one launch
 // Both passes in one launch, ordered per XCD so that pass B of a vector reads
 // the X and Y that pass A left in that XCD's L2 instead of HBM.  The vectors
@@ -624,6 +631,14 @@ __global__ void __launch_bounds__((Cfg<NT, CS>::THREADS)) fdm_bf2_kernel(const F
     fdm_bf2_plane<PASS, NT, CS, MULTI>(tasks[plane_y(PASS == 1)], plane_x(PASS == 1), gridDim.x, smem);
 }
 
+template <int PASS, int NT, int CS, bool MULTI>
+__global__ void __launch_bounds__((Cfg<NT, CS>::THREADS)) fdm_bf2_one_kernel(FdmOne one)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    fdm_bf2_plane<PASS, NT, CS, MULTI>(task_of(one, plane_y(PASS == 1), one.t.src32 ? 4 : 8, one.t.dst32 ? 4 : 8),
+                                       plane_x(PASS == 1), gridDim.x, smem);
+}
+
 // ------------------------------------------------------------------ preconditioner, one launch
 // The three passes of the split-BF16 preconditioner in one launch, ordered per
 // XCD as the one-launch H*X is: the vectors split into eight contiguous runs,
@@ -715,31 +730,47 @@ int env_or(const char *env, int def)
 }
 
 template <int NT, int CS>
-void hx_bf2_launch(const HxJob *d, int n, int pa, int pb, hipStream_t s)
+void hx_bf2_launch(const HxJob *d, const HxJob *one, int n, int pa, int pb, hipStream_t s)
 {
     static std::once_flag once;
     std::call_once(once, [] {
         allow_lds(hx_bf2_kernel<0, NT, CS>);
         allow_lds(hx_bf2_kernel<1, NT, CS>);
+        allow_lds(hx_bf2_one_kernel<0, NT, CS>);
+        allow_lds(hx_bf2_one_kernel<1, NT, CS>);
     });
     const size_t lds = bf2_lds(16 * NT);
     const dim3 blk(Cfg<NT, CS>::THREADS);
     // pass A uses only the i-major plane (first half of the layout)
+    if (one) {
+        hipLaunchKernelGGL((hx_bf2_one_kernel<0, NT, CS>), dim3(pa), blk, lds / 2, s, *one);
+        hipLaunchKernelGGL((hx_bf2_one_kernel<1, NT, CS>), dim3(pb), blk, lds, s, *one);
+        return;
+    }
     hipLaunchKernelGGL((hx_bf2_kernel<0, NT, CS>), dim3(pa, n), blk, lds / 2, s, d);
     hipLaunchKernelGGL((hx_bf2_kernel<1, NT, CS>), dim3(pb, n), blk, lds, s, d);
 }
 
 template <int NT, int CS, bool MULTI>
-void fdm_bf2_launch(const FdmTask *d, int n, int nplanes, hipStream_t s, int ppw = 1)
+void fdm_bf2_launch(const FdmTask *d, const FdmOne *one, int n, int nplanes, hipStream_t s, int ppw = 1)
 {
     static std::once_flag once;
     std::call_once(once, [] {
         allow_lds(fdm_bf2_kernel<0, NT, CS, MULTI>);
         allow_lds(fdm_bf2_kernel<1, NT, CS, MULTI>);
         allow_lds(fdm_bf2_kernel<2, NT, CS, MULTI>);
+        allow_lds(fdm_bf2_one_kernel<0, NT, CS, MULTI>);
+        allow_lds(fdm_bf2_one_kernel<1, NT, CS, MULTI>);
+        allow_lds(fdm_bf2_one_kernel<2, NT, CS, MULTI>);
     });
     const size_t lds = bf2_lds(16 * NT);
     const dim3 grid((nplanes + ppw - 1) / ppw, n), blk(Cfg<NT, CS>::THREADS);
+    if (one) {
+        hipLaunchKernelGGL((fdm_bf2_one_kernel<0, NT, CS, MULTI>), grid, blk, lds, s, *one);
+        hipLaunchKernelGGL((fdm_bf2_one_kernel<1, NT, CS, MULTI>), grid, blk, lds, s, *one);
+        hipLaunchKernelGGL((fdm_bf2_one_kernel<2, NT, CS, MULTI>), grid, blk, lds, s, *one);
+        return;
+    }
     hipLaunchKernelGGL((fdm_bf2_kernel<0, NT, CS, MULTI>), grid, blk, lds, s, d);
     hipLaunchKernelGGL((fdm_bf2_kernel<1, NT, CS, MULTI>), grid, blk, lds, s, d);
     hipLaunchKernelGGL((fdm_bf2_kernel<2, NT, CS, MULTI>), grid, blk, lds, s, d);
@@ -747,17 +778,18 @@ void fdm_bf2_launch(const FdmTask *d, int n, int nplanes, hipStream_t s, int ppw
 
 }  // namespace
 
-void hx_mfma_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_planes_b, int max_n,
-                    int precision, hipStream_t s)
+namespace {
+void hx_dispatch(const HxJob *d_jobs, const HxJob *one, int njobs, int max_planes_a, int max_planes_b,
+                 int max_n, int precision, hipStream_t s)
 {
     if (njobs <= 0) return;
     PC_REQUIRE(max_n > 0 && max_n <= 128, PISCES_ERR_UNSUPPORTED, "grid dimension above 128");
     if (precision != PISCES_BF16X2) {
-        hx_f_launch(d_jobs, njobs, max_planes_a, max_planes_b, max_n, precision, s);
+        hx_f_launch(d_jobs, one, njobs, max_planes_a, max_planes_b, max_n, precision, s);
         return;
     }
     const int np = axis_pad(max_n);
-    if (np <= 32) hx_bf2_launch<2, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+    if (np <= 32) hx_bf2_launch<2, 2>(d_jobs, one, njobs, max_planes_a, max_planes_b, s);
     else if (np <= 64) {
         // Few planes: eight waves each, for the latency of a plane; more than
         // about 1.5 a CU: four waves and fewer registers, so that four planes
@@ -765,13 +797,25 @@ void hx_mfma_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_pl
         // 4 vectors 14.4 / 15.2, 8 20.8 / 20.1, 32 49.9 / 47.8, 128 161 / 147;
         // at 48^3 128 vectors 102 / 75.
         if ((long long)njobs * max_planes_a < 384)
-            hx_bf2_launch<4, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+            hx_bf2_launch<4, 2>(d_jobs, one, njobs, max_planes_a, max_planes_b, s);
         else
-            hx_bf2_launch<4, 1>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+            hx_bf2_launch<4, 1>(d_jobs, one, njobs, max_planes_a, max_planes_b, s);
     }
-    else if (np <= 96) hx_bf2_launch<6, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
-    else hx_bf2_launch<8, 2>(d_jobs, njobs, max_planes_a, max_planes_b, s);
+    else if (np <= 96) hx_bf2_launch<6, 2>(d_jobs, one, njobs, max_planes_a, max_planes_b, s);
+    else hx_bf2_launch<8, 2>(d_jobs, one, njobs, max_planes_a, max_planes_b, s);
     PC_HIP(hipGetLastError());
+}
+}  // namespace
+
+void hx_mfma_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_planes_b, int max_n,
+                    int precision, hipStream_t s)
+{
+    hx_dispatch(d_jobs, nullptr, njobs, max_planes_a, max_planes_b, max_n, precision, s);
+}
+
+void hx_launch_one(const HxJob &J, int precision, hipStream_t s)
+{
+    hx_dispatch(nullptr, &J, 1, J.nz * J.nvec, J.ny * J.nvec, std::max(J.nx, std::max(J.ny, J.nz)), precision, s);
 }
 
 int hx_fused_plan_ints(const HxJob *h_jobs, int njobs)
@@ -995,18 +1039,20 @@ bool fdm_fused_enabled()
     return on;
 }
 
-void fdm_launch(const FdmTask *d_tasks, int ntasks, int max_n, int precision, hipStream_t s)
+namespace {
+void fdm_dispatch(const FdmTask *d_tasks, const FdmOne *one, int ntasks, int max_n, int precision,
+                  hipStream_t s)
 {
     if (ntasks <= 0) return;
     PC_REQUIRE(max_n > 0 && max_n <= 128, PISCES_ERR_UNSUPPORTED, "grid dimension above 128");
     if (precision == PISCES_FP64) {
-        fdm_f64_launch(d_tasks, ntasks, max_n, s);
+        fdm_f64_launch(d_tasks, one, ntasks, max_n, s);
         return;
     }
     const int np = axis_pad(max_n);
     // planes per pass: the largest of ny (pass 1) and nz (passes 0, 2) <= max_n
     if (np <= 32) {
-        fdm_bf2_launch<2, 2, false>(d_tasks, ntasks, max_n, s);
+        fdm_bf2_launch<2, 2, false>(d_tasks, one, ntasks, max_n, s);
     } else if (np <= 64) {
         // Planes per workgroup by the number of planes: a plane's three matrix
         // fragments are as many bytes from the L2 as six planes, so workgroups
@@ -1018,12 +1064,24 @@ void fdm_launch(const FdmTask *d_tasks, int ntasks, int max_n, int precision, hi
         const long long planes = (long long)ntasks * max_n;
         static const int ppw_env = env_or("PISCES_PPW_FDM", 0);
         const int ppw = ppw_env ? ppw_env : planes < 600 ? 1 : planes < 1800 ? 2 : planes < 4096 ? 4 : 8;
-        if (ppw == 1) fdm_bf2_launch<4, 2, false>(d_tasks, ntasks, max_n, s);
-        else fdm_bf2_launch<4, 2, true>(d_tasks, ntasks, max_n, s, ppw);
+        if (ppw == 1) fdm_bf2_launch<4, 2, false>(d_tasks, one, ntasks, max_n, s);
+        else fdm_bf2_launch<4, 2, true>(d_tasks, one, ntasks, max_n, s, ppw);
     }
-    else if (np <= 96) fdm_bf2_launch<6, 2, false>(d_tasks, ntasks, max_n, s);
-    else fdm_bf2_launch<8, 2, false>(d_tasks, ntasks, max_n, s);
+    else if (np <= 96) fdm_bf2_launch<6, 2, false>(d_tasks, one, ntasks, max_n, s);
+    else fdm_bf2_launch<8, 2, false>(d_tasks, one, ntasks, max_n, s);
     PC_HIP(hipGetLastError());
+}
+}  // namespace
+
+void fdm_launch(const FdmTask *d_tasks, int ntasks, int max_n, int precision, hipStream_t s)
+{
+    fdm_dispatch(d_tasks, nullptr, ntasks, max_n, precision, s);
+}
+
+void fdm_launch_one(const FdmOne &one, int nvec, int precision, hipStream_t s)
+{
+    const AxisMats *ax = one.t.ax;
+    fdm_dispatch(nullptr, &one, nvec, std::max(ax[0].n, std::max(ax[1].n, ax[2].n)), precision, s);
 }
 
 }  // namespace pisces

@@ -11,9 +11,10 @@ namespace pisces {
 
 // FP64 and FP32 forms (plane_f.hip).  max_planes_a, _b: the largest number of
 // planes of a job in pass A and B; max_n: the largest axis of any job or task.
-void hx_f_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_planes_b, int max_n,
+// `one`, where not null, replaces the d_jobs / d_tasks in memory.
+void hx_f_launch(const HxJob *d_jobs, const HxJob *one, int njobs, int max_planes_a, int max_planes_b, int max_n,
                  int precision, hipStream_t s);
-void fdm_f64_launch(const FdmTask *d_tasks, int ntasks, int max_n, hipStream_t s);
+void fdm_f64_launch(const FdmTask *d_tasks, const FdmOne *one, int ntasks, int max_n, hipStream_t s);
 
 namespace {
 
@@ -84,6 +85,17 @@ __device__ __forceinline__ bool geo_of(int kind, int nx, int ny, int nz, int nve
 // previous pass left last in the L2 and the memory-side cache.
 __device__ __forceinline__ int plane_x(bool rev) { return rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x; }
 __device__ __forceinline__ int plane_y(bool rev) { return rev ? gridDim.y - 1 - blockIdx.y : blockIdx.y; }
+
+// task of vector blockIdx.y (reversed as plane_y) of a grid passed by value;
+// elements of es_src, es_dst bytes
+__device__ __forceinline__ FdmTask task_of(const FdmOne &one, int v, int es_src, int es_dst)
+{
+    FdmTask t = one.t;
+    t.src = static_cast<const char *>(t.src) + one.ngp * v * es_src;
+    t.dst = static_cast<char *>(t.dst) + one.ngp * v * es_dst;
+    t.work += one.ngp * v;
+    return t;
+}
 
 // Raises a kernel's dynamic LDS limit to `bytes` (the 160 KB of a CU less the
 // kernel's static LDS); a failure is reported, not left behind as the thread's

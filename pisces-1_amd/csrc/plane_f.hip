@@ -268,6 +268,124 @@ __global__ void __launch_bounds__((Cfg<T, NT>::THREADS)) hx_f_kernel(const HxJob
     hx_plane<T, PASS, NT>(jobs[plane_y(PASS == 1)], plane_x(PASS == 1), smem);
 }
 
+template <typename T, int PASS, int NT>
+__global__ void __launch_bounds__((Cfg<T, NT>::THREADS)) hx_f_one_kernel(HxJob J)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    hx_plane<T, PASS, NT>(J, plane_x(PASS == 1), smem);
+}
+
+// ------------------------------------------------------------------ H*X, small grids
+// Both passes in one launch for grids of at most 32 points per axis: a workgroup
+// owns one 16 x 16 tile of the (i,j) plane at k, contracts the plane along j and
+// i on the matrix cores as above, and adds the z sum of its points on the VALU,
+//   Y(i,j,k) += sum_k' Tz[k][k'] X(i,j,k'),
+// reading the other planes' tiles straight from the caches (a vector is at most
+// 256 KB).  There is no intermediate Y and no second launch.  The four waves split
+// k' and the two contractions; their sums meet in LDS in a fixed order.
+constexpr int kSmallN = 32, kSmallThreads = 256;
+
+template <typename T>
+__global__ void __launch_bounds__(kSmallThreads) hx_small_kernel(HxJob J, int nti, int ntiles)
+{
+    typedef typename Acc<T>::type acc_t;
+    constexpr int PITCH = kSmallN + (sizeof(T) == 8 ? 2 : 4), KZ = kSmallN / 4;
+    __shared__ T P[kSmallN * PITCH], Ml[kSmallN * PITCH];
+    __shared__ T red[3][4][64];  // wave - 1, element, lane
+    const int pv = blockIdx.x / ntiles, tile = blockIdx.x - pv * ntiles;
+    const int v = pv / J.nz, k = pv - v * J.nz;
+    const int lane = threadIdx.x & 63, zq = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+    const int r0 = 16 * (tile / nti), i = 16 * (tile % nti) + l16;
+    const int nx = J.nx, ny = J.ny, nz = J.nz;
+    const unsigned plane = (unsigned)nx * ny;
+    const gptr<const T> X = glb(static_cast<const T *>(J.X)) + J.ld * v;
+    const gptr<const T> xp = X + (size_t)k * plane;
+    // the lane's four points of the tile
+    unsigned off[4];
+    bool ok[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int c = r0 + Acc<T>::row(lq, r);
+        ok[r] = c < ny && i < nx;
+        off[r] = ok[r] ? (unsigned)(c * nx + i) : 0u;
+    }
+    // the plane and Tx on their way to LDS, this wave's planes k', V, Ty
+    T ps[4], ms[4], xz[KZ][4], tz[KZ], xk[4], vk[4], af[8];
+    const int pi = threadIdx.x & 31, pc = threadIdx.x >> 5;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int c = pc + 8 * u;
+        const bool in = pi < nx && c < ny;
+        ps[u] = at<T>(xp, in ? (unsigned)(c * nx + pi) : 0u);
+        ps[u] = in ? ps[u] : T(0);
+        ms[u] = glb(tmat<T>(J.ax[0]))[c * kSmallN + pi];
+    }
+    const gptr<const T> Tz = glb(tmat<T>(J.ax[2])) + k * kSmallN;
+    const int zs = (nz + 3) / 4, k0 = zs * zq;
+#pragma unroll
+    for (int u = 0; u < KZ; ++u) {
+        const bool on = u < zs && k0 + u < nz;
+        tz[u] = T(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xz[u][r] = T(0);
+        if (on) {
+            tz[u] = Tz[k0 + u];
+            const gptr<const T> xq = X + (size_t)(k0 + u) * plane;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) xz[u][r] = at<T>(xq, off[r]);
+        }
+    }
+    if (zq == 0) {
+        const gptr<const T> V = glb(static_cast<const T *>(J.V)) + (size_t)k * plane;
+        const gptr<const T> Ty = glb(tmat<T>(J.ax[1]));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            xk[r] = at<T>(xp, off[r]);
+            vk[r] = at<T>(V, off[r]);
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) af[s] = Ty[(4 * s + lq) * kSmallN + r0 + l16];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        P[(pc + 8 * u) * PITCH + pi] = ps[u];
+        Ml[(pc + 8 * u) * PITCH + pi] = ms[u];
+    }
+    __syncthreads();
+    acc_t acc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = zq == 0 && ok[r] ? vk[r] * xk[r] : T(0);
+    const int sy = (ny + 3) / 4, sx = (nx + 3) / 4;  // k-steps that hold points
+    if (zq == 0) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (s < sy) acc = mma(af[s], P[(4 * s + lq) * PITCH + i], acc);
+    } else if (zq == 1) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (s < sx) acc = mma(P[(r0 + l16) * PITCH + 4 * s + lq], Ml[(4 * s + lq) * PITCH + i], acc);
+    }
+    T z[4] = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int u = 0; u < KZ; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[r] += tz[u] * xz[u][r];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) z[r] += acc[r];
+    if (zq > 0)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[zq - 1][r][lane] = z[r];
+    __syncthreads();
+    if (zq > 0) return;
+    const gptr<T> y = glb(static_cast<T *>(J.Y)) + (J.ld * v + (long long)k * plane);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const T s = z[r] + ((red[0][r][lane] + red[1][r][lane]) + red[2][r][lane]);
+        if (ok[r]) y[off[r]] = s;
+    }
+}
+
 // ------------------------------------------------------------------ preconditioner
 // Passes as in plane.hip; passes 1 and 2 work in place in dst, where every
 // plane is read (into LDS) and written by its one workgroup only.
@@ -360,32 +478,56 @@ __global__ void __launch_bounds__((Cfg<double, NT>::THREADS)) fdm_f64_kernel(con
     fdm_plane<PASS, NT>(tasks[plane_y(PASS == 1)], plane_x(PASS == 1), smem);
 }
 
+template <int PASS, int NT>
+__global__ void __launch_bounds__((Cfg<double, NT>::THREADS)) fdm_f64_one_kernel(FdmOne one)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    fdm_plane<PASS, NT>(task_of(one, plane_y(PASS == 1), 8, 8), plane_x(PASS == 1), smem);
+}
+
 // ------------------------------------------------------------------ launches
 template <typename T, int NT>
-void hx_nt_launch(const HxJob *d, int n, int pa, int pb, hipStream_t s)
+void hx_nt_launch(const HxJob *d, const HxJob *one, int n, int pa, int pb, hipStream_t s)
 {
     typedef Cfg<T, NT> C;
     static std::once_flag once;
     std::call_once(once, [] {
         allow_lds(hx_f_kernel<T, 0, NT>);
         allow_lds(hx_f_kernel<T, 1, NT>);
+        allow_lds(hx_f_one_kernel<T, 0, NT>);
+        allow_lds(hx_f_one_kernel<T, 1, NT>);
     });
     const size_t la = C::plane_bytes, lb = C::BIG ? la : 2 * la;
+    if (one) {
+        hipLaunchKernelGGL((hx_f_one_kernel<T, 0, NT>), dim3(pa), dim3(C::THREADS), la, s, *one);
+        hipLaunchKernelGGL((hx_f_one_kernel<T, 1, NT>), dim3(pb), dim3(C::THREADS), lb, s, *one);
+        return;
+    }
     hipLaunchKernelGGL((hx_f_kernel<T, 0, NT>), dim3(pa, n), dim3(C::THREADS), la, s, d);
     hipLaunchKernelGGL((hx_f_kernel<T, 1, NT>), dim3(pb, n), dim3(C::THREADS), lb, s, d);
 }
 
+// Most tiles (workgroups) for which the one-launch form is taken: beyond about
+// four a CU its repeated reads of the vector cost more than the second launch.
+// us, one launch / two: 12^3 x 1 3.5 / 6.5 (FP64), 32^3 x 1 4.1 / 7.7, x 4 5.6 / 8.0,
+// x 8 (1024 tiles) 8.6 / 8.5, x 16 14.0 / 10.8; FP32 32^3 x 1 3.6 / 6.7, x 8 5.7 / 7.1,
+// x 16 9.7 / 8.1.
+constexpr int kSmallTiles = 1000;
+
 template <typename T>
-void hx_t_launch(const HxJob *d, int n, int pa, int pb, int np, hipStream_t s)
+void hx_t_launch(const HxJob *d, const HxJob *one, int n, int pa, int pb, int np, hipStream_t s)
 {
-    if (np <= 32) hx_nt_launch<T, 2>(d, n, pa, pb, s);
-    else if (np <= 64) hx_nt_launch<T, 4>(d, n, pa, pb, s);
-    else if (np <= 96) hx_nt_launch<T, 6>(d, n, pa, pb, s);
-    else hx_nt_launch<T, 8>(d, n, pa, pb, s);
+    const int nti = one ? (one->nx + 15) / 16 : 0, ntiles = one ? nti * ((one->ny + 15) / 16) : 0;
+    if (one && np <= 32 && (long long)pa * ntiles <= kSmallTiles)
+        hipLaunchKernelGGL((hx_small_kernel<T>), dim3(pa * ntiles), dim3(kSmallThreads), 0, s, *one, nti, ntiles);
+    else if (np <= 32) hx_nt_launch<T, 2>(d, one, n, pa, pb, s);
+    else if (np <= 64) hx_nt_launch<T, 4>(d, one, n, pa, pb, s);
+    else if (np <= 96) hx_nt_launch<T, 6>(d, one, n, pa, pb, s);
+    else hx_nt_launch<T, 8>(d, one, n, pa, pb, s);
 }
 
 template <int NT>
-void fdm_nt_launch(const FdmTask *d, int n, int planes, hipStream_t s)
+void fdm_nt_launch(const FdmTask *d, const FdmOne *one, int n, int planes, hipStream_t s)
 {
     typedef Cfg<double, NT> C;
     static std::once_flag once;
@@ -393,9 +535,18 @@ void fdm_nt_launch(const FdmTask *d, int n, int planes, hipStream_t s)
         allow_lds(fdm_f64_kernel<0, NT>);
         allow_lds(fdm_f64_kernel<1, NT>);
         allow_lds(fdm_f64_kernel<2, NT>);
+        allow_lds(fdm_f64_one_kernel<0, NT>);
+        allow_lds(fdm_f64_one_kernel<1, NT>);
+        allow_lds(fdm_f64_one_kernel<2, NT>);
     });
     const size_t l1 = C::plane_bytes, l2 = C::BIG ? l1 : 2 * l1;
     const dim3 grid(planes, n), blk(C::THREADS);
+    if (one) {
+        hipLaunchKernelGGL((fdm_f64_one_kernel<0, NT>), grid, blk, l2, s, *one);
+        hipLaunchKernelGGL((fdm_f64_one_kernel<1, NT>), grid, blk, l1, s, *one);
+        hipLaunchKernelGGL((fdm_f64_one_kernel<2, NT>), grid, blk, l2, s, *one);
+        return;
+    }
     hipLaunchKernelGGL((fdm_f64_kernel<0, NT>), grid, blk, l2, s, d);
     hipLaunchKernelGGL((fdm_f64_kernel<1, NT>), grid, blk, l1, s, d);
     hipLaunchKernelGGL((fdm_f64_kernel<2, NT>), grid, blk, l2, s, d);
@@ -403,23 +554,23 @@ void fdm_nt_launch(const FdmTask *d, int n, int planes, hipStream_t s)
 
 }  // namespace
 
-void hx_f_launch(const HxJob *d_jobs, int njobs, int max_planes_a, int max_planes_b, int max_n,
+void hx_f_launch(const HxJob *d_jobs, const HxJob *one, int njobs, int max_planes_a, int max_planes_b, int max_n,
                  int precision, hipStream_t s)
 {
     const int np = axis_pad(max_n);
-    if (precision == PISCES_FP32) hx_t_launch<float>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
-    else hx_t_launch<double>(d_jobs, njobs, max_planes_a, max_planes_b, np, s);
+    if (precision == PISCES_FP32) hx_t_launch<float>(d_jobs, one, njobs, max_planes_a, max_planes_b, np, s);
+    else hx_t_launch<double>(d_jobs, one, njobs, max_planes_a, max_planes_b, np, s);
     PC_HIP(hipGetLastError());
 }
 
-void fdm_f64_launch(const FdmTask *d_tasks, int ntasks, int max_n, hipStream_t s)
+void fdm_f64_launch(const FdmTask *d_tasks, const FdmOne *one, int ntasks, int max_n, hipStream_t s)
 {
     const int np = axis_pad(max_n);
     // planes per pass: the largest of ny (pass 1) and nz (passes 0, 2) <= max_n
-    if (np <= 32) fdm_nt_launch<2>(d_tasks, ntasks, max_n, s);
-    else if (np <= 64) fdm_nt_launch<4>(d_tasks, ntasks, max_n, s);
-    else if (np <= 96) fdm_nt_launch<6>(d_tasks, ntasks, max_n, s);
-    else fdm_nt_launch<8>(d_tasks, ntasks, max_n, s);
+    if (np <= 32) fdm_nt_launch<2>(d_tasks, one, ntasks, max_n, s);
+    else if (np <= 64) fdm_nt_launch<4>(d_tasks, one, ntasks, max_n, s);
+    else if (np <= 96) fdm_nt_launch<6>(d_tasks, one, ntasks, max_n, s);
+    else fdm_nt_launch<8>(d_tasks, one, ntasks, max_n, s);
     PC_HIP(hipGetLastError());
 }
 

@@ -1,17 +1,19 @@
 """FP64 and FP32 plane kernels (H*X, preconditioner) at the edges of their tile
 forms: axes one below, at and one above multiples of 16 and 32, every tile
-form (32, 64, 96, 128 points), planes whose two axes take different paddings."""
+form (32, 64, 96, 128 points), planes whose two axes take different paddings,
+and, up to 32 points, both sides of the line between one launch and two (1000
+tiles: 8 vectors of 32^3 are beyond it)."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(2, 3, 2), (15, 17, 16), (33, 31, 32), (47, 49, 64), (65, 9, 48), (80, 81, 3),
+SHAPES = [(2, 3, 2), (15, 17, 16), (32, 32, 32), (5, 32, 31), (16, 2, 29), (33, 31, 32), (47, 49, 64), (65, 9, 48), (80, 81, 3),
           (96, 33, 97), (97, 16, 5), (128, 4, 113)]
 
 
 @pytest.mark.parametrize("n", SHAPES)
-@pytest.mark.parametrize("nvec", [1, 3])
+@pytest.mark.parametrize("nvec", [1, 3, 8])
 def test_apply_h_tile_edges(pisces, oracle_mod, n, nvec):
     print("hx edges", n, nvec, flush=True)
     L = tuple(0.6 * (v + 1) for v in n)
