@@ -322,7 +322,8 @@ int pisces_piab(pisces_ctx *ctx, double *wf);
 
 typedef struct {
     int nconv;        /* converged roots                                      */
-    int n_matvec;     /* H*x products (vectors) in the final precision         */
+    int n_matvec;     /* H*x products (vectors) in the final precision that
+                         entered the solve (one root: one more is queued)   */
     int n_matvec_lo;  /* H*x products in the low precision (mixed forms)       */
     int n_iter;       /* Davidson iterations (subspace expansions)             */
     int n_macro;      /* macro iterations (restarts + 1)                      */

@@ -45,6 +45,27 @@ void jd_finish(double *C, const double *J, long long ldc, long long N, int k,
 void cholinv(const double *d_G, int k, double *d_W, int *d_info, double rel_tol, hipStream_t s);
 void diag_h(const double *V, const double *Tx, const double *Ty, const double *Tz, int nx,
             int ny, int nz, double *D, hipStream_t s);
+// One-root Davidson iteration (one_root.hip): B, Z hold m <= 63 columns (ld N);
+// the dot products of each kernel go to a buffer of one_part_doubles(N).
+constexpr int kOneLd = 66;
+int one_rows(long long N);
+inline size_t one_part_doubles(long long N) { return (size_t)(one_rows(N) + 1) * kOneLd; }
+// C = (Z y - theta B y) / (theta - D); dots: B^T C (m), ||Z y - theta B y||^2,
+// ||B y||^2.  U = B y and ZV = Z y are stored where U is given.  y: host.
+void one_ritz(const double *B, const double *Z, const double *D, long long N, int m, const double *y,
+              double theta, double *C, double *U, double *ZV, double *part, hipStream_t s);
+// b = C made orthogonal to B (two Gram-Schmidt passes, the first from part_h's
+// B^T C) and normalised, or 0; C is overwritten
+void one_orth(const double *B, long long N, int m, double *C, double *b, double *part_h, double *part_n,
+              hipStream_t s);
+// dots: A^T x (m <= 64 columns) and ||x||^2
+void one_dots(const double *A, long long N, int m, const double *x, double *part, hipStream_t s);
+// out[0 .. n2): sums j0 .. of part2, then n sums from i0 on of part (out: host memory)
+void one_finish(const double *part, long long N, int i0, int n, const double *part2, int j0, int n2,
+                double *out, hipStream_t s);
+// xo = f x, yo = g y
+void one_scale(const double *x, double f, double *xo, const double *y, double g, double *yo, long long N,
+               hipStream_t s);
 void to_f32(const double *x, float *y, long long n, hipStream_t s);
 void to_f64(const float *x, double *y, long long n, hipStream_t s);
 // x[i] = uniform in [-1, 1) from a counter-based hash of (seed, i)
@@ -59,5 +80,7 @@ void stream_probe(const void *src, long long bytes, bool nontemporal, unsigned *
 // cyclic Jacobi, ascending eigenvalues; reads the upper triangle of A
 // (column-major, lda).  Replaces LAPACK dsyev at src/Davidson.cpp:224.
 void syev_host(int n, const double *A, int lda, double *W, double *V, int ldv);
+// The lowest eigenpair only: Householder tridiagonalisation and implicit QL.
+void lowest_eigenpair(int n, const double *A, int lda, double &w, double *v);
 
 }  // namespace pisces

