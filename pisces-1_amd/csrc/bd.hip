@@ -258,7 +258,7 @@ __device__ __forceinline__ double wave_reduce_scatter64(double (&v)[64])
 }
 
 __global__ void __launch_bounds__(kT) gram_valu_kernel(const GramTask *__restrict__ tasks,
-                                                       double *__restrict__ partial, int rows)
+                                                       double *__restrict__ partial)
 {
     const GramTask t = tasks[blockIdx.y];
     if (t.kind != 0) return;
@@ -269,8 +269,8 @@ __global__ void __launch_bounds__(kT) gram_valu_kernel(const GramTask *__restric
     const int nta = (t.ma + kGTile - 1) / kGTile;
     const int a0 = (tile % nta) * kGTile, b0 = (tile / nta) * kGTile;
     const int na = min(kGTile, t.ma - a0), nb = min(kGTile, t.mb - b0);
-    const long long r0 = (long long)chunk * rows;
-    const long long r1 = min(r0 + rows, t.N);
+    const long long r0 = (long long)chunk * t.rows;
+    const long long r1 = min(r0 + t.rows, t.N);
     double acc[kGTile * kGTile];
 #pragma unroll
     for (int i = 0; i < kGTile * kGTile; ++i) acc[i] = 0.0;
@@ -304,13 +304,13 @@ __global__ void __launch_bounds__(kT) gram_valu_kernel(const GramTask *__restric
 
 template <int LONG>
 __global__ void __launch_bounds__(kT) gram_kernel(const GramTask *__restrict__ tasks,
-                                                  double *__restrict__ partial, int rows)
+                                                  double *__restrict__ partial)
 {
     const GramTask &t = tasks[blockIdx.y];
     if (t.kind != 0 || (int)blockIdx.x >= t.nch) return;
     if (t.skip && *cst(t.skip)) return;
-    const long long r_beg = (long long)blockIdx.x * rows;
-    const long long r_end = min(r_beg + rows, t.N);
+    const long long r_beg = (long long)blockIdx.x * t.rows;
+    const long long r_end = min(r_beg + t.rows, t.N);
     // 16-byte loads need every column start aligned: uniform per task
     const int ea = t.a32 ? 4 : 8, eb = t.b32 ? 4 : 8;
     const bool vec = ((reinterpret_cast<uintptr_t>(t.A) | reinterpret_cast<uintptr_t>(t.B)) & 15) == 0 &&
@@ -447,8 +447,8 @@ __global__ void __launch_bounds__(kT) gram_narrow_kernel(const GramTask *__restr
     const int tile = blockIdx.x / t.nch, chunk = blockIdx.x - tile * t.nch;
     const int a0 = tile * kGNarrowA;
     const int na = min(kGNarrowA, t.ma - a0), nb = t.mb;
-    const long long r0 = (long long)chunk * kGRowsNarrow;
-    const long long r1 = min(r0 + kGRowsNarrow, t.N);
+    const long long r0 = (long long)chunk * t.rows;
+    const long long r1 = min(r0 + t.rows, t.N);
     double acc[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) acc[i] = 0.0;
@@ -528,19 +528,20 @@ __device__ __forceinline__ double group_sum(const double *__restrict__ p, int n,
     return v;
 }
 
-// Gram entries: kGramRedLanes lanes per entry, kT / kGramRedLanes entries per
-// workgroup; the entry's chunk partials are summed as above
-constexpr int kGramRedLanes = 8;
+// Gram entries: L lanes per entry, kT / L entries per workgroup; the entry's
+// chunk partials are summed as above.  8 lanes hold 64 chunks in one run of
+// loads; with more chunks a whole wave takes the entry.
+template <int L>
 __global__ void __launch_bounds__(kT) gram_reduce_kernel(const GramTask *__restrict__ tasks,
                                                          const double *__restrict__ partial)
 {
     const GramTask t = tasks[blockIdx.y];
     if (t.skip && *cst(t.skip)) return;
-    const int o = blockIdx.x * (kT / kGramRedLanes) + threadIdx.x / kGramRedLanes;
-    const int j = threadIdx.x & (kGramRedLanes - 1);
+    const int o = blockIdx.x * (kT / L) + threadIdx.x / L;
+    const int j = threadIdx.x & (L - 1);
     // whole lane groups leave together, so the group's shuffles see only live lanes
     if (o >= t.ma * t.mb) return;
-    const double s = group_sum<kGramRedLanes>(partial + t.part_off + (long long)o * t.nch, t.nch, j);
+    const double s = group_sum<L>(partial + t.part_off + (long long)o * t.nch, t.nch, j);
     if (j == 0) t.out[(o % t.ma) + (long long)t.out_ld * (o / t.ma)] = s;
 }
 
@@ -1049,9 +1050,93 @@ __global__ void __launch_bounds__(kT) ritz_reduce_kernel(const RitzTask *__restr
 }
 
 // ------------------------------------------------------------------ orthogonalisation factor
-// One 64-lane workgroup per task: S = G - h^T h (h may be absent), Cholesky
-// with dropping, W = L^{-T}, F = -h W.  Shared by the Cholesky-QR factor.
-__device__ void orth_factor(const double *__restrict__ hg, int hld, const double *__restrict__ Gin,
+// The small factor kernels: one workgroup of kOT lanes per task, a chain of a
+// few small products and one or two Cholesky factorisations, each step waiting
+// on the one before.  What bounds them is that chain's latency (LDS and global
+// loads, barriers), so the products are spread over four waves, the partial
+// sums are loaded in groups of eight, and a factorisation runs on one wave
+// without a barrier.  (H2O)24 64^3, one wave per task against four: FP64 block
+// of 8, 32.6 -> 12.8 us; both rounds of a block of 4 (orth2), 40.8 -> 25.4 us.
+constexpr int kOT = 256;
+
+// [V | T]^T T (ma x nt) from its chunk partials (fixed order per entry), handed
+// to put(a, c, sum)
+template <typename F>
+__device__ __forceinline__ void part_sums(const double *part, long long part_off, int nch, int ma, int nt, F put)
+{
+    const int j = threadIdx.x & 7;
+    // whole groups of eight lanes share an entry, so their shuffles are complete
+    for (int idx = threadIdx.x >> 3; idx < ma * nt; idx += kOT / 8) {
+        const double sum = group_sum<8>(part + part_off + (long long)idx * nch, nch, j);
+        if (j == 0) put(idx % ma, idx / ma, sum);
+    }
+}
+
+// Cholesky with dropping of the nt x nt matrix A (LDS, ld kBdMaxK, lower
+// triangle read), then W = L^{-T} (upper triangular, zero columns for dropped
+// ones).  Column j is kept if kin[j] (null: all) and its pivot exceeds
+// tol * dref[j * dstep].  Called by all threads; wave 0 does the work with row
+// i of A and L, then column i of W, in the registers of lane i, and leaves W
+// and keep in LDS after a barrier.
+__device__ __forceinline__ void chol_winv(const double *A, const double *dref, int dstep, int nt,
+                                          const int *kin, double tol, double *W, int *keep)
+{
+    constexpr int K = kBdMaxK;
+    if (threadIdx.x < 64) {
+        const int l = threadIdx.x;
+        const bool in = l < nt;
+        double a[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) a[j] = (in && j <= l && j < nt) ? A[l + K * j] : 0.0;
+        const double dr = in ? dref[l * dstep] : 0.0;
+        const int ki = (in && kin) ? kin[l] : 1;
+        unsigned kept = 0;
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            if (j >= nt) break;
+            const double d = lane_value(a[j], j);
+            const bool kj = __builtin_amdgcn_readlane(ki, j) && d > tol * lane_value(dr, j) && d > 0.0;
+            if (!kj) {
+                a[j] = 0.0;  // column j of L
+                continue;
+            }
+            kept |= 1u << j;
+            const double ljj = sqrt(d);
+            a[j] = l == j ? ljj : (l > j ? a[j] / ljj : 0.0);
+#pragma unroll
+            for (int c = j + 1; c < K; ++c) {
+                if (c >= nt) break;
+                const double v = a[j] * lane_value(a[j], c);
+                if (l >= c) a[c] -= v;
+            }
+        }
+        const bool kl = (kept >> (l & 31)) & 1u;
+        double w[K];
+#pragma unroll
+        for (int i = K - 1; i >= 0; --i) {
+            w[i] = 0.0;
+            if (i >= nt || !((kept >> i) & 1u)) continue;
+            double v = (i == l) ? 1.0 : 0.0;
+#pragma unroll
+            for (int p = i + 1; p < K; ++p) {
+                if (p >= nt) break;
+                v -= lane_value(a[i], p) * w[p];
+            }
+            w[i] = kl ? v / lane_value(a[i], i) : 0.0;
+        }
+        if (in) {
+#pragma unroll
+            for (int i = 0; i < K; ++i)
+                if (i < nt) W[i + K * l] = w[i];
+            keep[l] = kl ? 1 : 0;
+        }
+    }
+    __syncthreads();
+}
+
+// S = G - h^T h (h may be absent), Cholesky with dropping, W = L^{-T},
+// F = -h W.  Shared by the Cholesky-QR factor.
+__device__ __forceinline__ void orth_factor(const double *__restrict__ hg, int hld, const double *__restrict__ Gin,
                             int gld, int m, int nt, double *__restrict__ Wo,
                             double *__restrict__ Fo, const int *kin, int *kout, int *kcopy,
                             double tol, int *skip = nullptr, double skip_tol = 0.0,
@@ -1059,85 +1144,42 @@ __device__ void orth_factor(const double *__restrict__ hg, int hld, const double
 {
     constexpr int K = kBdMaxK;
     __shared__ double h[kBdMaxM * kBdMaxK];
-    __shared__ double S[K * K], L[K * K], W[K * K], Gs[K * K];
+    __shared__ double S[K * K], W[K * K], Gs[K * K];
     __shared__ int keep[K];
+    __shared__ double s_dev[kOT / 64];
     const int tid = threadIdx.x;
     if (part) {
-        // [V | T]^T T from its chunk partials (fixed order per entry)
-        const int ma = m + nt;
-        for (int idx = tid; idx < ma * nt; idx += 64) {
-            const int a = idx % ma, c = idx / ma;
-            const double *p = part + part_off + (long long)(a + ma * c) * nch;
-            double sum = 0.0;
-            for (int q = 0; q < nch; ++q) sum += p[q];
+        part_sums(part, part_off, nch, m + nt, nt, [&](int a, int c, double sum) {
             if (a < m) h[a + m * c] = sum;
             else Gs[(a - m) + K * c] = sum;
-        }
+        });
     } else {
-        for (int idx = tid; idx < m * nt; idx += 64) {
+        for (int idx = tid; idx < m * nt; idx += kOT) {
             const int a = idx % m, c = idx / m;
             h[idx] = hg[a + (long long)hld * c];
         }
-        for (int idx = tid; idx < nt * nt; idx += 64) {
+        for (int idx = tid; idx < nt * nt; idx += kOT) {
             const int i = idx % nt, j = idx / nt;
             Gs[i + K * j] = Gin[i + (long long)gld * j];
         }
     }
     __syncthreads();
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, j = idx / nt;
         double v = Gs[i + K * j];
         for (int a = 0; a < m; ++a) v -= h[a + m * i] * h[a + m * j];
         S[i + K * j] = v;
-        L[i + K * j] = 0.0;
     }
     __syncthreads();
-    for (int j = 0; j < nt; ++j) {
-        if (tid == 0) {
-            const double d = S[j + K * j];
-            const int ki = kin ? kin[j] : 1;
-            const int kj = (ki && d > tol * Gs[j + K * j] && d > 0.0) ? 1 : 0;
-            keep[j] = kj;
-            L[j + K * j] = kj ? sqrt(d) : 0.0;
-        }
-        __syncthreads();
-        if (keep[j]) {
-            const double ljj = L[j + K * j];
-            for (int i = j + 1 + tid; i < nt; i += 64) L[i + K * j] = S[i + K * j] / ljj;
-            __syncthreads();
-            // trailing update of the lower triangle
-            for (int idx = tid; idx < nt * nt; idx += 64) {
-                const int i = idx % nt, l = idx / nt;
-                if (l > j && i >= l) S[i + K * l] -= L[i + K * j] * L[l + K * j];
-            }
-        }
-        __syncthreads();
-    }
-    // W = L^{-T} (upper triangular), one column per thread
-    if (tid < nt) {
-        const int c = tid;
-        for (int i = nt - 1; i >= 0; --i) {
-            if (!keep[i] || !keep[c]) {
-                W[i + K * c] = 0.0;
-                continue;
-            }
-            double v = (i == c) ? 1.0 : 0.0;
-            for (int p = i + 1; p < nt; ++p) v -= L[p + K * i] * W[p + K * c];
-            W[i + K * c] = v / L[i + K * i];
-        }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    chol_winv(S, Gs, K + 1, nt, kin, tol, W, keep);
+    double dev = 0.0;  // max |W - I|, |F| over this thread's entries
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, c = idx / nt;
         Wo[i + (long long)nt * c] = W[i + K * c];
-    }
-    double dev = 0.0;  // max |W - I|, |F| over this thread's entries
-    for (int idx = tid; idx < nt * nt; idx += 64) {
-        const int i = idx % nt, c = idx / nt;
         dev = fmax(dev, fabs(W[i + K * c] - (i == c ? 1.0 : 0.0)));
     }
     if (Fo)
-        for (int idx = tid; idx < m * nt; idx += 64) {
+        for (int idx = tid; idx < m * nt; idx += kOT) {
             const int a = idx % m, c = idx / m;
             double f = 0.0;
             for (int i = 0; i < nt; ++i) f -= h[a + m * i] * W[i + K * c];
@@ -1148,90 +1190,50 @@ __device__ void orth_factor(const double *__restrict__ hg, int hld, const double
         kout[tid] = keep[tid];
         if (kcopy) kcopy[tid] = keep[tid];
     }
-    if (skip) {
-        int dropped = (tid < nt && !keep[tid]) ? 1 : 0;
+    if (skip) {  // uniform over the workgroup
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            dev = fmax(dev, __shfl_xor(dev, off, 64));
-            dropped |= __shfl_xor(dropped, off, 64);
-        }
-        if (tid == 0) *skip = (!dropped && dev < skip_tol) ? 1 : 0;
-    }
-}
-
-// Cholesky with dropping of the nt x nt matrix A (LDS, ld kBdMaxK; its lower
-// triangle is overwritten), then W = L^{-T} (zero columns for dropped ones).
-// Column j is kept if kin[j] (null: all) and its pivot exceeds tol * dref[j].
-// All 64 threads take part.
-__device__ void chol_winv(double *A, const double *dref, int nt, const int *kin, double tol,
-                          double *L, double *W, int *keep)
-{
-    constexpr int K = kBdMaxK;
-    const int tid = threadIdx.x;
-    for (int idx = tid; idx < nt * nt; idx += 64) L[(idx % nt) + K * (idx / nt)] = 0.0;
-    __syncthreads();
-    for (int j = 0; j < nt; ++j) {
+        for (int off = 32; off >= 1; off >>= 1) dev = fmax(dev, __shfl_xor(dev, off, 64));
+        if ((tid & 63) == 0) s_dev[tid >> 6] = dev;
+        __syncthreads();
         if (tid == 0) {
-            const double d = A[j + K * j];
-            const int ki = kin ? kin[j] : 1;
-            const int kj = (ki && d > tol * dref[j] && d > 0.0) ? 1 : 0;
-            keep[j] = kj;
-            L[j + K * j] = kj ? sqrt(d) : 0.0;
-        }
-        __syncthreads();
-        if (keep[j]) {
-            const double ljj = L[j + K * j];
-            for (int i = j + 1 + tid; i < nt; i += 64) L[i + K * j] = A[i + K * j] / ljj;
-            __syncthreads();
-            for (int idx = tid; idx < nt * nt; idx += 64) {
-                const int i = idx % nt, l = idx / nt;
-                if (l > j && i >= l) A[i + K * l] -= L[i + K * j] * L[l + K * j];
-            }
-        }
-        __syncthreads();
-    }
-    if (tid < nt) {
-        const int c = tid;
-        for (int i = nt - 1; i >= 0; --i) {
-            if (!keep[i] || !keep[c]) {
-                W[i + K * c] = 0.0;
-                continue;
-            }
-            double v = (i == c) ? 1.0 : 0.0;
-            for (int p = i + 1; p < nt; ++p) v -= L[p + K * i] * W[p + K * c];
-            W[i + K * c] = v / L[i + K * i];
+            for (int w = 1; w < kOT / 64; ++w) dev = fmax(dev, s_dev[w]);
+            int dropped = 0;
+            for (int j = 0; j < nt; ++j) dropped |= keep[j] ? 0 : 1;
+            *skip = (!dropped && dev < skip_tol) ? 1 : 0;
         }
     }
-    __syncthreads();
 }
 
 // S is written one column at a time (rows 0 .. of the basis it then had), so
 // only its upper triangle is current: S(a, b) = S[min + lds * max]
-__device__ __forceinline__ double sym_at(cptr<double> S, int lds, int a, int b)
-{
-    return a <= b ? S[a + (long long)lds * b] : S[b + (long long)lds * a];
-}
 
-__global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__ tasks)
+__global__ void __launch_bounds__(kOT) orth2_kernel(const Orth2Task *__restrict__ tasks)
 {
     constexpr int K = kBdMaxK, M = kBdMaxM;
     const Orth2Task &t = tasks[blockIdx.x];
     const int m = t.m, nt = t.nt, ma = m + nt, tid = threadIdx.x;
     __shared__ double h0[M * K], F1[M * K], h1[M * K];
-    __shared__ double G0[K * K], A[K * K], L[K * K], W1[K * K], W2[K * K], G1[K * K], dref[K];
+    __shared__ double G0[K * K], A[K * K], W1[K * K], W2[K * K], G1[K * K], dref[K];
     __shared__ int keep1[K], keep2[K];
-    // h0, G0 from the chunk partials (fixed order per entry)
-    for (int idx = tid; idx < ma * nt; idx += 64) {
-        const int a = idx % ma, c = idx / ma;
-        const double *p = t.part + t.part_off + (long long)(a + ma * c) * t.nch;
-        double sum = 0.0;
-        for (int q = 0; q < t.nch; ++q) sum += p[q];
+    // S in full, so that the products below read it from LDS; its loads are in
+    // flight with the partials'
+    __shared__ double Ss[M * (M + 1)];
+    const cptr<double> Sv = cst(t.Sv);
+    for (int idx = tid; idx < m * m; idx += kOT) {
+        const int a = idx % m, b = idx / m;
+        if (a > b) continue;
+        const double v = Sv[a + (long long)t.lds * b];
+        Ss[a + (M + 1) * b] = v;
+        Ss[b + (M + 1) * a] = v;
+    }
+    // h0, G0 from the chunk partials
+    part_sums(t.part, t.part_off, t.nch, ma, nt, [&](int a, int c, double sum) {
         if (a < m) h0[a + M * c] = sum;
         else G0[(a - m) + K * c] = sum;
-    }
+    });
     __syncthreads();
     // round 1
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, j = idx / nt;
         double v = G0[i + K * j];
         for (int a = 0; a < m; ++a) v -= h0[a + M * i] * h0[a + M * j];
@@ -1249,10 +1251,10 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
         }
         s_alg = ok;
     }
-    chol_winv(A, dref, nt, nullptr, t.tol1, L, W1, keep1);
+    chol_winv(A, dref, 1, nt, nullptr, t.tol1, W1, keep1);
     const bool alg = s_alg != 0;  // written before chol_winv's barriers
     // F1 = -h0 W1; P = h0 W1 (kept in h1 for now)
-    for (int idx = tid; idx < m * nt; idx += 64) {
+    for (int idx = tid; idx < m * nt; idx += kOT) {
         const int a = idx % m, c = idx / m;
         double pv = 0.0;
         for (int i = 0; i < nt; ++i) pv += h0[a + M * i] * W1[i + K * c];
@@ -1262,11 +1264,11 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
     __syncthreads();
     if (!alg) {
         // round 1 alone; the second round runs on the data
-        for (int idx = tid; idx < nt * nt; idx += 64) {
+        for (int idx = tid; idx < nt * nt; idx += kOT) {
             const int i = idx % nt, c = idx / nt;
             t.W[i + (long long)nt * c] = W1[i + K * c];
         }
-        for (int idx = tid; idx < m * nt; idx += 64) {
+        for (int idx = tid; idx < m * nt; idx += kOT) {
             const int a = idx % m, c = idx / m;
             t.F[a + (long long)m * c] = F1[a + M * c];
         }
@@ -1280,16 +1282,15 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
     }
     // Q = S F1, then h1 = P + Q and
     // G1 = W1^T G0 W1 + P^T F1 + F1^T P + F1^T Q (P = h0 W1, held in h1)
-    const cptr<double> Sv = cst(t.Sv);
     __shared__ double Q[M * K];
-    for (int idx = tid; idx < m * nt; idx += 64) {
+    for (int idx = tid; idx < m * nt; idx += kOT) {
         const int a = idx % m, c = idx / m;
         double v = 0.0;
-        for (int b = 0; b < m; ++b) v += sym_at(Sv, t.lds, a, b) * F1[b + M * c];
+        for (int b = 0; b < m; ++b) v += Ss[a + (M + 1) * b] * F1[b + M * c];
         Q[a + M * c] = v;
     }
     __syncthreads();
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, j = idx / nt;
         if (i < j) continue;
         double v = 0.0;
@@ -1304,13 +1305,13 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
         G1[j + K * i] = v;
     }
     __syncthreads();
-    for (int idx = tid; idx < m * nt; idx += 64) {
+    for (int idx = tid; idx < m * nt; idx += kOT) {
         const int a = idx % m, c = idx / m;
         h1[a + M * c] += Q[a + M * c];
     }
     __syncthreads();
     // round 2
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, j = idx / nt;
         double v = G1[i + K * j];
         for (int a = 0; a < m; ++a) v -= h1[a + M * i] * h1[a + M * j];
@@ -1318,17 +1319,17 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
     }
     if (tid < nt) dref[tid] = G1[tid + K * tid];
     __syncthreads();
-    chol_winv(A, dref, nt, keep1, t.tol2, L, W2, keep2);
+    chol_winv(A, dref, 1, nt, keep1, t.tol2, W2, keep2);
     // W = W1 W2 (into W1's place: Wm), F = (F1 - h1) W2 (into F1's place)
     __shared__ double Wm[K * K];
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, c = idx / nt;
         double v = 0.0;
         for (int p = 0; p < nt; ++p) v += W1[i + K * p] * W2[p + K * c];
         Wm[i + K * c] = v;
         t.W[i + (long long)nt * c] = v;
     }
-    for (int idx = tid; idx < m * nt; idx += 64) {
+    for (int idx = tid; idx < m * nt; idx += kOT) {
         const int a = idx % m, c = idx / m;
         double v = 0.0;
         for (int p = 0; p < nt; ++p) v += (F1[a + M * p] - h1[a + M * p]) * W2[p + K * c];
@@ -1341,21 +1342,21 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
     // V^T T' = P' + Q',  T'^T T' = W^T G0 W + P'^T F + F^T P' + F^T Q'
     // (the rounding of the stored block, ~1e-10 here, is not captured; every
     // restart rebuilds S from the data)
-    for (int idx = tid; idx < m * nt; idx += 64) {
+    for (int idx = tid; idx < m * nt; idx += kOT) {
         const int a = idx % m, c = idx / m;
         double pv = 0.0, qv = 0.0;
         for (int p = 0; p < nt; ++p) pv += h0[a + M * p] * Wm[p + K * c];
-        for (int b = 0; b < m; ++b) qv += sym_at(Sv, t.lds, a, b) * Q[b + M * c];
+        for (int b = 0; b < m; ++b) qv += Ss[a + (M + 1) * b] * Q[b + M * c];
         F1[a + M * c] = pv;  // P'
         h1[a + M * c] = qv;  // Q'
     }
     __syncthreads();
     double *So = t.Sout;
-    for (int idx = tid; idx < m * nt; idx += 64) {
+    for (int idx = tid; idx < m * nt; idx += kOT) {
         const int a = idx % m, c = idx / m;
         So[a + (long long)t.lds * (m + c)] = F1[a + M * c] + h1[a + M * c];
     }
-    for (int idx = tid; idx < nt * nt; idx += 64) {
+    for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, j = idx / nt;
         if (i > j) continue;
         double v = 0.0;
@@ -1378,7 +1379,7 @@ __global__ void __launch_bounds__(64) orth2_kernel(const Orth2Task *__restrict__
     }
 }
 
-__global__ void __launch_bounds__(64) orth_kernel(const OrthTask *__restrict__ tasks)
+__global__ void __launch_bounds__(kOT) orth_kernel(const OrthTask *__restrict__ tasks)
 {
     const OrthTask &t = tasks[blockIdx.x];
     if (t.noop && *cst(t.noop)) return;
@@ -1387,7 +1388,7 @@ __global__ void __launch_bounds__(64) orth_kernel(const OrthTask *__restrict__ t
                 t.tol, t.skip, t.skip_tol, t.part, t.part_off, t.nch);
 }
 
-__global__ void __launch_bounds__(64) cholinv_batched_kernel(const CholTask *__restrict__ tasks)
+__global__ void __launch_bounds__(kOT) cholinv_batched_kernel(const CholTask *__restrict__ tasks)
 {
     const CholTask &t = tasks[blockIdx.x];
     orth_factor(nullptr, 0, t.G, t.k, 0, t.k, t.W, nullptr, t.keep_in, t.keep_out, t.keep_copy, t.tol);
@@ -1409,14 +1410,10 @@ __global__ void __launch_bounds__(kT) prec_kernel(const PrecTask *__restrict__ t
 }
 
 // ------------------------------------------------------------------ restart directions
-// One 64-lane workgroup per task; lane = coefficient row (m <= 64).
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
+// One 64-lane workgroup per task; lane = coefficient row (m <= 64).  A chain of
+// k (2 k + c + 1) dot products over the lanes, so the time is that of one dot
+// product: the sum goes through the VALU's lane moves (k = 8, m = 32: 47.8 us
+// through the LDS, 21.6 us here).
 __global__ void __launch_bounds__(64) coef_kernel(const CoefTask *__restrict__ tasks)
 {
     const CoefTask t = tasks[blockIdx.x];
@@ -1440,17 +1437,17 @@ __global__ void __launch_bounds__(64) coef_kernel(const CoefTask *__restrict__ t
 #pragma unroll
             for (int j = 0; j < kBdMaxK; ++j) {
                 if (j >= t.k) break;
-                const double h = wave_sum(y[j] * q[c]);
+                const double h = lanes_sum(y[j] * q[c]);
                 q[c] -= h * y[j];
             }
 #pragma unroll
             for (int j = 0; j < kBdMaxK; ++j) {
                 if (j >= c) break;
                 if (!keep[j]) continue;
-                const double h = wave_sum(q[j] * q[c]);
+                const double h = lanes_sum(q[j] * q[c]);
                 q[c] -= h * q[j];
             }
-            nrm = sqrt(wave_sum(q[c] * q[c]));
+            nrm = sqrt(lanes_sum(q[c] * q[c]));
             if (!(nrm > 1e-14)) break;  // the direction is numerically zero
             q[c] /= nrm;
         }
@@ -1491,7 +1488,7 @@ bool gram_narrow(int mb)
     return on && mb <= kGNarrowB;
 }
 
-int gram_chunks(long long N) { return (int)((N + g_gram.rows - 1) / g_gram.rows); }
+int gram_rows() { return g_gram.rows; }
 
 int gram_blocks_per_chunk(int ma, int mb)
 {
@@ -1500,24 +1497,27 @@ int gram_blocks_per_chunk(int ma, int mb)
 }
 
 void bd_gram(const GramTask *d_tasks, int ntasks, int max_blocks, int max_blocks_narrow,
-             int max_mamb, double *d_partial, hipStream_t s, bool reduce)
+             int max_mamb, int max_nch, double *d_partial, hipStream_t s, bool reduce)
 {
     if (ntasks <= 0) return;
-    const int v = g_gram.variant, rows = g_gram.rows;
+    const int v = g_gram.variant;
     if (max_blocks_narrow > 0)
         hipLaunchKernelGGL(gram_narrow_kernel, dim3(max_blocks_narrow, ntasks), dim3(kT), 0, s,
                            d_tasks, d_partial);
     if (max_blocks <= 0) {
     } else if (v == 0)
-        hipLaunchKernelGGL(gram_valu_kernel, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial, rows);
+        hipLaunchKernelGGL(gram_valu_kernel, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial);
     else if (v == 1)
-        hipLaunchKernelGGL(gram_kernel<0>, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial, rows);
+        hipLaunchKernelGGL(gram_kernel<0>, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial);
     else
-        hipLaunchKernelGGL(gram_kernel<1>, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial, rows);
-    if (reduce)
-        hipLaunchKernelGGL(gram_reduce_kernel,
-                           dim3((max_mamb + kT / kGramRedLanes - 1) / (kT / kGramRedLanes), ntasks), dim3(kT), 0,
-                           s, d_tasks, d_partial);
+        hipLaunchKernelGGL(gram_kernel<1>, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial);
+    if (reduce) {
+        auto grid = [&](int L) { return dim3((max_mamb + kT / L - 1) / (kT / L), ntasks); };
+        if (max_nch <= kGramPartMax)
+            hipLaunchKernelGGL(gram_reduce_kernel<8>, grid(8), dim3(kT), 0, s, d_tasks, d_partial);
+        else
+            hipLaunchKernelGGL(gram_reduce_kernel<64>, grid(64), dim3(kT), 0, s, d_tasks, d_partial);
+    }
     PC_HIP(hipGetLastError());
 }
 
@@ -1614,14 +1614,14 @@ void bd_ritz(const RitzTask *d_tasks, int ntasks, int max_nch, int k, double *d_
 void bd_orth2(const Orth2Task *d_tasks, int ntasks, hipStream_t s)
 {
     if (ntasks <= 0) return;
-    hipLaunchKernelGGL(orth2_kernel, dim3(ntasks), dim3(64), 0, s, d_tasks);
+    hipLaunchKernelGGL(orth2_kernel, dim3(ntasks), dim3(kOT), 0, s, d_tasks);
     PC_HIP(hipGetLastError());
 }
 
 void bd_orth(const OrthTask *d_tasks, int ntasks, hipStream_t s)
 {
     if (ntasks <= 0) return;
-    hipLaunchKernelGGL(orth_kernel, dim3(ntasks), dim3(64), 0, s, d_tasks);
+    hipLaunchKernelGGL(orth_kernel, dim3(ntasks), dim3(kOT), 0, s, d_tasks);
     PC_HIP(hipGetLastError());
 }
 
@@ -1650,7 +1650,7 @@ void bd_precond(const PrecTask *d_tasks, int ntasks, long long max_N, hipStream_
 void bd_cholinv(const CholTask *d_tasks, int ntasks, hipStream_t s)
 {
     if (ntasks <= 0) return;
-    hipLaunchKernelGGL(cholinv_batched_kernel, dim3(ntasks), dim3(64), 0, s, d_tasks);
+    hipLaunchKernelGGL(cholinv_batched_kernel, dim3(ntasks), dim3(kOT), 0, s, d_tasks);
     PC_HIP(hipGetLastError());
 }
 

@@ -20,10 +20,11 @@ struct GramTask {
     long long N;
     double *out; int out_ld;
     long long part_off;  // this task's region of the partial buffer (doubles)
-    int nch;             // row chunks (gram_chunks(N))
+    int nch;             // row chunks of `rows` rows each
     int cpb;             // workgroups per chunk (gram_blocks_per_chunk(ma, mb))
     int kind;            // 0: the configured variant; 1: narrow-B VALU kernel (gram_narrow)
     const int *skip;     // optional: the task does nothing when *skip != 0 (set by an earlier launch)
+    int rows;            // rows per chunk (a multiple of 256)
 };
 
 // Y (set|-=|+=) A1 W1 + A2 W2 + A3 W3, W in device memory (column-major);
@@ -167,7 +168,7 @@ struct CoefTask {
 // max_blocks / max_blocks_narrow: max over the tasks of kind 0 / 1 of nch * cpb;
 // reduce = false leaves the partials to the consumer (OrthTask::part)
 void bd_gram(const GramTask *d_tasks, int ntasks, int max_blocks, int max_blocks_narrow,
-             int max_mamb, double *d_partial, hipStream_t s, bool reduce = true);
+             int max_mamb, int max_nch, double *d_partial, hipStream_t s, bool reduce = true);
 // max_mb: max over the tasks of mb
 void bd_combine(const CombTask *d_tasks, int ntasks, long long max_N, int max_mb, hipStream_t s);
 void bd_eig(const EigTask *d_tasks, int ntasks, hipStream_t s);
@@ -190,6 +191,17 @@ constexpr int kGRowsValu = 256 * 32; // VALU variant: rows per chunk (32 per thr
 // three lanes: 544 against 535 solves/s; 2048 rows: 538).
 constexpr int kGNarrowA = 8, kGNarrowB = 4, kGRowsNarrow = 256 * 16;
 bool gram_narrow(int mb);
+// A launch with fewer than kGramFill workgroups at these sizes halves its rows
+// per workgroup until it has them, down to kGRowsMin.  Two workgroups a CU: one
+// 64^3 instance made 64 of 4096 rows, and its launches left three CUs of four
+// idle (matrix-core kernel 70.2 us; 256 workgroups of 1024 rows 30.0 us).  The
+// block solve of one (H2O)24 64^3 instance: 26.7 ms at 4096 rows, 22.9 at 2048,
+// 21.4 at 1024, 21.5 at 512, 22.3 at 256 (each chunk is a partial sum to be
+// added up).  A batch that fills the chip keeps the configured rows.
+constexpr int kGramFill = 512, kGRowsMin = 1024;
+// chunks per entry up to which the small factor kernels sum them themselves
+// (eight loads by eight lanes); with more the reduction kernel does, 4.7 us
+constexpr int kGramPartMax = 64;
 // Gram kernel variant (0 VALU register tiles, 1 matrix cores with 16-row
 // blocks, 2 matrix cores with 64-row runs) and rows per workgroup, and the
 // task sizing they imply.
@@ -198,7 +210,7 @@ void gram_set(int variant, int rows);
 void gram_load_config();
 int gram_config(int *rows);
 int gram_variant();
-int gram_chunks(long long N);
+int gram_rows();
 int gram_blocks_per_chunk(int ma, int mb);
 constexpr int kBdResChunk = 1024; // rows per residual chunk
 // rows per Ritz workgroup for block size k (RitzTask::nch = ceil(N / ritz_rows(k)))

@@ -315,7 +315,7 @@ namespace {
 
 struct GramBatch {
     GramTask *h = nullptr, *d = nullptr;
-    int n = 0, max_blocks = 0, max_blocks_narrow = 0, max_mamb = 0;
+    int n = 0, max_blocks = 0, max_blocks_narrow = 0, max_mamb = 0, max_nch = 0;
     long long part = 0;
     bool reduce = true;  // false: every task's consumer sums the partials itself
     // tasks are sized (row chunks, workgroups, partial offsets) in finish(),
@@ -325,26 +325,32 @@ struct GramBatch {
     {
         PC_REQUIRE(ma >= 1 && ma <= kBdMaxM && mb >= 1 && mb <= kGramMaxB, PISCES_ERR_ARG,
                    "Gram task exceeds the kernel's column limits");
-        h[n++] = GramTask{A, N, ma, a32, B, N, mb, b32, N, out, out_ld, 0, 0, 0, 0};
+        h[n++] = GramTask{A, N, ma, a32, B, N, mb, b32, N, out, out_ld, 0, 0, 0, 0, nullptr, 0};
         max_mamb = std::max(max_mamb, ma * mb);
     }
     void finish()
     {
         part = 0;
-        max_blocks = max_blocks_narrow = 0;
+        max_blocks = max_blocks_narrow = max_nch = 0;
+        // workgroups at the configured rows; too few of them are made more
+        long long wg = 0;
         for (int i = 0; i < n; ++i) {
             GramTask &t = h[i];
-            t.part_off = part;
             t.kind = gram_narrow(t.mb) ? 1 : 0;
-            if (t.kind) {
-                t.nch = (int)((t.N + kGRowsNarrow - 1) / kGRowsNarrow);
-                t.cpb = (t.ma + kGNarrowA - 1) / kGNarrowA;
-                max_blocks_narrow = std::max(max_blocks_narrow, t.nch * t.cpb);
-            } else {
-                t.nch = gram_chunks(t.N);
-                t.cpb = gram_blocks_per_chunk(t.ma, t.mb);
-                max_blocks = std::max(max_blocks, t.nch * t.cpb);
-            }
+            t.rows = t.kind ? kGRowsNarrow : gram_rows();
+            t.cpb = t.kind ? (t.ma + kGNarrowA - 1) / kGNarrowA : gram_blocks_per_chunk(t.ma, t.mb);
+            wg += (t.N + t.rows - 1) / t.rows * t.cpb;
+        }
+        int half = 0;
+        while ((wg << half) < kGramFill && half < 4) ++half;
+        for (int i = 0; i < n; ++i) {
+            GramTask &t = h[i];
+            for (int k = 0; k < half && t.rows / 2 >= kGRowsMin && (t.rows / 2) % 256 == 0; ++k) t.rows /= 2;
+            t.nch = (int)((t.N + t.rows - 1) / t.rows);
+            int &mx = t.kind ? max_blocks_narrow : max_blocks;
+            mx = std::max(mx, t.nch * t.cpb);
+            max_nch = std::max(max_nch, t.nch);
+            t.part_off = part;
             part += (long long)t.ma * t.mb * t.nch;
         }
     }
@@ -372,7 +378,7 @@ struct GramBatch {
     {
         if (!n) return;
         ProfScope ps(all_skip() ? PK_CHOL : PK_GRAM, s, prof_enabled() ? bytes() : 0.0);
-        bd_gram(d, n, max_blocks, max_blocks_narrow, max_mamb, dp, s, reduce);
+        bd_gram(d, n, max_blocks, max_blocks_narrow, max_mamb, max_nch, dp, s, reduce);
     }
 };
 
@@ -1065,10 +1071,13 @@ int BdEngine::step_b()
     grow_part(sizeof(double) * (size_t)partB);
     double *dp = dpart_.as<double>();
     for (int pass = 0; pass < 2; ++pass) {
+        // many chunks per entry: a reduction over the whole chip, and the factor
+        // kernels read its sums
+        if (og[pass].max_nch > kGramPartMax) og_red[pass] = true;
         og[pass].reduce = og_red[pass];
         for (int i = 0; i < nc; ++i) {
             const int q = og_idx[pass][i];
-            if (q < 0) continue;
+            if (q < 0 || og[pass].max_nch > kGramPartMax) continue;
             hot[pass][i].part = dp;
             hot[pass][i].part_off = og[pass].h[q].part_off;
             hot[pass][i].nch = og[pass].h[q].nch;
@@ -1076,9 +1085,10 @@ int BdEngine::step_b()
     }
     for (int q = 0; q < n2; ++q) {
         const GramTask &gt = og[0].h[og_idx[0][o2_inst[q]]];
-        h2t[q].part = dp;
-        h2t[q].part_off = gt.part_off;
-        h2t[q].nch = gt.nch;
+        const bool red = og[0].max_nch > kGramPartMax;  // sums: one chunk per entry
+        h2t[q].part = red ? gt.out : dp;
+        h2t[q].part_off = red ? 0 : gt.part_off;
+        h2t[q].nch = red ? 1 : gt.nch;
     }
     B.flush(s_);
     {

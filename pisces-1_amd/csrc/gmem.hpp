@@ -79,4 +79,19 @@ __device__ __forceinline__ double row_sum(double x)
     return dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(x))));
 }
 
+// lane l's value of x, uniform over the wave
+__device__ __forceinline__ double lane_value(double x, int l)
+{
+    const long long v = __builtin_bit_cast(long long, x);
+    const int lo = __builtin_amdgcn_readlane((int)v, l);
+    const int hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+// the sum of the 64 lanes of a wave, in all of them
+__device__ __forceinline__ double lanes_sum(double x)
+{
+    const double r = row_sum(x);
+    return (lane_value(r, 0) + lane_value(r, 16)) + (lane_value(r, 32) + lane_value(r, 48));
+}
+
 }  // namespace pisces
