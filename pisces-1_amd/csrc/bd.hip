@@ -667,25 +667,38 @@ constexpr int kEigSweeps = 40;
 
 // Cyclic Jacobi with round-robin pairing: every round applies m/2 disjoint
 // rotations J as A <- J^T A J in one pass over 2 x 2 blocks (rows of one
-// pair, columns of another: each block reads and writes only its own four
-// entries) and V <- V J.  A pair is rotated only while its off-diagonal entry
-// is above 1e-17 (|a_pp| + |a_qq|); sweeps end after one with no rotation or
-// once the off-diagonal Frobenius norm is 1e-14 of the total.
+// pair, columns of another) and V <- V J.  A pair is rotated only while its
+// off-diagonal entry is above 1e-17 (|a_pp| + |a_qq|); sweeps end after one with
+// no rotation or once the off-diagonal Frobenius norm is 1e-14 of the total.
+// A round waits on its own chain: three entries, a rotation, the entries it
+// turns.  So every wave computes all the rotations for itself (lane = pair; the
+// waves would wait for one of them otherwise) and reads them back from its own
+// piece of LDS, A goes from one of two copies to the other, and a round has one
+// barrier; a thread loads its blocks before the rotations are known.  m = 8 .. 32
+// (one (H2O)24 64^3 instance, blocks of 8): 127.9 us with the rotations of one
+// wave published behind a second barrier, 114.9 us so.
 __global__ void __launch_bounds__(kEigT) eig_kernel(const EigTask *__restrict__ tasks)
 {
     const EigTask &t = tasks[blockIdx.x];
     constexpr int LD = kBdMaxM + 1;
-    __shared__ double A[kBdMaxM * LD];
+    __shared__ double As[2][kBdMaxM * LD];
     __shared__ double V[kBdMaxM * LD];
-    __shared__ double cs[kBdMaxM / 2], sn[kBdMaxM / 2];
-    __shared__ int pp[kBdMaxM / 2], qq[kBdMaxM / 2];
+    __shared__ f64x2 rot[kEigT / 64][kBdMaxM / 2];  // (c, s) of each pair, per wave
     __shared__ double red[kEigT / 64][2];
     __shared__ int order[kBdMaxM];
-    __shared__ int s_stop, s_rot;
     const int m = t.m, tid = threadIdx.x;
+    const int mp = m + (m & 1);
+    double *A = As[0];
     const int mw = (t.Vfull && t.mwarm > 0 && t.mwarm <= m) ? t.mwarm : 0;
-    for (int idx = tid; idx < m * m; idx += kEigT) {
-        const int i = idx % m, j = idx / m;
+    // odd m: a row and a column of zeros make up the last pair, which is never
+    // rotated and stays zero
+    for (int idx = tid; idx < mp * mp; idx += kEigT) {
+        const int i = idx % mp, j = idx / mp;
+        if (i >= m || j >= m) {
+            A[i + LD * j] = 0.0;
+            V[i + LD * j] = 0.0;
+            continue;
+        }
         double g = (i <= j) ? t.G[i + (long long)t.ldg * j] : t.G[j + (long long)t.ldg * i];
         const bool di = t.keep && !t.keep[i];
         const bool dj = t.keep && !t.keep[j];
@@ -700,7 +713,7 @@ __global__ void __launch_bounds__(kEigT) eig_kernel(const EigTask *__restrict__ 
         // and A[i, j] = A[j, i] = Tm[i, j] for i >= mw > j.  The leading block
         // comes out diagonal up to rounding (Vp diagonalised it last step), so
         // only the new rows and columns are left to rotate.
-        __shared__ double Tm[kBdMaxM * LD];
+        double *Tm = As[1];
         for (int idx = tid; idx < m * mw; idx += kEigT) {
             const int i = idx % m, j = idx / m;
             double acc = 0.0;
@@ -721,11 +734,11 @@ __global__ void __launch_bounds__(kEigT) eig_kernel(const EigTask *__restrict__ 
         }
         __syncthreads();
     }
-    const int mp = m + (m & 1);
     const int npair = mp / 2;
     const int lane = tid & 63, wave = tid >> 6;
-    // this thread's 2 x 2 blocks (b = tid + kEigT q) and V items, fixed for
-    // every round: their pair indices are divided out once here
+    // this thread's 2 x 2 blocks and V items, fixed for every round: their pair
+    // indices are divided out once here.  The V items are dealt from the last
+    // thread on, so that few threads have both
     constexpr int kNB = (kBdMaxM / 2) * (kBdMaxM / 2) / kEigT, kNV = kBdMaxM * (kBdMaxM / 2) / kEigT;
     int bP1[kNB], bP2[kNB], vK[kNV], vP[kNV];
 #pragma unroll
@@ -736,10 +749,16 @@ __global__ void __launch_bounds__(kEigT) eig_kernel(const EigTask *__restrict__ 
     }
 #pragma unroll
     for (int q = 0; q < kNV; ++q) {
-        const int item = tid + kEigT * q;
+        const int item = (kEigT - 1 - tid) + kEigT * q;
         vK[q] = item % m;
         vP[q] = item / m;
     }
+    const int nblock = npair * npair, nitem = m * npair;
+    auto pair_of = [&](int i, int r, int &p, int &q) {
+        const int x = rr_index(i, r, mp), y = rr_index(mp - 1 - i, r, mp);
+        p = min(x, y);
+        q = max(x, y);
+    };
     for (int sweep = 0; sweep < kEigSweeps; ++sweep) {
         double off = 0.0, tot = 0.0;
         for (int idx = tid; idx < m * m; idx += kEigT) {
@@ -748,91 +767,95 @@ __global__ void __launch_bounds__(kEigT) eig_kernel(const EigTask *__restrict__ 
             if (i != j && fabs(A[i + LD * i]) < 1e29 && fabs(A[j + LD * j]) < 1e29) off += a * a;
             else if (i == j && fabs(a) < 1e29) tot += a * a;
         }
-        for (int o = 32; o >= 1; o >>= 1) {
-            off += __shfl_xor(off, o, 64);
-            tot += __shfl_xor(tot, o, 64);
-        }
+        off = lanes_sum(off);
+        tot = lanes_sum(tot);
         if (lane == 0) {
             red[wave][0] = off;
             red[wave][1] = tot;
         }
         __syncthreads();
-        if (tid == 0) {
-            double so = 0, st = 0;
-            for (int w = 0; w < kEigT / 64; ++w) {
-                so += red[w][0];
-                st += red[w][1];
-            }
-            s_stop = (so <= 1e-28 * (st + so)) ? 1 : 0;
-            s_rot = 0;
+        double so = 0, st = 0;
+        for (int w = 0; w < kEigT / 64; ++w) {
+            so += red[w][0];
+            st += red[w][1];
         }
-        __syncthreads();
-        if (s_stop) break;
+        if (so <= 1e-28 * (st + so)) break;  // the same sums in every thread
+        bool any = false;                    // of all rotations of the sweep, the same in every wave
         for (int r = 0; r < mp - 1; ++r) {
-            if (tid < npair) {
-                int p = rr_index(tid, r, mp), q = rr_index(mp - 1 - tid, r, mp);
-                if (p > q) { const int x = p; p = q; q = x; }
-                double c = 1.0, s = 0.0;
-                if (q < m) {
-                    const double apq = A[p + LD * q];
-                    const double app = A[p + LD * p], aqq = A[q + LD * q];
-                    if (fabs(apq) > 1e-17 * (fabs(app) + fabs(aqq)) + 1e-300) {
-                        // t = tan of the annihilating angle to ~1 ulp; any t
-                        // gives an exact rotation (c^2 + s^2 = 1 to rounding)
-                        const double th = (aqq - app) * rcp64(2.0 * apq);
-                        double tt;
-                        if (fabs(th) > 1e150) {
-                            tt = 0.5 * rcp64(th);
-                        } else {
-                            const double h = fma(th, th, 1.0);
-                            tt = copysign(rcp64(fabs(th) + h * rsq64(h)), th);
-                        }
-                        c = rsq64(fma(tt, tt, 1.0));
-                        s = tt * c;
-                        s_rot = 1;  // every writer stores 1
+            double *const An = A == As[0] ? As[1] : As[0];
+            double blk[kNB][4];
+            int at[kNB][4];
+#pragma unroll
+            for (int x = 0; x < kNB; ++x) {
+                if (tid + kEigT * x >= nblock) break;
+                int p1, q1, p2, q2;
+                pair_of(bP1[x], r, p1, q1);
+                pair_of(bP2[x], r, p2, q2);
+                at[x][0] = p1 + LD * p2;
+                at[x][1] = p1 + LD * q2;
+                at[x][2] = q1 + LD * p2;
+                at[x][3] = q1 + LD * q2;
+#pragma unroll
+                for (int y = 0; y < 4; ++y) blk[x][y] = A[at[x][y]];
+            }
+            double c = 1.0, s = 0.0;
+            if (lane < npair) {
+                int p, q;
+                pair_of(lane, r, p, q);
+                const double apq = A[p + LD * q];
+                const double app = A[p + LD * p], aqq = A[q + LD * q];
+                if (fabs(apq) > 1e-17 * (fabs(app) + fabs(aqq)) + 1e-300) {
+                    // cos and sin of the annihilating angle, tan 2 phi = b / d: with
+                    // x = |d| / sqrt(d^2 + b^2), c^2 = (1 + x) / 2 and
+                    // s = b / (2 c sqrt(d^2 + b^2)); c^2 + s^2 = 1 to rounding.
+                    // The larger of |d|, |b| is brought near 1 where the squares
+                    // could leave the range.
+                    double d = aqq - app, b = 2.0 * apq;
+                    const double big = fmax(fabs(d), fabs(b));
+                    if (big > 1e150 || big < 1e-130) {
+                        int e;
+                        (void)frexp(big, &e);
+                        d = ldexp(d, -e);
+                        b = ldexp(b, -e);
                     }
+                    const double rs = rsq64(fma(d, d, b * b));
+                    const double c2 = fma(0.5 * fabs(d), rs, 0.5);
+                    const double rc = rsq64(c2);
+                    c = c2 * rc;
+                    s = (d < 0.0 ? -0.5 : 0.5) * b * rs * rc;
                 }
-                pp[tid] = p;
-                qq[tid] = q;
-                cs[tid] = c;
-                sn[tid] = s;
+                rot[wave][lane] = f64x2{c, s};
             }
-            __syncthreads();
+            any |= __any(s != 0.0) != 0;
+            __builtin_amdgcn_wave_barrier();  // the wave's LDS operations stay in order
 #pragma unroll
-            for (int qb = 0; qb < kNB; ++qb) {
-                if (tid + kEigT * qb >= npair * npair) break;
-                const int P1 = bP1[qb], P2 = bP2[qb];
-                const double s1 = sn[P1], s2 = sn[P2];
-                if (s1 == 0.0 && s2 == 0.0) continue;
-                const double c1 = cs[P1], c2 = cs[P2];
-                const int p1 = pp[P1], q1 = qq[P1], p2 = pp[P2], q2 = qq[P2];
-                const bool v1 = q1 < m, v2 = q2 < m;
-                const double b00 = A[p1 + LD * p2];
-                const double b01 = v2 ? A[p1 + LD * q2] : 0.0;
-                const double b10 = v1 ? A[q1 + LD * p2] : 0.0;
-                const double b11 = (v1 && v2) ? A[q1 + LD * q2] : 0.0;
-                const double x00 = b00 * c2 - b01 * s2, x01 = b00 * s2 + b01 * c2;
-                const double x10 = b10 * c2 - b11 * s2, x11 = b10 * s2 + b11 * c2;
-                A[p1 + LD * p2] = c1 * x00 - s1 * x10;
-                if (v2) A[p1 + LD * q2] = c1 * x01 - s1 * x11;
-                if (v1) A[q1 + LD * p2] = s1 * x00 + c1 * x10;
-                if (v1 && v2) A[q1 + LD * q2] = s1 * x01 + c1 * x11;
+            for (int x = 0; x < kNB; ++x) {
+                if (tid + kEigT * x >= nblock) break;
+                const f64x2 r1 = rot[wave][bP1[x]], r2 = rot[wave][bP2[x]];
+                const double c1 = r1[0], s1 = r1[1], c2 = r2[0], s2 = r2[1];
+                const double x00 = blk[x][0] * c2 - blk[x][1] * s2, x01 = blk[x][0] * s2 + blk[x][1] * c2;
+                const double x10 = blk[x][2] * c2 - blk[x][3] * s2, x11 = blk[x][2] * s2 + blk[x][3] * c2;
+                An[at[x][0]] = c1 * x00 - s1 * x10;
+                An[at[x][1]] = c1 * x01 - s1 * x11;
+                An[at[x][2]] = s1 * x00 + c1 * x10;
+                An[at[x][3]] = s1 * x01 + c1 * x11;
             }
 #pragma unroll
-            for (int qv = 0; qv < kNV; ++qv) {
-                if (tid + kEigT * qv >= m * npair) break;
-                const int k = vK[qv], pr = vP[qv];
-                const double s = sn[pr];
-                if (s == 0.0) continue;
-                const int p = pp[pr], q = qq[pr];
-                const double c = cs[pr];
+            for (int x = 0; x < kNV; ++x) {
+                if ((kEigT - 1 - tid) + kEigT * x >= nitem) break;
+                const f64x2 rv = rot[wave][vP[x]];
+                if (rv[1] == 0.0) continue;
+                int p, q;
+                pair_of(vP[x], r, p, q);
+                const int k = vK[x];
                 const double vkp = V[k + LD * p], vkq = V[k + LD * q];
-                V[k + LD * p] = c * vkp - s * vkq;
-                V[k + LD * q] = s * vkp + c * vkq;
+                V[k + LD * p] = rv[0] * vkp - rv[1] * vkq;
+                V[k + LD * q] = rv[1] * vkp + rv[0] * vkq;
             }
             __syncthreads();
+            A = An;
         }
-        if (!s_rot) break;  // uniform: read after the round's final barrier
+        if (!any) break;
     }
     // ascending order by rank (ties by index)
     if (tid < m) {
