@@ -263,23 +263,18 @@ int build_potential_impl(pisces_ctx *c, const int flags[6], const double *potpar
                    "PolType 3 takes the polarizable-site lists (pisces_build_potential_scp)");
         P.ion_r = ion_r;
         c->last_sites.assign(sites, sites + 3 * (size_t)nsites);
-        dbuf ds, dq, diq, dd, did, drep, direp, dipps, dix, diq2, drp, depc, dinv;
-        upload(ds, sites, sizeof(double) * 3 * nsites, c->stream);
-        if (nq) { upload(dq, q, sizeof(double) * nq, c->stream); upload(diq, iq, sizeof(int) * nq, c->stream); }
-        if (nd) { upload(dd, d, sizeof(double) * 3 * nd, c->stream); upload(did, id, sizeof(int) * nd, c->stream); }
-        if (!rep.empty()) {
-            upload(drep, rep.data(), sizeof(double) * rep.size(), c->stream);
-            upload(direp, irep.data(), sizeof(int) * irep.size(), c->stream);
-        }
-        if (!ipps.empty()) upload(dipps, ipps.data(), sizeof(int) * ipps.size(), c->stream);
+        dbuf dent, dd, drep, dix, diq2, drp, depc, dinv;
+        std::vector<double> rep_by_site(rep);
+        const std::vector<PotSite> ent = pot_sites(nsites, sites, nq, q, iq, nd, id, rep_by_site, irep, ipps);
+        if (!ent.empty()) upload(dent, ent.data(), sizeof(PotSite) * ent.size(), c->stream);
+        if (nd) upload(dd, d, sizeof(double) * 3 * nd, c->stream);
+        if (!rep.empty()) upload(drep, rep_by_site.data(), sizeof(double) * rep.size(), c->stream);
         if (nion) {
             upload(dix, ion_xyz, sizeof(double) * 3 * nion, c->stream);
             upload(diq2, ion_q, sizeof(double) * nion, c->stream);
         }
-        PotDev D{nsites, nq, nd, (int)irep.size(), (int)ipps.size(), nion,
-                 ds.as<double>(), dq.as<double>(), diq.as<int>(), dd.as<double>(), did.as<int>(),
-                 drep.as<double>(), direp.as<int>(), dipps.as<int>(), dix.as<double>(),
-                 diq2.as<double>()};
+        PotDev D{nsites, (int)ent.size(), nion, dent.as<PotSite>(), dd.as<double>(), drep.as<double>(),
+                 dix.as<double>(), diq2.as<double>()};
         const int n3p = np > 0 ? pol3_padded(np) : 0;
         PC_REQUIRE(n3p <= kPol3MaxN, PISCES_ERR_UNSUPPORTED, "too many polarizable sites");
         std::vector<double> rp((size_t)3 * np), ep((size_t)n3p, 0.0);

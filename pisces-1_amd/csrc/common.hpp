@@ -145,13 +145,26 @@ bool potential_setup(const int *flags, const double *pp, int nsites, PotParams &
                      std::vector<double> &rep, std::vector<int> &irep,
                      std::vector<int> &ipps);
 
+// One site of the cluster as the grid pass reads it: what acts from one point
+// shares its distance.  dip: index of its point dipole or -1; its cores are
+// rep[2 c], rep[2 c + 1] (exponent, factor) for r0 <= c < r1; pol: 1 if it is a
+// non-interacting polarizable site.
+struct PotSite {
+    double x, y, z, q;
+    int dip, r0, r1, pol;
+};
+// The lists of a cluster by site, in the order of the sites; a second charge,
+// dipole or polarizability of one site goes into another entry for it.  rep is
+// put into the order of the entries.
+std::vector<PotSite> pot_sites(int nsites, const double *sites, int nq, const double *q, const int *iq, int nd,
+                               const int *id, std::vector<double> &rep, const std::vector<int> &irep,
+                               const std::vector<int> &ipps);
 struct PotDev {
-    int nsites, nq, nd, nrep, npps, nion;
-    const double *sites;   // 3*nsites
-    const double *q; const int *iq;
-    const double *d; const int *id;
-    const double *rep; const int *irep;
-    const int *ipps;
+    int nsites;            // sites of the cluster
+    int nent, nion;
+    const PotSite *ent;    // nent entries (pot_sites)
+    const double *d;       // point dipoles
+    const double *rep;
     const double *ion_xyz; const double *ion_q;
 };
 void potential_grid_launch(const PotParams &P, const PotDev &D, int nx, int ny, int nz,
@@ -166,8 +179,8 @@ struct PotTask {
     double *v;
     float *v32;
 };
-void potential_grid_batched_launch(const PotParams &P, const PotTask *d_tasks, int ntasks,
-                                   long long max_ng, hipStream_t s);
+void potential_grid_batched_launch(const PotParams &P, const PotTask *h_tasks, const PotTask *d_tasks,
+                                   int ntasks, hipStream_t s);
 int potential_max_sites();
 
 // ------------------------------------- self-consistent polarization (PolType 3)

@@ -56,10 +56,9 @@ __device__ __forceinline__ double rcp64(double x)
 }
 __device__ __forceinline__ double rsq64(double x)
 {
-    double y = __builtin_amdgcn_rsq(x);
-    y = y * fma(-0.5 * x, y * y, 1.5);
-    y = y * fma(-0.5 * x, y * y, 1.5);
-    return y;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 // x plus x of the lane that a DPP control names, and sums over groups of lanes

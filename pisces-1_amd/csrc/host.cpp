@@ -456,6 +456,37 @@ bool sym_inverse(int n, std::vector<double> &A, int n3p, double *inva, int metho
 }
 
 // ------------------------------------------------------------------ potential
+std::vector<PotSite> pot_sites(int nsites, const double *sites, int nq, const double *q, const int *iq, int nd,
+                               const int *id, std::vector<double> &rep, const std::vector<int> &irep,
+                               const std::vector<int> &ipps)
+{
+    struct Lists {
+        std::vector<int> q, d, rep;
+        int pol = 0;
+    };
+    std::vector<Lists> at((size_t)nsites);
+    for (int i = 0; i < nq; ++i) at[iq[i]].q.push_back(i);
+    for (int i = 0; i < nd; ++i) at[id[i]].d.push_back(i);
+    for (size_t i = 0; i < irep.size(); ++i) at[irep[i]].rep.push_back((int)i);
+    for (int s : ipps) ++at[s].pol;
+    std::vector<PotSite> out;
+    std::vector<double> r;
+    for (int s = 0; s < nsites; ++s) {
+        const Lists &l = at[s];
+        const size_t n = std::max({l.q.size(), l.d.size(), (size_t)l.pol, (size_t)(l.rep.empty() ? 0 : 1)});
+        for (size_t i = 0; i < n; ++i) {
+            PotSite e{sites[3 * s], sites[3 * s + 1], sites[3 * s + 2], i < l.q.size() ? q[l.q[i]] : 0.0,
+                      i < l.d.size() ? l.d[i] : -1, (int)(r.size() / 2), 0, (int)i < l.pol ? 1 : 0};
+            if (i == 0)
+                for (int c : l.rep) r.insert(r.end(), {rep[2 * c], rep[2 * c + 1]});
+            e.r1 = (int)(r.size() / 2);
+            out.push_back(e);
+        }
+    }
+    rep.swap(r);
+    return out;
+}
+
 // Potential::SetupDPPGTOP (src/Potential.cpp:234-593) with the repulsive cores
 // Set6GTORepCore / Set12GTORepCore / Set4STORepCore (:598-728).  The numeric
 // tables are the reference's published model parameters.

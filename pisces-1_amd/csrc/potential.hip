@@ -3,17 +3,16 @@
 //
 // Grid build: DVR::ComputePotential with sampling 1 (src/DVR.cpp:661-859) calls
 // Potential::Evaluate (src/Potential.cpp:128-182) -> EvaluateDPPGTOP (:844-956)
-// at every grid point.  Here one thread evaluates one grid point; the site,
-// charge, dipole, repulsive-core and polarizable-site tables of the cluster are
-// staged once per workgroup in LDS (at most a few KB) and every thread walks
-// them.  The per-site distance table of the reference (Rx, Ry, Rz, R2, R,
-// Rminus3; src/Potential.cpp:136-146) is recomputed per use instead of stored,
-// with the same expressions, so the FP64 result agrees with the reference to
-// rounding.  The work is N_grid x N_site FP64 arithmetic with one reciprocal
-// square root per site (1/R to ~1 ulp; R, R^-3, R^-4 follow by products, exact
-// divisions only inside the damping radii) and one exp per repulsive core:
-// compute-bound on the FP64 VALU.  The per-cluster tables are read as scalar
-// loads through the constant address space.
+// at every grid point.  The work is N_grid x N_site FP64 arithmetic, compute-bound
+// on the FP64 VALU: a reciprocal square root per distance (1/R to ~1 ulp; R, R^-3,
+// R^-4 follow by products, exact divisions only inside the damping radii) and one
+// exp per repulsive core.  So the cluster's lists are merged by site on the host
+// (a water's three charges, three dipoles, four cores and one polarizability sit
+// on four sites: four distances instead of eleven), a thread of a large launch
+// takes two points of one column, which share x, y and the entry's loads, and the entries are read as
+// scalar loads through the constant address space.  The per-site distance table
+// of the reference (Rx, Ry, Rz, R2, R, Rminus3; src/Potential.cpp:136-146) is
+// recomputed instead of stored, with expressions that agree with it to rounding.
 #include "common.hpp"
 #include "gmem.hpp"
 
@@ -25,11 +24,14 @@ namespace pisces {
 namespace {
 
 constexpr int kPotThreads = 256;
-constexpr int kMaxSites = 1024;  // LDS budget check (4 sites per water)
-
-struct SiteLds {
-    double x, y, z;
-};
+constexpr int kMaxSites = 1024;
+// Points of a thread: 2 from kPotTwo points a launch on, 1 below, where the waves
+// would be too few to cover the entries' loads.  us, 1 / 2 points: one 24-water
+// 64^3 grid (262144 points) 68 / 74, 45 waters 96^3 (884736) 300 / 253, 32
+// grids of 24 waters 64^3 in one launch 1590 / 1279; 4 points: 97, 273, 1269.
+// (Eleven distances a water and one point: 98, 358, 2505.)
+constexpr long long kPotTwo = 524288;
+int pot_points(long long points) { return points >= kPotTwo ? 2 : 1; }
 
 __device__ inline double reff(double r, double r0)
 {
@@ -44,131 +46,146 @@ __device__ inline double reff(double r, double r0)
 // |r| from r^2 and 1/|r| (0 at r = 0, where 1/|r| is infinite)
 __device__ __forceinline__ double norm_of(double r2, double ri) { return r2 > 0.0 ? r2 * ri : 0.0; }
 
-__device__ __forceinline__ void potential_point(const PotParams &P, const PotDev &D, const SiteLds *__restrict__ S,
-                                int nx, int ny, int nz, const double *__restrict__ gx,
-                                const double *__restrict__ gy, const double *__restrict__ gz,
-                                double *__restrict__ v, float *__restrict__ v32, long long g)
+// Thread t of a grid: the points (i, j, k), (i, j, k + zh), ... of a column,
+// zh = ceil(nz / K).
+template <int DAMP, int K>
+__device__ __forceinline__ void potential_points(const PotParams &P, const PotDev &D, int nx, int ny, int nz,
+                                 const double *__restrict__ gx, const double *__restrict__ gy,
+                                 const double *__restrict__ gz, double *__restrict__ v,
+                                 float *__restrict__ v32, long long t)
 {
-    const int i = (int)(g % nx);
-    const int j = (int)((g / nx) % ny);
-    const int k = (int)(g / ((long long)nx * ny));
-    const double r0 = gx[i], r1 = gy[j], r2 = gz[k];
-    const cptr<double> q = cst(D.q), dm = cst(D.d), rp = cst(D.rep), ionx = cst(D.ion_xyz),
-                       ionq = cst(D.ion_q);
-    const cptr<int> iq = cst(D.iq), id = cst(D.id), irep = cst(D.irep), ipps = cst(D.ipps);
-
-    // point charges, src/Potential.cpp:1168-1210
-    double vpc = 0.0;
-    for (int c = 0; c < D.nq; ++c) {
-        const SiteLds s = S[iq[c]];
-        const double rx = r0 - s.x, ry = r1 - s.y, rz = r2 - s.z;
-        const double R2 = rx * rx + ry * ry + rz * rz;
-        const double ri = rsq64(R2);
-        if (P.damp_type == 1) {
-            vpc += -q[c] * ri * (1.0 - exp(-P.qdamp * R2));
-        } else {
-            const double R = norm_of(R2, ri);
-            vpc += (R < P.qdamp) ? -q[c] / reff(R, P.qdamp) : -q[c] * ri;
-        }
+    const int zh = (nz + K - 1) / K;
+    const long long nxy = (long long)nx * ny;
+    if (t >= nxy * zh) return;
+    int i, j, k0;
+    if (nxy * zh <= 0x7fffffff) {  // 32-bit divisions; uniform
+        const unsigned u = (unsigned)t, w = u / (unsigned)nx;
+        i = (int)(u - w * (unsigned)nx);
+        k0 = (int)(w / (unsigned)ny);
+        j = (int)(w - (unsigned)k0 * (unsigned)ny);
+    } else {
+        const long long w = t / nx;
+        i = (int)(t - w * nx);
+        k0 = (int)(w / ny);
+        j = (int)(w - (long long)k0 * ny);
     }
-    // point dipoles, src/Potential.cpp:1222-1270
-    double vind = 0.0;
-    for (int c = 0; c < D.nd; ++c) {
-        const SiteLds s = S[id[c]];
-        const double rx = r0 - s.x, ry = r1 - s.y, rz = r2 - s.z;
-        const double R2 = rx * rx + ry * ry + rz * rz;
-        const double ri = rsq64(R2);
-        const double dot = rx * dm[3 * c] + ry * dm[3 * c + 1] + rz * dm[3 * c + 2];
-        double rm3 = ri * ri * ri;
-        if (P.damp_type == 1) {
-            const double dd = 1.0 - exp(-P.ddamp * R2);
-            vind += -dot * rm3 * dd * dd;
-        } else {
-            const double R = norm_of(R2, ri);
-            if (R < P.ddamp) {
-                const double re = reff(R, P.ddamp);
-                rm3 = 1.0 / (re * re * re);
-            }
-            vind += -dot * rm3;
+    const double r0 = gx[i], r1 = gy[j];
+    double r2[K];
+#pragma unroll
+    for (int p = 0; p < K; ++p) r2[p] = gz[min(k0 + p * zh, nz - 1)];
+    const cptr<double> ionx = cst(D.ion_xyz), ionq = cst(D.ion_q);
+    const cptr<PotSite> ent = cst(D.ent);
+    const cptr<double> dm = cst(D.d), rp = cst(D.rep);
+    double vpc[K] = {}, vind[K] = {}, vrep[K] = {}, sp[K] = {};
+    const double qd2 = P.qdamp * P.qdamp, dd2 = P.ddamp * P.ddamp, pd2 = P.pdamp * P.pdamp;
+    for (int c = 0; c < D.nent; ++c) {
+        const cptr<PotSite> ep = ent + c;
+        const PotSite e{ep->x, ep->y, ep->z, ep->q, ep->dip, ep->r0, ep->r1, ep->pol};
+        const double ez = e.z, eq = e.q;
+        const int dip = e.dip, c0 = e.r0, c1 = e.r1, pol = e.pol;
+        const double rx = r0 - e.x, ry = r1 - e.y, rxy = rx * rx + ry * ry;
+        double rz[K], R2[K], ri[K];
+#pragma unroll
+        for (int p = 0; p < K; ++p) {
+            rz[p] = r2[p] - ez;
+            R2[p] = fma(rz[p], rz[p], rxy);
+            ri[p] = rsq64(R2[p]);
         }
-    }
-    // repulsive cores, src/Potential.cpp:1282-1315
-    double vrep = 0.0;
-    if (P.rep_type > 0) {
-        for (int c = 0; c < D.nrep; ++c) {
-            const SiteLds s = S[irep[c]];
-            const double rx = r0 - s.x, ry = r1 - s.y, rz = r2 - s.z;
-            const double R2 = rx * rx + ry * ry + rz * rz;
-            if (P.rep_type == 1) vrep += rp[2 * c + 1] * exp(-rp[2 * c] * R2);
-            else vrep += rp[2 * c + 1] * exp(-rp[2 * c] * norm_of(R2, rsq64(R2)));
-        }
-    }
-    // polarization of non-interacting sites, src/Potential.cpp:1331-1374, :875-887
-    double vpol = 0.0;
-    if (P.pol_type == 1) {
-        double sp = 0.0;
-        for (int c = 0; c < D.npps; ++c) {
-            const SiteLds s = S[ipps[c]];
-            const double rx = r0 - s.x, ry = r1 - s.y, rz = r2 - s.z;
-            const double rsq = rx * rx + ry * ry + rz * rz;
-            const double ri = rsq64(rsq), ri2 = ri * ri;
-            if (P.damp_type == 1) {
-                const double dd = 1.0 - exp(-P.pdamp * rsq);
-                sp += P.alpha * dd * dd * (ri2 * ri2);
-            } else {
-                const double R = norm_of(rsq, ri);
-                if (R < P.pdamp) {
-                    const double re = reff(R, P.pdamp);
-                    const double re2 = re * re;
-                    sp += P.alpha * rsq / (re2 * re2 * re2);
+        // point charge, src/Potential.cpp:1168-1210
+        if (eq != 0.0) {
+#pragma unroll
+            for (int p = 0; p < K; ++p) {
+                if (DAMP == 1) {
+                    vpc[p] += -eq * ri[p] * (1.0 - exp(-P.qdamp * R2[p]));
                 } else {
-                    sp += P.alpha * (ri2 * ri2);
+                    double u = ri[p];
+                    if (R2[p] < qd2) u = 1.0 / reff(norm_of(R2[p], ri[p]), P.qdamp);
+                    vpc[p] = fma(-eq, u, vpc[p]);
                 }
             }
         }
-        vpol = P.adiabatic ? P.eps - sqrt(P.eps * (P.eps + sp)) : -0.5 * sp;
+        // point dipole, src/Potential.cpp:1222-1270
+        if (dip >= 0) {
+            const double dz = dm[3 * dip + 2], dxy = rx * dm[3 * dip] + ry * dm[3 * dip + 1];
+#pragma unroll
+            for (int p = 0; p < K; ++p) {
+                const double dot = fma(rz[p], dz, dxy);
+                double rm3 = ri[p] * ri[p] * ri[p];
+                if (DAMP == 1) {
+                    const double dd = 1.0 - exp(-P.ddamp * R2[p]);
+                    vind[p] += -dot * rm3 * dd * dd;
+                } else {
+                    if (R2[p] < dd2) {
+                        const double re = reff(norm_of(R2[p], ri[p]), P.ddamp);
+                        rm3 = 1.0 / (re * re * re);
+                    }
+                    vind[p] = fma(-dot, rm3, vind[p]);
+                }
+            }
+        }
+        // repulsive cores, src/Potential.cpp:1282-1315
+        for (int r = c0; r < c1; ++r) {
+            const double ea = rp[2 * r], ef = rp[2 * r + 1];
+#pragma unroll
+            for (int p = 0; p < K; ++p)
+                vrep[p] = fma(ef, exp(-ea * (P.rep_type == 1 ? R2[p] : norm_of(R2[p], ri[p]))), vrep[p]);
+        }
+        // polarization of a non-interacting site, src/Potential.cpp:1331-1374, :875-887
+        if (pol) {
+#pragma unroll
+            for (int p = 0; p < K; ++p) {
+                const double ri2 = ri[p] * ri[p];
+                double u = ri2 * ri2;
+                if (DAMP == 1) {
+                    const double dd = 1.0 - exp(-P.pdamp * R2[p]);
+                    u *= dd * dd;
+                } else if (R2[p] < pd2) {
+                    const double re = reff(norm_of(R2[p], ri[p]), P.pdamp), re2 = re * re;
+                    u = R2[p] / (re2 * re2 * re2);
+                }
+                sp[p] = fma(P.alpha, u, sp[p]);
+            }
+        }
     }
-    // ions: erf-damped charges (Bloomfield form, src/NaCl.cpp:300-307)
-    double vion = 0.0;
-    for (int c = 0; c < D.nion; ++c) {
-        const double rx = r0 - ionx[3 * c], ry = r1 - ionx[3 * c + 1], rz = r2 - ionx[3 * c + 2];
-        const double R2 = rx * rx + ry * ry + rz * rz;
-        const double ri = rsq64(R2);
-        vion += -ionq[c] * erf(norm_of(R2, ri) / P.ion_r) * ri;
+#pragma unroll
+    for (int p = 0; p < K; ++p) {
+        const int k = k0 + p * zh;
+        if (k >= nz) break;
+        double vt = vpc[p] + vind[p] + vrep[p];
+        if (P.pol_type == 1) vt += P.adiabatic ? P.eps - sqrt(P.eps * (P.eps + sp[p])) : -0.5 * sp[p];
+        // ions: erf-damped charges (Bloomfield form, src/NaCl.cpp:300-307)
+        for (int c = 0; c < D.nion; ++c) {
+            const double rx = r0 - ionx[3 * c], ry = r1 - ionx[3 * c + 1], rz = r2[p] - ionx[3 * c + 2];
+            const double R2 = rx * rx + ry * ry + rz * rz;
+            const double ri = rsq64(R2);
+            vt += -ionq[c] * erf(norm_of(R2, ri) / P.ion_r) * ri;
+        }
+        const long long g = i + (long long)nx * j + nxy * k;
+        if (v) v[g] = vt;
+        if (v32) v32[g] = (float)vt;
     }
-    const double vt = vpc + vind + vrep + vpol + vion;
-    if (v) v[g] = vt;
-    if (v32) v32[g] = (float)vt;
 }
 
+template <int K>
 __global__ void __launch_bounds__(kPotThreads)
 potential_grid_kernel(PotParams P, PotDev D, int nx, int ny, int nz, const double *__restrict__ gx,
                       const double *__restrict__ gy, const double *__restrict__ gz,
                       double *__restrict__ v, float *__restrict__ v32)
 {
-    __shared__ SiteLds S[kMaxSites];
-    for (int s = threadIdx.x; s < D.nsites; s += blockDim.x)
-        S[s] = SiteLds{D.sites[3 * s], D.sites[3 * s + 1], D.sites[3 * s + 2]};
-    __syncthreads();
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (long long)nx * ny * nz) return;
-    potential_point(P, D, S, nx, ny, nz, gx, gy, gz, v, v32, g);
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (P.damp_type == 1) potential_points<1, K>(P, D, nx, ny, nz, gx, gy, gz, v, v32, t);
+    else potential_points<2, K>(P, D, nx, ny, nz, gx, gy, gz, v, v32, t);
 }
 
 // many clusters in one launch: blockIdx.y selects the task
+template <int K>
 __global__ void __launch_bounds__(kPotThreads)
 potential_grid_batched_kernel(PotParams P, const PotTask *__restrict__ tasks)
 {
-    const PotTask &t = tasks[blockIdx.y];
-    const long long ng = (long long)t.nx * t.ny * t.nz;
-    if ((long long)blockIdx.x * blockDim.x >= ng) return;
-    __shared__ SiteLds S[kMaxSites];
-    for (int s = threadIdx.x; s < t.D.nsites; s += blockDim.x)
-        S[s] = SiteLds{t.D.sites[3 * s], t.D.sites[3 * s + 1], t.D.sites[3 * s + 2]};
-    __syncthreads();
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ng) return;
-    potential_point(P, t.D, S, t.nx, t.ny, t.nz, t.gx, t.gy, t.gz, t.v, t.v32, g);
+    const PotTask &q = tasks[blockIdx.y];
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (P.damp_type == 1) potential_points<1, K>(P, q.D, q.nx, q.ny, q.nz, q.gx, q.gy, q.gz, q.v, q.v32, t);
+    else potential_points<2, K>(P, q.D, q.nx, q.ny, q.nz, q.gx, q.gy, q.gz, q.v, q.v32, t);
 }
 
 // --------------------------------------------------------------------------
@@ -417,21 +434,30 @@ void potential_grid_launch(const PotParams &P, const PotDev &D, int nx, int ny, 
                            const double *d_x, const double *d_y, const double *d_z,
                            double *d_v, float *d_v32, hipStream_t s)
 {
-    PC_REQUIRE(D.nsites <= kMaxSites, PISCES_ERR_UNSUPPORTED, "too many sites for the LDS table");
-    const long long ng = (long long)nx * ny * nz;
-    const unsigned blocks = (unsigned)((ng + kPotThreads - 1) / kPotThreads);
-    hipLaunchKernelGGL(potential_grid_kernel, dim3(blocks), dim3(kPotThreads), 0, s, P, D, nx,
-                       ny, nz, d_x, d_y, d_z, d_v, d_v32);
+    PC_REQUIRE(D.nsites <= kMaxSites, PISCES_ERR_UNSUPPORTED, "too many sites");
+    const int K = pot_points((long long)nx * ny * nz);
+    const long long threads = (long long)nx * ny * ((nz + K - 1) / K);
+    const unsigned blocks = (unsigned)((threads + kPotThreads - 1) / kPotThreads);
+    auto *kernel = K == 2 ? potential_grid_kernel<2> : potential_grid_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kPotThreads), 0, s, P, D, nx, ny, nz, d_x, d_y, d_z, d_v,
+                       d_v32);
     PC_HIP(hipGetLastError());
 }
 
-void potential_grid_batched_launch(const PotParams &P, const PotTask *d_tasks, int ntasks,
-                                   long long max_ng, hipStream_t s)
+void potential_grid_batched_launch(const PotParams &P, const PotTask *h_tasks, const PotTask *d_tasks,
+                                   int ntasks, hipStream_t s)
 {
     if (ntasks <= 0) return;
-    const unsigned blocks = (unsigned)((max_ng + kPotThreads - 1) / kPotThreads);
-    hipLaunchKernelGGL(potential_grid_batched_kernel, dim3(blocks, ntasks), dim3(kPotThreads), 0, s,
-                       P, d_tasks);
+    long long points = 0, threads = 0;
+    for (int i = 0; i < ntasks; ++i) points += (long long)h_tasks[i].nx * h_tasks[i].ny * h_tasks[i].nz;
+    const int K = pot_points(points);
+    for (int i = 0; i < ntasks; ++i) {
+        const PotTask &t = h_tasks[i];
+        threads = std::max(threads, (long long)t.nx * t.ny * ((t.nz + K - 1) / K));
+    }
+    const unsigned blocks = (unsigned)((threads + kPotThreads - 1) / kPotThreads);
+    auto *kernel = K == 2 ? potential_grid_batched_kernel<2> : potential_grid_batched_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3(blocks, ntasks), dim3(kPotThreads), 0, s, P, d_tasks);
     PC_HIP(hipGetLastError());
 }
 

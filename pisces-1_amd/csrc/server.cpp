@@ -229,9 +229,9 @@ size_t footprint(pisces_server *sv, long long N, int nroots)
 struct Prep {
     Pending *p;
     std::shared_ptr<InstRes> res;
-    std::vector<double> sites, q, rep;
-    std::vector<int> iq, id, irep, ipps;
-    size_t o_sites, o_q, o_iq, o_id, o_rep, o_irep, o_ipps, o_ion, o_ionq;  // upload offsets
+    std::vector<double> sites, rep;
+    std::vector<PotSite> ent;
+    size_t o_sites, o_ent, o_rep, o_ion, o_ionq;  // upload offsets
     size_t o_mu, o_epc, o_work, o_info;                                   // work offsets
 };
 
@@ -258,18 +258,18 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
         r.sites.resize((size_t)12 * nw);
         PC_REQUIRE(water_sites_host(nw, r.p->xyz.data(), r.sites.data()), PISCES_ERR_NUMERIC,
                    "water projection produced non-finite coordinates");
-        water_lists_host(nw, r.q, r.iq, r.id);
-        PC_REQUIRE(potential_setup(flags, pp, 4 * nw, P, r.rep, r.irep, r.ipps), PISCES_ERR_ARG,
+        std::vector<double> q;
+        std::vector<int> iq, id, irep, ipps;
+        water_lists_host(nw, q, iq, id);
+        PC_REQUIRE(potential_setup(flags, pp, 4 * nw, P, r.rep, irep, ipps), PISCES_ERR_ARG,
                    "potential setup");
+        r.ent = pot_sites(4 * nw, r.sites.data(), (int)q.size(), q.data(), iq.data(), (int)id.size(), id.data(),
+                          r.rep, irep, ipps);
         const int ns = 3 * nw, nion = r.p->req.nion;
         auto put = [&](size_t bytes) { const size_t o = up; up += align256(bytes); return o; };
         r.o_sites = put(sizeof(double) * r.sites.size());
-        r.o_q = put(sizeof(double) * r.q.size());
-        r.o_iq = put(sizeof(int) * r.iq.size());
-        r.o_id = put(sizeof(int) * r.id.size());
+        r.o_ent = put(sizeof(PotSite) * r.ent.size());
         r.o_rep = put(sizeof(double) * r.rep.size());
-        r.o_irep = put(sizeof(int) * r.irep.size());
-        r.o_ipps = put(sizeof(int) * r.ipps.size());
         r.o_ion = put(sizeof(double) * 3 * nion);
         r.o_ionq = put(sizeof(double) * nion);
         auto wput = [&](size_t bytes) { const size_t o = wk; wk += align256(bytes); return o; };
@@ -291,7 +291,6 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
     unsigned char *d = sv->s_up.as<unsigned char>(), *w = sv->s_wk.as<unsigned char>();
     ScfTask *scf = reinterpret_cast<ScfTask *>(h);
     PotTask *pot = reinterpret_cast<PotTask *>(h + align256(sizeof(ScfTask) * nb));
-    long long max_ng = 0;
     int max_nw = 0;
     for (int i = 0; i < nb; ++i) {
         Prep &r = batch[i];
@@ -301,12 +300,8 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
         const int nw = r.p->req.nw, nion = r.p->req.nion;
         max_nw = std::max(max_nw, nw);
         cp(r.o_sites, r.sites.data(), sizeof(double) * r.sites.size());
-        cp(r.o_q, r.q.data(), sizeof(double) * r.q.size());
-        cp(r.o_iq, r.iq.data(), sizeof(int) * r.iq.size());
-        cp(r.o_id, r.id.data(), sizeof(int) * r.id.size());
+        cp(r.o_ent, r.ent.data(), sizeof(PotSite) * r.ent.size());
         cp(r.o_rep, r.rep.data(), sizeof(double) * r.rep.size());
-        cp(r.o_irep, r.irep.data(), sizeof(int) * r.irep.size());
-        cp(r.o_ipps, r.ipps.data(), sizeof(int) * r.ipps.size());
         cp(r.o_ion, r.p->ion_xyz.data(), sizeof(double) * 3 * nion);
         cp(r.o_ionq, r.p->ion_q.data(), sizeof(double) * nion);
         double *mu = reinterpret_cast<double *>(w + r.o_mu);
@@ -316,14 +311,8 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
                          reinterpret_cast<int *>(w + r.o_info)};
         const GridShape &g = *r.res->shape;
         PotTask t{};
-        t.D = PotDev{4 * nw, (int)r.q.size(), (int)r.id.size(), (int)r.irep.size(),
-                     (int)r.ipps.size(), nion, reinterpret_cast<const double *>(d + r.o_sites),
-                     reinterpret_cast<const double *>(d + r.o_q),
-                     reinterpret_cast<const int *>(d + r.o_iq), mu,
-                     reinterpret_cast<const int *>(d + r.o_id),
+        t.D = PotDev{4 * nw, (int)r.ent.size(), nion, reinterpret_cast<const PotSite *>(d + r.o_ent), mu,
                      reinterpret_cast<const double *>(d + r.o_rep),
-                     reinterpret_cast<const int *>(d + r.o_irep),
-                     reinterpret_cast<const int *>(d + r.o_ipps),
                      reinterpret_cast<const double *>(d + r.o_ion),
                      reinterpret_cast<const double *>(d + r.o_ionq)};
         t.nx = g.n[0];
@@ -335,7 +324,6 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
         t.v = r.res->V64.as<double>();
         t.v32 = r.res->V32.as<float>();
         pot[i] = t;
-        max_ng = std::max(max_ng, g.N);
     }
     PC_HIP(hipMemcpyAsync(d, h, up, hipMemcpyHostToDevice, sv->stream));
     {
@@ -347,8 +335,7 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
         for (Prep &r : batch) bytes += (double)r.res->shape->N * (8 + 4 + 8 + 8);
         ProfScope ps(PK_POT, sv->stream, bytes);
         potential_grid_batched_launch(
-            P, reinterpret_cast<const PotTask *>(d + align256(sizeof(ScfTask) * nb)), nb, max_ng,
-            sv->stream);
+            P, pot, reinterpret_cast<const PotTask *>(d + align256(sizeof(ScfTask) * nb)), nb, sv->stream);
         for (Prep &r : batch) {
             const GridShape &g = *r.res->shape;
             diag_h(r.res->V64.as<double>(), g.dT64[0].as<double>(), g.dT64[1].as<double>(),
