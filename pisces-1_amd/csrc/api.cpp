@@ -25,6 +25,7 @@ pisces_ctx::~pisces_ctx()
     if (stream) static_cast<void>(hipStreamSynchronize(stream));
     if (hjobs) static_cast<void>(hipHostFree(hjobs));
     if (hsmall) static_cast<void>(hipHostFree(hsmall));
+    if (hpot) static_cast<void>(hipHostFree(hpot));
     if (stream) static_cast<void>(hipStreamDestroy(stream));
 }
 
@@ -110,6 +111,69 @@ void set_potential_device(pisces_ctx *c)
     to_f32(c->dV64.as<double>(), c->dV32.as<float>(), c->ngp, c->stream);
     c->has_v = true;
 }
+
+// The induced-dipole solve's buffers for nw waters
+struct ScfBufs {
+    double *mu, *epc, *work;
+    int *info;
+};
+ScfBufs scf_bufs(pisces_ctx *c, int nw)
+{
+    const size_t n = 9 * (size_t)nw, work = (water_scf_work_bytes(nw) + 15) / 16 * 2;  // doubles
+    c->wscf.ensure(sizeof(double) * (2 * n + work + 1));
+    double *p = c->wscf.as<double>();
+    return {p + work, p + work + n, p, reinterpret_cast<int *>(p + work + 2 * n)};
+}
+
+// A cluster whose induced dipoles are solved on the way: nw waters at `sites`
+// (the site list), the dipoles in the order of the water model's list
+struct Waters {
+    int nw;
+    double *mu;  // host, 9 nw, or null
+    int ok;      // out: the solve converged
+};
+
+// Tables in one pinned piece of memory and its copy on the device
+class PotTables {
+public:
+    template <typename T> size_t add(const T *p, size_t n)
+    {
+        const size_t at = (used_ + 255) & ~(size_t)255;
+        if (n) items_.push_back({p, at, n * sizeof(T)});
+        used_ = at + n * sizeof(T);
+        return at;
+    }
+    // uploads them, with `tail` more bytes of pinned memory behind
+    void send(pisces_ctx *c, size_t tail)
+    {
+        if (c->pot_busy) c->sync();
+        tail_ = (used_ + 255) & ~(size_t)255;
+        if (c->hpot_cap < tail_ + tail) {
+            if (c->hpot) PC_HIP(hipHostFree(c->hpot));
+            c->hpot = nullptr;
+            c->hpot_cap = 0;
+            PC_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->hpot), tail_ + tail, hipHostMallocDefault));
+            c->hpot_cap = tail_ + tail;
+        }
+        c->dpot.ensure(tail_);
+        c->pot_busy = true;
+        for (const Item &i : items_) std::memcpy(c->hpot + i.at, i.p, i.n);
+        if (used_) PC_HIP(hipMemcpyAsync(c->dpot.p, c->hpot, used_, hipMemcpyHostToDevice, c->stream));
+        dev_ = c->dpot.as<unsigned char>();
+        host_ = c->hpot;
+    }
+    template <typename T> const T *at(size_t o) const { return reinterpret_cast<const T *>(dev_ + o); }
+    void *tail() const { return host_ + tail_; }
+
+private:
+    struct Item {
+        const void *p;
+        size_t at, n;
+    };
+    std::vector<Item> items_;
+    size_t used_ = 0, tail_ = 0;
+    unsigned char *dev_ = nullptr, *host_ = nullptr;
+};
 
 }  // namespace
 
@@ -245,12 +309,18 @@ int pisces_get_potential(const pisces_ctx *c, double *v)
 namespace {
 
 // Potential::Setup + DVR::ComputePotential: the site terms on the grid, then
-// (np > 0, PolType 3) the self-consistent polarization added on top
+// (np > 0, PolType 3) the self-consistent polarization added on top.
+// What bounds a small build is the host: tables go up in one copy from pinned
+// memory and the buffers stay with the context, and with `waters` the dipoles
+// go from the induced-dipole solve to the grid pass on the device, so that the
+// host waits once, at the end.  (H2O)24 64^3 with the values read back (2 MB), of
+// which the kernels take 165 us: 405 us with ten allocations and nine copies a
+// build, 357 us so.
 int build_potential_impl(pisces_ctx *c, const int flags[6], const double *potpara, int nsites,
                          const double *sites, int nq, const double *q, const int *iq, int nd,
                          const double *d, const int *id, int np, const double *alpha,
                          const int *ip, const double *epc, double vpol_ww, int nion,
-                         const double *ion_xyz, const double *ion_q, double ion_r)
+                         const double *ion_xyz, const double *ion_q, double ion_r, Waters *waters = nullptr)
 {
     return guarded([&] {
         PC_HIP(hipSetDevice(c->device));
@@ -263,23 +333,35 @@ int build_potential_impl(pisces_ctx *c, const int flags[6], const double *potpar
                    "PolType 3 takes the polarizable-site lists (pisces_build_potential_scp)");
         P.ion_r = ion_r;
         c->last_sites.assign(sites, sites + 3 * (size_t)nsites);
-        dbuf dent, dd, drep, dix, diq2, drp, depc, dinv;
+        dbuf drp, depc, dinv;
         std::vector<double> rep_by_site(rep);
         const std::vector<PotSite> ent = pot_sites(nsites, sites, nq, q, iq, nd, id, rep_by_site, irep, ipps);
-        if (!ent.empty()) upload(dent, ent.data(), sizeof(PotSite) * ent.size(), c->stream);
-        if (nd) upload(dd, d, sizeof(double) * 3 * nd, c->stream);
-        if (!rep.empty()) upload(drep, rep_by_site.data(), sizeof(double) * rep.size(), c->stream);
-        if (nion) {
-            upload(dix, ion_xyz, sizeof(double) * 3 * nion, c->stream);
-            upload(diq2, ion_q, sizeof(double) * nion, c->stream);
+        PotTables tab;
+        const size_t o_ent = tab.add(ent.data(), ent.size());
+        const size_t o_rep = tab.add(rep_by_site.data(), rep_by_site.size());
+        const size_t o_ix = tab.add(ion_xyz, 3 * (size_t)nion), o_iq = tab.add(ion_q, (size_t)nion);
+        const size_t o_al = tab.add(alpha, (size_t)np), o_d = tab.add(waters ? nullptr : d, waters ? 0 : 3 * (size_t)nd);
+        const size_t o_s = tab.add(sites, waters ? 3 * (size_t)nsites : 0);
+        const size_t nmu = waters ? 9 * (size_t)waters->nw : 0;
+        tab.send(c, sizeof(double) * (nmu + 1));
+        const double *dip = tab.at<double>(o_d);
+        int *info = static_cast<int *>(tab.tail());  // 2 ints, then the dipoles
+        double *mu = static_cast<double *>(tab.tail()) + 1;
+        if (waters) {
+            const ScfBufs w = scf_bufs(c, waters->nw);
+            water_scf_launch(waters->nw, tab.at<double>(o_s), w.mu, w.epc, w.work, w.info, c->stream);
+            PC_HIP(hipMemcpyAsync(info, w.info, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+            if (waters->mu)
+                PC_HIP(hipMemcpyAsync(mu, w.mu, sizeof(double) * nmu, hipMemcpyDeviceToHost, c->stream));
+            dip = w.mu;
         }
-        PotDev D{nsites, (int)ent.size(), nion, dent.as<PotSite>(), dd.as<double>(), drep.as<double>(),
-                 dix.as<double>(), diq2.as<double>()};
+        PotDev D{nsites, (int)ent.size(), nion, tab.at<PotSite>(o_ent), dip, tab.at<double>(o_rep),
+                 tab.at<double>(o_ix), tab.at<double>(o_iq)};
         const int n3p = np > 0 ? pol3_padded(np) : 0;
         PC_REQUIRE(n3p <= kPol3MaxN, PISCES_ERR_UNSUPPORTED, "too many polarizable sites");
         std::vector<double> rp((size_t)3 * np), ep((size_t)n3p, 0.0);
         int *flag = reinterpret_cast<int *>(c->hsmall);
-        dbuf dalpha, dtmp, dflag;
+        dbuf dtmp, dflag;
         if (np > 0) {
             // SetupDPPGTOP case 3 (src/Potential.cpp:387-432): InvA of the
             // polarizable sites, inverted before the grid pass so that the host
@@ -291,11 +373,10 @@ int build_potential_impl(pisces_ctx *c, const int flags[6], const double *potpar
                 }
             upload(drp, rp.data(), sizeof(double) * rp.size(), c->stream);
             upload(depc, ep.data(), sizeof(double) * ep.size(), c->stream);
-            upload(dalpha, alpha, sizeof(double) * np, c->stream);
             dinv.alloc(sizeof(double) * (size_t)n3p * n3p);
             dtmp.alloc(sizeof(double) * 2 * (size_t)n3p * n3p);
             dflag.alloc(sizeof(int));
-            pol3_inva_launch(np, drp.as<double>(), dalpha.as<double>(), n3p, dtmp.as<double>(),
+            pol3_inva_launch(np, drp.as<double>(), tab.at<double>(o_al), n3p, dtmp.as<double>(),
                              dinv.as<double>(), dflag.as<int>(), c->stream);
             PC_HIP(hipMemcpyAsync(flag, dflag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         }
@@ -359,6 +440,11 @@ int build_potential_impl(pisces_ctx *c, const int flags[6], const double *potpar
         }
         set_potential_device(c);
         c->sync();
+        c->pot_busy = false;
+        if (waters) {
+            waters->ok = info[0];
+            if (waters->mu) std::memcpy(waters->mu, mu, sizeof(double) * nmu);
+        }
         return 0;
     });
 }
@@ -422,53 +508,52 @@ int pisces_build_cluster_potential(pisces_ctx *c, int nw, const double *xyz_ang,
         PC_REQUIRE(water_sites_host(nw, xyz_ang, sites.data()), PISCES_ERR_NUMERIC,
                    "water projection produced non-finite coordinates");
         const int ns = 3 * nw;
-        dbuf dsites, dmu, depc, dwork, dinfo;
-        upload(dsites, sites.data(), sizeof(double) * sites.size(), c->stream);
-        dmu.alloc(sizeof(double) * 3 * ns);
-        depc.alloc(sizeof(double) * 3 * ns);
-        dwork.alloc(water_scf_work_bytes(nw));
-        dinfo.alloc(sizeof(int) * 2);
-        water_scf_launch(nw, dsites.as<double>(), dmu.as<double>(), depc.as<double>(),
-                         dwork.as<double>(), dinfo.as<int>(), c->stream);
-        int info[2] = {0, 0};
-        PC_HIP(hipMemcpyAsync(info, dinfo.p, sizeof(info), hipMemcpyDeviceToHost, c->stream));
-        std::vector<double> mu((size_t)3 * ns);
-        PC_HIP(hipMemcpyAsync(mu.data(), dmu.p, sizeof(double) * mu.size(), hipMemcpyDeviceToHost, c->stream));
-        PC_HIP(hipStreamSynchronize(c->stream));
-        if (sites_out) std::memcpy(sites_out, sites.data(), sizeof(double) * sites.size());
-        if (mu_out) std::memcpy(mu_out, mu.data(), sizeof(double) * mu.size());
         std::vector<double> q;
         std::vector<int> iq, id;
         water_lists_host(nw, q, iq, id);
-        int rc;
-        if (flags[3] == 3) {
-            // ReportPolSitesAndField (src/DPP.cpp:540-642): the sites O,H1,H2
-            // with their polarizabilities and permanent-charge field; and
-            // VpolWaterWater = the water-water polarization energy
-            // (src/ClusterAnion.cpp:173; WaterWaterPolarizationEnergy,
-            // src/DPP.cpp:1935-2024, summed over all pairs: -mu.Epc / 2)
-            std::vector<double> epc((size_t)3 * ns);
-            PC_HIP(hipMemcpyAsync(epc.data(), depc.p, sizeof(double) * epc.size(), hipMemcpyDeviceToHost,
-                                  c->stream));
-            PC_HIP(hipStreamSynchronize(c->stream));
-            const double a3 = 1.0 / (0.52917720859 * 0.52917720859 * 0.52917720859);
-            std::vector<double> alpha((size_t)ns);
-            std::vector<int> ip((size_t)ns);
-            double eww = 0.0;
-            for (int i = 0; i < ns; ++i) {
-                alpha[i] = (i % 3 == 0 ? 1.22 : 0.28) * a3;  // src/ttm_data.h:51-52
-                ip[i] = 4 * (i / 3) + i % 3;
-            }
-            for (int k = 0; k < 3 * ns; ++k) eww += mu[k] * epc[k];
-            rc = pisces_build_potential_scp(c, flags, potpara, 4 * nw, sites.data(), (int)q.size(),
-                                            q.data(), iq.data(), ns, alpha.data(), ip.data(),
-                                            epc.data(), -0.5 * eww, nion, ion_xyz_bohr, ion_q,
-                                            ion_r);
-        } else {
-            rc = pisces_build_potential(c, flags, potpara, 4 * nw, sites.data(), (int)q.size(),
-                                        q.data(), iq.data(), (int)id.size(), mu.data(), id.data(),
-                                        nion, ion_xyz_bohr, ion_q, ion_r);
+        if (sites_out) std::memcpy(sites_out, sites.data(), sizeof(double) * sites.size());
+        if (flags[3] != 3) {
+            Waters w{nw, mu_out, 0};
+            const int rc = build_potential_impl(c, flags, potpara, 4 * nw, sites.data(), (int)q.size(), q.data(),
+                                                iq.data(), (int)id.size(), nullptr, id.data(), 0, nullptr, nullptr,
+                                                nullptr, 0.0, nion, ion_xyz_bohr, ion_q, ion_r, &w);
+            return rc < 0 ? rc : w.ok ? 0 : 1;
         }
+        int info[2] = {0, 0};
+        std::vector<double> mu((size_t)3 * ns), epc((size_t)3 * ns);
+        {
+            PotTables tab;
+            const size_t o = tab.add(sites.data(), sites.size()), n = 3 * (size_t)ns;
+            tab.send(c, sizeof(double) * (2 * n + 1));
+            const ScfBufs w = scf_bufs(c, nw);
+            water_scf_launch(nw, tab.at<double>(o), w.mu, w.epc, w.work, w.info, c->stream);
+            // mu, epc and info lie in this order
+            double *h = static_cast<double *>(tab.tail());
+            PC_HIP(hipMemcpyAsync(h, w.mu, sizeof(double) * (2 * n + 1), hipMemcpyDeviceToHost, c->stream));
+            c->sync();
+            c->pot_busy = false;
+            std::copy(h, h + n, mu.begin());
+            std::copy(h + n, h + 2 * n, epc.begin());
+            std::memcpy(info, h + 2 * n, sizeof(info));
+        }
+        if (mu_out) std::memcpy(mu_out, mu.data(), sizeof(double) * mu.size());
+        // ReportPolSitesAndField (src/DPP.cpp:540-642): the sites O,H1,H2
+        // with their polarizabilities and permanent-charge field; and
+        // VpolWaterWater = the water-water polarization energy
+        // (src/ClusterAnion.cpp:173; WaterWaterPolarizationEnergy,
+        // src/DPP.cpp:1935-2024, summed over all pairs: -mu.Epc / 2)
+        const double a3 = 1.0 / (0.52917720859 * 0.52917720859 * 0.52917720859);
+        std::vector<double> alpha((size_t)ns);
+        std::vector<int> ip((size_t)ns);
+        double eww = 0.0;
+        for (int i = 0; i < ns; ++i) {
+            alpha[i] = (i % 3 == 0 ? 1.22 : 0.28) * a3;  // src/ttm_data.h:51-52
+            ip[i] = 4 * (i / 3) + i % 3;
+        }
+        for (int k = 0; k < 3 * ns; ++k) eww += mu[k] * epc[k];
+        const int rc = pisces_build_potential_scp(c, flags, potpara, 4 * nw, sites.data(), (int)q.size(),
+                                                  q.data(), iq.data(), ns, alpha.data(), ip.data(),
+                                                  epc.data(), -0.5 * eww, nion, ion_xyz_bohr, ion_q, ion_r);
         if (rc < 0) return rc;
         return info[0] ? 0 : 1;
     });

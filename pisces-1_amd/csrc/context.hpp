@@ -47,6 +47,12 @@ struct pisces_ctx {
     pisces::dbuf wB, wZ, wU, wZV, wR, wC, wJ, wdiag, wpart, wsmall, winfo, wX, wY;
     pisces::dbuf wB32, wZ32, wC32;
     pisces::dbuf wgrad;  // gradient workspace
+    // potential builds: the cluster's tables (pinned, and their device copy) and
+    // the induced-dipole solve's buffers, kept from build to build
+    pisces::dbuf dpot, wscf;
+    unsigned char *hpot = nullptr;
+    size_t hpot_cap = 0;
+    bool pot_busy = false;  // a build has not been waited for (it failed half-way)
     double *hsmall = nullptr;  // pinned, kSmall doubles
     static constexpr int kSmall = 1 << 16;
 
