@@ -833,7 +833,7 @@ def pol3_measure(P, workload):
         fl_exec = 256.0 * ncb * (ncb + 1) * ng
         fl_ref = 2.0 * n3 * n3 * ng                     # the reference's dsymv per point
         out[tag] = {"n_pol_dims": n3, "grid": n, "ms_kernel": round(1e3 * t, 4),
-                    # the whole build: water model, InvA on the host, uploads, kernels
+                    # the whole build: water model, uploads, InvA and grid kernels
                     "ms_build_total": round(1e3 * t_build, 3),
                     "TFLOPs_executed": round(fl_exec / t / 1e12, 2),
                     "TFLOPs_dsymv_equivalent": round(fl_ref / t / 1e12, 2),

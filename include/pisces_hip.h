@@ -69,7 +69,8 @@ unsigned pisces_debug_hx_spin_timeouts(void);
 /* Inverse of a symmetric n x n matrix (row-major) as the PolType 3 set-up
  * inverts the polarization matrix (ComputeInvA, src/MolPolAux.cpp:39-136, with
  * dsytrf/dsytri there): method 0 Cholesky where positive definite, else
- * Gauss-Jordan with partial pivoting (what pisces_build_potential_scp uses);
+ * Gauss-Jordan with partial pivoting (what pisces_build_potential_scp falls
+ * back on where its inversion on the GPU meets a pivot that is not positive);
  * 1 Cholesky only; 2 Gauss-Jordan only.  Host arithmetic, no device needed.
  * Errors: PISCES_ERR_ARG, PISCES_ERR_NUMERIC (singular; for method 1 also not
  * positive definite). */
@@ -278,9 +279,10 @@ int pisces_kinetic_precond(pisces_ctx *ctx, int nvec, const double *r, double sh
  * the reference; it is for callers that cannot allocate device memory (code
  * under stream capture, serving loops that forbid hipMalloc).  d_r and d_t are
  * distinct device arrays of nvec*ngp doubles.  The per-vector task
- * descriptors and, in the split-BF16 form, the BF16 intermediate between the
- * three plane passes live in a fixed array of pisces_noalloc_scratch_bytes()
- * bytes (32 MiB) that each GPU holds until the process ends, so the split-BF16
+ * descriptors are kernel arguments; in the split-BF16 form the BF16
+ * intermediate between the three plane passes lives in a fixed array of
+ * pisces_noalloc_scratch_bytes() bytes (32 MiB, of which the size limit
+ * below still counts the descriptors) that each GPU holds until the process ends, so the split-BF16
  * form takes at most about 16.7 million grid points x vectors (64^3 x 63
  * vectors); larger requests return PISCES_ERR_ARG before any launch.  All
  * calls on one GPU share that array: calls that overlap in time on one GPU
