@@ -1595,16 +1595,26 @@ int gram_config(int *rows)
     return g_gram.variant;
 }
 
-// rows per thread x columns: 4 x 4, 2 x 8, 1 x 16 (the same accumulator count)
+// rows per thread x columns: 4 x 4, 2 x 8, 1 x 16 (the same accumulator count);
+// fewer rows in a launch that has not kCombFill workgroups (four waves a SIMD) so.
+// One (H2O)24 64^3 instance, blocks of 8: 512 workgroups of 512 rows and none split
+// 21.2 ms a solve, split below 1024 workgroups 20.7, below 2048 20.6; the served
+// batch of 32: 55.0, 55.1, 55.3 ms.
+constexpr int kCombFill = 1024;
 void bd_combine(const CombTask *d_tasks, int ntasks, long long max_N, int max_mb, hipStream_t s)
 {
     if (ntasks <= 0) return;
     PC_REQUIRE(max_mb >= 1 && max_mb <= kBdMaxK, PISCES_ERR_ARG, "combination width 1..16");
     auto grid = [&](int rpt) { return dim3((unsigned)((max_N + kT * rpt - 1) / (kT * rpt)), ntasks); };
     const int rev = kCombReverse;
-    if (max_mb <= 4) hipLaunchKernelGGL((comb_kernel<4, 4>), grid(4), dim3(kT), 0, s, d_tasks, rev);
-    else if (max_mb <= 8) hipLaunchKernelGGL((comb_kernel<8, 2>), grid(2), dim3(kT), 0, s, d_tasks, rev);
-    else hipLaunchKernelGGL((comb_kernel<16, 1>), grid(1), dim3(kT), 0, s, d_tasks, rev);
+    int rpt = max_mb <= 4 ? 4 : max_mb <= 8 ? 2 : 1;
+    while (rpt > 1 && (long long)grid(rpt).x * ntasks < kCombFill) rpt /= 2;
+    auto *kernel = max_mb > 8    ? comb_kernel<16, 1>
+                   : max_mb > 4  ? (rpt == 2 ? comb_kernel<8, 2> : comb_kernel<8, 1>)
+                   : rpt == 4    ? comb_kernel<4, 4>
+                   : rpt == 2    ? comb_kernel<4, 2>
+                                 : comb_kernel<4, 1>;
+    hipLaunchKernelGGL(kernel, grid(rpt), dim3(kT), 0, s, d_tasks, rev);
     PC_HIP(hipGetLastError());
 }
 
