@@ -9,10 +9,11 @@
 // exp per repulsive core.  So the cluster's lists are merged by site on the host
 // (a water's three charges, three dipoles, four cores and one polarizability sit
 // on four sites: four distances instead of eleven), a thread of a large launch
-// takes two points of one column, which share x, y and the entry's loads, and the entries are read as
-// scalar loads through the constant address space.  The per-site distance table
-// of the reference (Rx, Ry, Rz, R2, R, Rminus3; src/Potential.cpp:136-146) is
-// recomputed instead of stored, with expressions that agree with it to rounding.
+// takes two points of one column, which share x, y and the entry's loads, and the
+// entries are read as scalar loads through the constant address space.  The
+// per-site distance table of the reference (Rx, Ry, Rz, R2, R, Rminus3;
+// src/Potential.cpp:136-146) is recomputed instead of stored, with expressions
+// that agree with it to rounding.
 #include "common.hpp"
 #include "gmem.hpp"
 
