@@ -48,9 +48,9 @@ template <typename T> __device__ __forceinline__ void stnt(gptr<T> p, T v)
 // estimate refined by two Newton-Raphson steps, r <- r + r (1 - x r), each
 // squaring the relative error.  The root: one cubic step, y <- y + y e (1/2 + 3 e / 8)
 // with e = 1 - x y^2, which leaves 5 e^3 / 16 of an estimate good to single
-// precision (below 2^-65), the rounding of x y in e (half an ulp) and that of the
-// last sum: no more than two quadratic steps' own roundings, in five operations
-// instead of eight.
+// precision (below 2^-65), the rounding of x y in e and that of the last sum, in
+// five operations.  Against 80-bit arithmetic, 4 M arguments in 2^-8 .. 2^14: at
+// most 0.99 ulp, 0.33 rms; two quadratic steps in eight operations: 1.64, 0.47.
 __device__ __forceinline__ double rcp64(double x)
 {
     double r = __builtin_amdgcn_rcp(x);
