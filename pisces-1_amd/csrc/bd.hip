@@ -530,19 +530,25 @@ __device__ __forceinline__ double group_sum(const double *__restrict__ p, int n,
 
 // Gram entries: L lanes per entry, kT / L entries per workgroup; the entry's
 // chunk partials are summed as above.  8 lanes hold 64 chunks in one run of
-// loads; with more chunks a whole wave takes the entry.
+// loads; with more chunks a whole wave takes the entry (chosen per task, so that
+// a task's sums do not depend on the others of the launch).
 template <int L>
-__global__ void __launch_bounds__(kT) gram_reduce_kernel(const GramTask *__restrict__ tasks,
-                                                         const double *__restrict__ partial)
+__device__ __forceinline__ void gram_reduce(const GramTask &t, const double *__restrict__ partial)
 {
-    const GramTask t = tasks[blockIdx.y];
-    if (t.skip && *cst(t.skip)) return;
     const int o = blockIdx.x * (kT / L) + threadIdx.x / L;
     const int j = threadIdx.x & (L - 1);
     // whole lane groups leave together, so the group's shuffles see only live lanes
     if (o >= t.ma * t.mb) return;
     const double s = group_sum<L>(partial + t.part_off + (long long)o * t.nch, t.nch, j);
     if (j == 0) t.out[(o % t.ma) + (long long)t.out_ld * (o / t.ma)] = s;
+}
+__global__ void __launch_bounds__(kT) gram_reduce_kernel(const GramTask *__restrict__ tasks,
+                                                         const double *__restrict__ partial)
+{
+    const GramTask t = tasks[blockIdx.y];
+    if (t.skip && *cst(t.skip)) return;
+    if (t.nch <= kGramPartMax) gram_reduce<8>(t, partial);
+    else gram_reduce<64>(t, partial);
 }
 
 // ------------------------------------------------------------------ combine
@@ -1511,7 +1517,13 @@ bool gram_narrow(int mb)
     return on && mb <= kGNarrowB;
 }
 
-int gram_rows() { return g_gram.rows; }
+int gram_task_rows(long long N, bool narrow)
+{
+    if (narrow) return kGRowsNarrow;
+    int rows = g_gram.rows;
+    while (rows / 2 >= kGRowsMin && (rows / 2) % 256 == 0 && (N + rows - 1) / rows < kGramFill) rows /= 2;
+    return rows;
+}
 
 int gram_blocks_per_chunk(int ma, int mb)
 {
@@ -1535,11 +1547,9 @@ void bd_gram(const GramTask *d_tasks, int ntasks, int max_blocks, int max_blocks
     else
         hipLaunchKernelGGL(gram_kernel<1>, dim3(max_blocks, ntasks), dim3(kT), 0, s, d_tasks, d_partial);
     if (reduce) {
-        auto grid = [&](int L) { return dim3((max_mamb + kT / L - 1) / (kT / L), ntasks); };
-        if (max_nch <= kGramPartMax)
-            hipLaunchKernelGGL(gram_reduce_kernel<8>, grid(8), dim3(kT), 0, s, d_tasks, d_partial);
-        else
-            hipLaunchKernelGGL(gram_reduce_kernel<64>, grid(64), dim3(kT), 0, s, d_tasks, d_partial);
+        const int L = max_nch <= kGramPartMax ? 8 : 64;
+        hipLaunchKernelGGL(gram_reduce_kernel, dim3((max_mamb + kT / L - 1) / (kT / L), ntasks), dim3(kT), 0, s,
+                           d_tasks, d_partial);
     }
     PC_HIP(hipGetLastError());
 }

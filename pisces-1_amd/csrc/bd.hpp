@@ -191,13 +191,16 @@ constexpr int kGRowsValu = 256 * 32; // VALU variant: rows per chunk (32 per thr
 // three lanes: 544 against 535 solves/s; 2048 rows: 538).
 constexpr int kGNarrowA = 8, kGNarrowB = 4, kGRowsNarrow = 256 * 16;
 bool gram_narrow(int mb);
-// A launch with fewer than kGramFill workgroups at these sizes halves its rows
-// per workgroup until it has them, down to kGRowsMin.  Two workgroups a CU: one
-// 64^3 instance made 64 of 4096 rows, and its launches left three CUs of four
-// idle (matrix-core kernel 70.2 us; 256 workgroups of 1024 rows 30.0 us).  The
-// block solve of one (H2O)24 64^3 instance: 26.7 ms at 4096 rows, 22.9 at 2048,
-// 21.4 at 1024, 21.5 at 512, 22.3 at 256 (each chunk is a partial sum to be
-// added up).  A batch that fills the chip keeps the configured rows.
+// A task's rows per chunk follow from its own N alone (gram_task_rows), so that
+// a request's sums are the same to the bit whatever else is in the launch.  A
+// task of the configured variant halves its rows until it has kGramFill chunks,
+// down to kGRowsMin: one 64^3 instance at 4096 rows made 64 workgroups, and its
+// launches left three CUs of four idle (matrix-core kernel 70.2 us; 256
+// workgroups of 1024 rows 30.0 us).  Narrow tasks have cpb workgroups a chunk and
+// keep kGRowsNarrow.  ms at rows of wide / narrow tasks 4096 / 4096, 1024 / 4096,
+// 1024 / 1024: the block solve of one (H2O)24 64^3 instance 30.4, 23.8, 23.8, of
+// one (H2O)16 48^3 14.7, 10.6, 10.6; the served batch of 32 (FP32 columns) 55.2,
+// 54.6, 58.8.
 constexpr int kGramFill = 512, kGRowsMin = 1024;
 // chunks per entry up to which the small factor kernels sum them themselves
 // (eight loads by eight lanes); with more the reduction kernel does, 4.7 us
@@ -210,7 +213,8 @@ void gram_set(int variant, int rows);
 void gram_load_config();
 int gram_config(int *rows);
 int gram_variant();
-int gram_rows();
+// rows per chunk of a task of N rows (narrow: gram_narrow(mb))
+int gram_task_rows(long long N, bool narrow);
 int gram_blocks_per_chunk(int ma, int mb);
 constexpr int kBdResChunk = 1024; // rows per residual chunk
 // rows per Ritz workgroup for block size k (RitzTask::nch = ceil(N / ritz_rows(k)))

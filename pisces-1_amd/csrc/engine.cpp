@@ -332,20 +332,11 @@ struct GramBatch {
     {
         part = 0;
         max_blocks = max_blocks_narrow = max_nch = 0;
-        // workgroups at the configured rows; too few of them are made more
-        long long wg = 0;
         for (int i = 0; i < n; ++i) {
             GramTask &t = h[i];
             t.kind = gram_narrow(t.mb) ? 1 : 0;
-            t.rows = t.kind ? kGRowsNarrow : gram_rows();
             t.cpb = t.kind ? (t.ma + kGNarrowA - 1) / kGNarrowA : gram_blocks_per_chunk(t.ma, t.mb);
-            wg += (t.N + t.rows - 1) / t.rows * t.cpb;
-        }
-        int half = 0;
-        while ((wg << half) < kGramFill && half < 4) ++half;
-        for (int i = 0; i < n; ++i) {
-            GramTask &t = h[i];
-            for (int k = 0; k < half && t.rows / 2 >= kGRowsMin && (t.rows / 2) % 256 == 0; ++k) t.rows /= 2;
+            t.rows = gram_task_rows(t.N, t.kind);
             t.nch = (int)((t.N + t.rows - 1) / t.rows);
             int &mx = t.kind ? max_blocks_narrow : max_blocks;
             mx = std::max(mx, t.nch * t.cpb);
@@ -1072,12 +1063,12 @@ int BdEngine::step_b()
     double *dp = dpart_.as<double>();
     for (int pass = 0; pass < 2; ++pass) {
         // many chunks per entry: a reduction over the whole chip, and the factor
-        // kernels read its sums
+        // kernel of that instance reads its sums
         if (og[pass].max_nch > kGramPartMax) og_red[pass] = true;
         og[pass].reduce = og_red[pass];
         for (int i = 0; i < nc; ++i) {
             const int q = og_idx[pass][i];
-            if (q < 0 || og[pass].max_nch > kGramPartMax) continue;
+            if (q < 0 || og[pass].h[q].nch > kGramPartMax) continue;
             hot[pass][i].part = dp;
             hot[pass][i].part_off = og[pass].h[q].part_off;
             hot[pass][i].nch = og[pass].h[q].nch;
@@ -1085,7 +1076,7 @@ int BdEngine::step_b()
     }
     for (int q = 0; q < n2; ++q) {
         const GramTask &gt = og[0].h[og_idx[0][o2_inst[q]]];
-        const bool red = og[0].max_nch > kGramPartMax;  // sums: one chunk per entry
+        const bool red = gt.nch > kGramPartMax;  // sums: one chunk per entry
         h2t[q].part = red ? gt.out : dp;
         h2t[q].part_off = red ? 0 : gt.part_off;
         h2t[q].nch = red ? 1 : gt.nch;
