@@ -222,7 +222,7 @@ struct ScfTask {
     double *mu, *epc, *work;
     int *info;
 };
-void water_scf_batched_launch(const ScfTask *d_tasks, int ntasks, int max_waters, hipStream_t s);
+void water_scf_batched_launch(const ScfTask *h_tasks, const ScfTask *d_tasks, int ntasks, hipStream_t s);
 // bytes of ScfTask::work (d_work) that a cluster of nw waters needs (0 for small ones)
 size_t water_scf_work_bytes(int nw);
 int water_scf_max_waters();

@@ -234,6 +234,9 @@ template <int NT> struct Scf {
     }
 };
 constexpr int kScfSmall = 640, kScfLarge = 1024;
+// the form of a cluster of ns sites: its order of summation, so never that of
+// another cluster of the launch
+__host__ __device__ inline int scf_threads(int ns) { return ns <= kScfSmall ? kScfSmall : kScfLarge; }
 constexpr double kA2B = 1.0 / 0.52917720859;
 constexpr double kPolO = 1.22 * kA2B * kA2B * kA2B, kPolH = 0.28 * kA2B * kA2B * kA2B;
 
@@ -421,11 +424,12 @@ water_scf_kernel(int nw, const double *__restrict__ sites, double *__restrict__ 
     water_scf_body<NT>(nw, sites, mu_out, epc_out, work, info);
 }
 
-// one cluster per workgroup
+// one cluster per workgroup; clusters of the other form are left to its launch
 template <int NT>
 __global__ void __launch_bounds__(NT) water_scf_batched_kernel(const ScfTask *__restrict__ tasks)
 {
     const ScfTask &t = tasks[blockIdx.x];
+    if (scf_threads(3 * t.nw) != NT) return;
     water_scf_body<NT>(t.nw, t.sites, t.mu, t.epc, t.work, t.info);
 }
 
@@ -487,23 +491,26 @@ template <int NT> size_t scf_work_bytes(int ns)
 int water_scf_max_waters() { return kScfLarge / 3; }
 int potential_max_sites() { return kMaxSites; }
 
-// for either form: a batch takes the one its largest cluster needs
 size_t water_scf_work_bytes(int nw)
 {
-    const size_t l = scf_work_bytes<kScfLarge>(3 * nw);
-    return 3 * nw > kScfSmall ? l : std::max(l, scf_work_bytes<kScfSmall>(3 * nw));
+    return scf_threads(3 * nw) == kScfSmall ? scf_work_bytes<kScfSmall>(3 * nw) : scf_work_bytes<kScfLarge>(3 * nw);
 }
 
-void water_scf_batched_launch(const ScfTask *d_tasks, int ntasks, int max_waters, hipStream_t s)
+// a launch per form that the batch holds, its LDS sized by the form's largest cluster
+void water_scf_batched_launch(const ScfTask *h_tasks, const ScfTask *d_tasks, int ntasks, hipStream_t s)
 {
-    if (ntasks <= 0) return;
-    const int ns = 3 * max_waters;
-    if (ns <= kScfSmall)
+    int small = 0, large = 0;  // sites of the largest cluster of each form
+    for (int i = 0; i < ntasks; ++i) {
+        const int ns = 3 * h_tasks[i].nw;
+        int &m = scf_threads(ns) == kScfSmall ? small : large;
+        m = std::max(m, ns);
+    }
+    if (small)
         hipLaunchKernelGGL((water_scf_batched_kernel<kScfSmall>), dim3(ntasks), dim3(kScfSmall),
-                           scf_lds_bytes<kScfSmall>(ns), s, d_tasks);
-    else
+                           scf_lds_bytes<kScfSmall>(small), s, d_tasks);
+    if (large)
         hipLaunchKernelGGL((water_scf_batched_kernel<kScfLarge>), dim3(ntasks), dim3(kScfLarge),
-                           scf_lds_bytes<kScfLarge>(ns), s, d_tasks);
+                           scf_lds_bytes<kScfLarge>(large), s, d_tasks);
     PC_HIP(hipGetLastError());
 }
 
@@ -513,7 +520,7 @@ void water_scf_launch(int nw, const double *d_sites, double *d_mu, double *d_epc
     PC_REQUIRE(nw > 0 && nw <= water_scf_max_waters(), PISCES_ERR_UNSUPPORTED,
                "too many waters for the dipole solve");
     const int ns = 3 * nw;
-    if (ns <= kScfSmall)
+    if (scf_threads(ns) == kScfSmall)
         hipLaunchKernelGGL((water_scf_kernel<kScfSmall>), dim3(1), dim3(kScfSmall),
                            scf_lds_bytes<kScfSmall>(ns), s, nw, d_sites, d_mu, d_epc, d_work, d_info);
     else

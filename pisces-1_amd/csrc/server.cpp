@@ -291,14 +291,12 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
     unsigned char *d = sv->s_up.as<unsigned char>(), *w = sv->s_wk.as<unsigned char>();
     ScfTask *scf = reinterpret_cast<ScfTask *>(h);
     PotTask *pot = reinterpret_cast<PotTask *>(h + align256(sizeof(ScfTask) * nb));
-    int max_nw = 0;
     for (int i = 0; i < nb; ++i) {
         Prep &r = batch[i];
         auto cp = [&](size_t off, const void *src, size_t bytes) {
             if (bytes) std::memcpy(h + off, src, bytes);
         };
         const int nw = r.p->req.nw, nion = r.p->req.nion;
-        max_nw = std::max(max_nw, nw);
         cp(r.o_sites, r.sites.data(), sizeof(double) * r.sites.size());
         cp(r.o_ent, r.ent.data(), sizeof(PotSite) * r.ent.size());
         cp(r.o_rep, r.rep.data(), sizeof(double) * r.rep.size());
@@ -328,7 +326,7 @@ void build_potentials(pisces_server *sv, std::vector<Prep> &batch)
     PC_HIP(hipMemcpyAsync(d, h, up, hipMemcpyHostToDevice, sv->stream));
     {
         ProfScope ps(PK_SCF, sv->stream, 0.0);
-        water_scf_batched_launch(reinterpret_cast<const ScfTask *>(d), nb, max_nw, sv->stream);
+        water_scf_batched_launch(scf, reinterpret_cast<const ScfTask *>(d), nb, sv->stream);
     }
     {
         double bytes = 0;  // V written in FP64 and FP32, read once more with diag H written

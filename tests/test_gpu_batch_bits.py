@@ -38,3 +38,39 @@ def test_same_bits_alone_and_in_the_mix(pisces, precision):
         np.testing.assert_array_equal(r["resid"], mix[i]["resid"])
         np.testing.assert_array_equal(sv.vectors(i), vecs[i])
     sv.close()
+
+
+@pytest.mark.parametrize("large", [214, 250])
+def test_small_clusters_beside_a_large_one(pisces, large):
+    """Dipoles of a batch whose largest cluster takes the 1024-thread form (above
+    640 sites): the others keep theirs, with pairs in registers, LDS and memory,
+    and give the bits they give without it; each agrees with its own potential
+    built and solved singly."""
+    import workload
+    n, L = (12, 11, 12), (44.0, 44.0, 44.0)
+    nws = [3, 27, 107, 213]
+    xyz = {nw: workload.water_cluster(nw, max(3.0, 2.3 * nw ** (1 / 3)), 900 + nw)[0] for nw in nws + [large]}
+
+    def serve(sizes):
+        sv = pisces.Server(hbm_cap_bytes=8 << 30, max_slots=8, precision=pisces.FP64, ptol=9)
+        for nw in sizes:
+            sv.submit(n, L, xyz[nw], 1)
+        res = {r["id"]: r for r in sv.run_until_done()}
+        sv.close()
+        return [res[i] for i in range(len(sizes))]
+
+    print("batch", nws, large, flush=True)
+    without, with_large = serve(nws), serve(nws + [large])
+    for nw, r in zip(nws + [large], with_large):
+        assert r["status"] == 1
+        with pisces.Context(n, L) as ctx:
+            _, _, rc = ctx.build_cluster_potential(xyz[nw])
+            assert rc == 0
+            one = ctx.solve(1, pisces.start_vectors(ctx, 1), maxsub=20, maxmacro=200, ptol=9, corrflag=1)
+        assert one["nconv"] == 1
+        # residuals of 1e-9 put either eigenvalue within 1e-9 of the level
+        assert abs(r["evals"][0] - one["evals"][0]) <= 2e-9
+    for a, b in zip(without, with_large):
+        assert a["n_iter"] == b["n_iter"]
+        np.testing.assert_array_equal(a["evals"], b["evals"])
+        np.testing.assert_array_equal(a["resid"], b["resid"])
