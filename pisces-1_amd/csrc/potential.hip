@@ -310,7 +310,8 @@ __device__ __forceinline__ void water_scf_body(int nw, const double *__restrict_
     for (int u = 0; u < HELD; ++u) {
         const int j = part + (u << lg), jj = j < ns ? j : 0;
         const f64x2 c = pair(j);
-        const double sa = sqrt(c[0]);
+        // a is the rounding of its factor, either sign, between sites that nearly coincide
+        const double sa = sqrt(c[0] < 0.0 ? 0.0 : c[0]);
         sx[u] = sa * (xi - px[3 * jj]);
         sy[u] = sa * (yi - px[3 * jj + 1]);
         sz[u] = sa * (zi - px[3 * jj + 2]);
