@@ -833,7 +833,7 @@ __global__ void __launch_bounds__(kEigT) eig_kernel(const EigTask *__restrict__ 
                 rot[wave][lane] = f64x2{c, s};
             }
             any |= __any(s != 0.0) != 0;
-            __builtin_amdgcn_wave_barrier();  // the wave's LDS operations stay in order
+            wave_lds_sync();
 #pragma unroll
             for (int x = 0; x < kNB; ++x) {
                 if (tid + kEigT * x >= nblock) break;

@@ -82,6 +82,16 @@ __device__ __forceinline__ double row_sum(double x)
     return dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(x))));
 }
 
+// Between a wave's writes to LDS and its lanes' reads of each other's: the
+// hardware runs a wave's LDS operations in order, and this keeps the compiler
+// from moving them across (no instruction, no wait).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // lane l's value of x, uniform over the wave
 __device__ __forceinline__ double lane_value(double x, int l)
 {

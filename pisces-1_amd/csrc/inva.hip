@@ -130,6 +130,7 @@ inva_step_kernel(const double *__restrict__ In_, double *__restrict__ Out_, int 
 #pragma unroll
         for (int r = 0; r < 4; ++r) Ws[wave][lq + 4 * r][l16] = D[lq + 4 * r][l16];
     }
+    wave_lds_sync();
     double a[4];  // -A_iK D, or D in row block K, in A form
 #pragma unroll
     for (int s = 0; s < 4; ++s) a[s] = Ws[wave][l16][4 * s + lq];
