@@ -1086,6 +1086,7 @@ __global__ void __launch_bounds__(kT) ritz_reduce_kernel(const RitzTask *__restr
 // sums are loaded in groups of eight, and a factorisation runs on one wave
 // without a barrier.  (H2O)24 64^3, one wave per task against four: FP64 block
 // of 8, 32.6 -> 12.8 us; both rounds of a block of 4 (orth2), 40.8 -> 25.4 us.
+// (A factor without products, cholinv, keeps one wave.)
 constexpr int kOT = 256;
 
 // [V | T]^T T (ma x nt) from its chunk partials (fixed order per entry), handed
@@ -1101,22 +1102,22 @@ __device__ __forceinline__ void part_sums(const double *part, long long part_off
     }
 }
 
-// Cholesky with dropping of the nt x nt matrix A (LDS, ld kBdMaxK, lower
-// triangle read), then W = L^{-T} (upper triangular, zero columns for dropped
-// ones).  Column j is kept if kin[j] (null: all) and its pivot exceeds
+// Cholesky with dropping of the nt x nt matrix A (leading dimension lda, lower
+// triangle read), then W = L^{-T} (ld ldw, upper triangular, zero columns for
+// dropped ones).  Column j is kept if kin[j] (null: all) and its pivot exceeds
 // tol * dref[j * dstep].  Called by all threads; wave 0 does the work with row
-// i of A and L, then column i of W, in the registers of lane i, and leaves W
-// and keep in LDS after a barrier.
-__device__ __forceinline__ void chol_winv(const double *A, const double *dref, int dstep, int nt,
-                                          const int *kin, double tol, double *W, int *keep)
+// i of A and L, then column i of W, in the registers of lane i, and has written
+// W and keep after the barrier.  K >= nt; PA, PW: pointers to LDS or global memory.
+template <int K = kBdMaxK, typename PA, typename PW>
+__device__ __forceinline__ void chol_winv(PA A, int lda, PA dref, int dstep, int nt, const int *kin,
+                                          double tol, PW W, int ldw, int *keep)
 {
-    constexpr int K = kBdMaxK;
     if (threadIdx.x < 64) {
         const int l = threadIdx.x;
         const bool in = l < nt;
         double a[K];
 #pragma unroll
-        for (int j = 0; j < K; ++j) a[j] = (in && j <= l && j < nt) ? A[l + K * j] : 0.0;
+        for (int j = 0; j < K; ++j) a[j] = (in && j <= l && j < nt) ? A[l + lda * j] : 0.0;
         const double dr = in ? dref[l * dstep] : 0.0;
         const int ki = (in && kin) ? kin[l] : 1;
         unsigned kept = 0;
@@ -1156,7 +1157,7 @@ __device__ __forceinline__ void chol_winv(const double *A, const double *dref, i
         if (in) {
 #pragma unroll
             for (int i = 0; i < K; ++i)
-                if (i < nt) W[i + K * l] = w[i];
+                if (i < nt) W[i + ldw * l] = w[i];
             keep[l] = kl ? 1 : 0;
         }
     }
@@ -1200,7 +1201,7 @@ __device__ __forceinline__ void orth_factor(const double *__restrict__ hg, int h
         S[i + K * j] = v;
     }
     __syncthreads();
-    chol_winv(S, Gs, K + 1, nt, kin, tol, W, keep);
+    chol_winv(S, K, Gs, K + 1, nt, kin, tol, W, K, keep);
     double dev = 0.0;  // max |W - I|, |F| over this thread's entries
     for (int idx = tid; idx < nt * nt; idx += kOT) {
         const int i = idx % nt, c = idx / nt;
@@ -1280,7 +1281,7 @@ __global__ void __launch_bounds__(kOT) orth2_kernel(const Orth2Task *__restrict_
         }
         s_alg = ok;
     }
-    chol_winv(A, dref, 1, nt, nullptr, t.tol1, W1, keep1);
+    chol_winv(A, K, dref, 1, nt, nullptr, t.tol1, W1, K, keep1);
     const bool alg = s_alg != 0;  // written before chol_winv's barriers
     // F1 = -h0 W1; P = h0 W1 (kept in h1 for now)
     for (int idx = tid; idx < m * nt; idx += kOT) {
@@ -1348,7 +1349,7 @@ __global__ void __launch_bounds__(kOT) orth2_kernel(const Orth2Task *__restrict_
     }
     if (tid < nt) dref[tid] = G1[tid + K * tid];
     __syncthreads();
-    chol_winv(A, dref, 1, nt, keep1, t.tol2, W2, keep2);
+    chol_winv(A, K, dref, 1, nt, keep1, t.tol2, W2, K, keep2);
     // W = W1 W2 (into W1's place: Wm), F = (F1 - h1) W2 (into F1's place)
     __shared__ double Wm[K * K];
     for (int idx = tid; idx < nt * nt; idx += kOT) {
@@ -1417,10 +1418,23 @@ __global__ void __launch_bounds__(kOT) orth_kernel(const OrthTask *__restrict__ 
                 t.tol, t.skip, t.skip_tol, t.part, t.part_off, t.nch);
 }
 
-__global__ void __launch_bounds__(kOT) cholinv_batched_kernel(const CholTask *__restrict__ tasks)
+// The factor alone: no products to spread, so one wave, from memory to memory,
+// with code for its size (a launch's time is the fetch of cold code, its loads and
+// the chain of square roots and divisions).  us a launch with one wave in LDS,
+// four waves in the registers of the 16-column form, and so: blocks of 4 5.2,
+// 6.8, 4.2; of 8 and 4 in equal parts 8.0, 10.8, 5.5.
+__global__ void __launch_bounds__(64) cholinv_batched_kernel(const CholTask *__restrict__ tasks)
 {
     const CholTask &t = tasks[blockIdx.x];
-    orth_factor(nullptr, 0, t.G, t.k, 0, t.k, t.W, nullptr, t.keep_in, t.keep_out, t.keep_copy, t.tol);
+    __shared__ int keep[kBdMaxK];
+    const gptr<const double> G = glb(t.G);
+    if (t.k <= 4) chol_winv<4>(G, t.k, G, t.k + 1, t.k, t.keep_in, t.tol, glb(t.W), t.k, keep);
+    else if (t.k <= 8) chol_winv<8>(G, t.k, G, t.k + 1, t.k, t.keep_in, t.tol, glb(t.W), t.k, keep);
+    else chol_winv<kBdMaxK>(G, t.k, G, t.k + 1, t.k, t.keep_in, t.tol, glb(t.W), t.k, keep);
+    if ((int)threadIdx.x < t.k) {
+        t.keep_out[threadIdx.x] = keep[threadIdx.x];
+        if (t.keep_copy) t.keep_copy[threadIdx.x] = keep[threadIdx.x];
+    }
 }
 
 // ------------------------------------------------------------------ correction
@@ -1693,7 +1707,7 @@ void bd_precond(const PrecTask *d_tasks, int ntasks, long long max_N, hipStream_
 void bd_cholinv(const CholTask *d_tasks, int ntasks, hipStream_t s)
 {
     if (ntasks <= 0) return;
-    hipLaunchKernelGGL(cholinv_batched_kernel, dim3(ntasks), dim3(kOT), 0, s, d_tasks);
+    hipLaunchKernelGGL(cholinv_batched_kernel, dim3(ntasks), dim3(64), 0, s, d_tasks);
     PC_HIP(hipGetLastError());
 }
 
