@@ -75,6 +75,11 @@ unsigned pisces_debug_hx_spin_timeouts(void);
  * Errors: PISCES_ERR_ARG, PISCES_ERR_NUMERIC (singular; for method 1 also not
  * positive definite). */
 int pisces_debug_sym_inverse(int n, const double *a, int method, double *inv);
+/* Lowest eigenvalue w and its unit eigenvector v of a symmetric n x n matrix as
+ * the one-root pisces_solve takes them of its projected matrix (dsyev in the
+ * reference, src/Davidson.cpp:224).  Host arithmetic, no device needed.
+ * Errors: PISCES_ERR_ARG. */
+int pisces_debug_lowest_eigenpair(int n, const double *a, double *w, double *v);
 
 /* Launch timing: when enabled, the solver brackets each of its batched launch
  * families with HIP events on the stream they run on and accumulates time,

@@ -967,6 +967,16 @@ int pisces_debug_sym_inverse(int n, const double *a, int method, double *inv)
     });
 }
 
+// test hook: the projected eigensolve of the one-root solve (no device work)
+int pisces_debug_lowest_eigenpair(int n, const double *a, double *w, double *v)
+{
+    return guarded([&] {
+        PC_REQUIRE(n > 0 && a && w && v, PISCES_ERR_ARG, "pisces_debug_lowest_eigenpair: bad arguments");
+        lowest_eigenpair(n, a, n, *w, v);
+        return PISCES_OK;
+    });
+}
+
 // test hook: the H*X kernels of one context (0 VALU, 1 matrix cores, 2 matrix
 // cores with every form in its multi-launch shape, 3 matrix cores with the
 // split-BF16 H*X and preconditioner in their one-launch XCD-ordered form)

@@ -629,14 +629,15 @@ void lowest_eigenpair(int n, const double *A, int lda, double &w, double *v)
         for (int i = 0; i <= j; ++i) a[(size_t)i * n + j] = a[(size_t)j * n + i] = A[i + (size_t)lda * j];
     for (int i = 0; i < n; ++i) q[(size_t)i * n + i] = 1.0;  // rows: the transposed basis
     for (int k = 0; k + 2 < n; ++k) {
-        // reflect rows and columns k+1.. so that column k ends at row k+1
-        double norm2 = 0.0;
+        // reflect rows and columns k+1.. so that column k ends at row k+1; what lies
+        // below is summed by itself: beside the first entry it may be lost in rounding
+        double tail2 = 0.0;
         for (int i = k + 1; i < n; ++i) {
             x[i] = a[(size_t)i * n + k];
-            norm2 += x[i] * x[i];
+            if (i > k + 1) tail2 += x[i] * x[i];
         }
-        const double tail2 = norm2 - x[k + 1] * x[k + 1];
         if (!(tail2 > 0.0)) continue;
+        const double norm2 = x[k + 1] * x[k + 1] + tail2;
         const double alpha = x[k + 1] > 0.0 ? -std::sqrt(norm2) : std::sqrt(norm2);
         const double beta = 1.0 / (norm2 - x[k + 1] * alpha);  // 2 / |x - alpha e|^2
         x[k + 1] -= alpha;

@@ -172,6 +172,18 @@ def sym_inverse(a, method=0):
     return out
 
 
+def lowest_eigenpair(a):
+    """Lowest eigenvalue and unit eigenvector of a symmetric matrix by the
+    one-root solve's host routine (pisces_debug_lowest_eigenpair)."""
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    if a.ndim != 2 or a.shape[0] != a.shape[1]:
+        raise ValueError("a square matrix expected")
+    w, v = ctypes.c_double(), np.empty(a.shape[0])
+    check(lib().pisces_debug_lowest_eigenpair(a.shape[0], _p(a), ctypes.byref(w), _p(v)),
+          "pisces_debug_lowest_eigenpair")
+    return w.value, v
+
+
 def noalloc_scratch_bytes():
     L = lib()
     L.pisces_noalloc_scratch_bytes.restype = ctypes.c_size_t

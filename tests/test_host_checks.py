@@ -1,6 +1,6 @@
 """Host-side logic of the library that runs without a GPU: the polarization
-matrix inverse behind PolType 3 (both of its methods), the argument checks
-of the PolType 3 potential build's binding and of the bandwidth probes."""
+matrix inverse behind PolType 3 (both of its methods), the projected eigensolve of
+the one-root solve, the argument checks of the PolType 3 potential build's binding and of the bandwidth probes."""
 import numpy as np
 import pytest
 
@@ -49,6 +49,41 @@ def test_zero_diagonal_needs_a_pivot(pisces):
     A = np.block([[np.zeros((2, 2)), B], [B.T, np.zeros((2, 2))]])
     out = pisces.sym_inverse(A, 0)
     np.testing.assert_allclose(out @ A, np.eye(4), rtol=0, atol=1e-14)
+
+
+def _eigen_cases():
+    rng = np.random.default_rng(11)
+    for n in (1, 2, 3, 4, 5, 9, 20, 33, 64):
+        a = rng.standard_normal((n, n))
+        yield "random %d" % n, a + a.T
+        # a Davidson subspace: couplings to the first vectors fall off by decades
+        a = np.diag(-0.5 + np.sort(rng.uniform(0, 3, n)))
+        for i in range(n):
+            for j in range(i):
+                a[i, j] = a[j, i] = rng.standard_normal() * 10.0 ** (-0.7 * (i - j)) * 0.3
+        yield "graded %d" % n, a
+    # a coupling far below its column's first one that splits a degenerate level
+    for d in (1e-3, 1e-7, 1e-9, 1e-11):
+        yield "degenerate %g" % d, np.array([[0.0, 1, d], [1, 0, 0], [d, 0, -1]])
+        a = np.diag([0.0, 0, 5, 6, -1, -1])
+        a[0, 1] = a[1, 0] = 1
+        a[0, 4] = a[4, 0] = d
+        a[0, 5] = a[5, 0] = -2 * d
+        yield "degenerate six %g" % d, a
+    yield "diagonal", np.diag([3.0, -2, 5, -2, 0])
+    yield "zero", np.zeros((4, 4))
+
+
+@pytest.mark.parametrize("name,a", list(_eigen_cases()), ids=lambda x: x if isinstance(x, str) else "")
+def test_lowest_eigenpair(pisces, name, a):
+    w, v = pisces.lowest_eigenpair(a)
+    n = len(a)
+    ref = np.linalg.eigvalsh(a)
+    # backward stable: some ten roundings a row of the matrix's norm
+    tol = 20 * n * 2.0 ** -53 * max(np.abs(ref).max(), 1e-300)
+    assert abs(w - ref[0]) <= tol
+    assert abs(np.linalg.norm(v) - 1) <= 20 * n * 2.0 ** -53
+    assert np.linalg.norm(a @ v - w * v) <= 2 * tol
 
 
 def test_singular_matrix_is_an_error(pisces):
