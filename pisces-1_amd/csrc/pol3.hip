@@ -203,12 +203,13 @@ void pol3_grid_launch(const Pol3Dev &D, int nx, int ny, int nz, const double *d_
     // with the threads below: 359 / 3377, 341 / 3311, 381 / 3325.
     const char *rb_e = std::getenv("PISCES_POL3_RB");  // read per build: not a hot path
     const int rb_env = rb_e ? std::atoi(rb_e) : 0;
-    // threads per workgroup (PISCES_POL3_NT = 256, 512 or 1024): with 32-point
-    // tiles 512 / 1024 threads take 341 / 400 us at 216 dimensions (two
-    // workgroups a CU fit) and 3655 / 3311 us at 405 (one does): 1024 from 24
-    // column blocks on.
+    // threads per workgroup (PISCES_POL3_NT = 256, 512 or 1024): 512 as long as
+    // the LDS of two workgroups with 32-point tiles fits a CU (19 column blocks),
+    // 1024 beyond.  us at 64^3, 512 / 1024 threads, by column blocks (waters): 14
+    // (24) 332 / 399, 18 (32) 506 / 572, 19 (33) 556 / 638, 20 (34) 750 / 690, 23 (40)
+    // 937 / 876, 26 (45) 1157 / 1045, 36 (64) 2075 / 1851; the same line at 48^3.
     const char *nt_e = std::getenv("PISCES_POL3_NT");
-    const int nt_v = nt_e ? std::atoi(nt_e) : (D.n3p / 16 >= 24 ? 1024 : 512);
+    const int nt_v = nt_e ? std::atoi(nt_e) : (D.n3p / 16 >= 20 ? 1024 : 512);
     const int nt = (nt_v == 256 || nt_v == 1024) ? nt_v : 512;
     const size_t row = (size_t)(D.n3p + 1) * sizeof(double);
     int rb = (rb_env == 1 || rb_env == 2 || rb_env == 4) ? rb_env : 2;

@@ -27,11 +27,14 @@ namespace {
 constexpr int kPotThreads = 256;
 constexpr int kMaxSites = 1024;
 // Points of a thread: 2 from kPotTwo points a launch on, 1 below, where the waves
-// would be too few to cover the entries' loads.  us, 1 / 2 points: one 24-water
-// 64^3 grid (262144 points) 68 / 74, 45 waters 96^3 (884736) 300 / 253, 32
-// grids of 24 waters 64^3 in one launch 1590 / 1279; 4 points: 97, 273, 1269.
-// (Eleven distances a water and one point: 98, 358, 2505.)
-constexpr long long kPotTwo = 524288;
+// would be too few to cover the entries' loads.  us, 1 / 2 points, at 8, 24 and 45
+// waters: 64^3 (262144 points) 26.4 / 28.4, 70.2 / 75.9, 126 / 132; 72 x 64^2
+// (294912) 30.5 / 30.8, 80.4 / 81.7, 145 / 147; 72^3 (373248) 34.8 / 32.0, 92.3 /
+// 83.9, 167 / 152; 80^3 (512000) 44.6 / 38.4, 119 / 103, 214 / 186; 96^3 70.0 /
+// 59.3, 194 / 164, 354 / 295; 32 grids of 24 waters 64^3 in one launch 1590 / 1279.
+// Four points at 64^3, 96^3 and the 32 grids: 97, 273, 1269.  (Eleven distances a
+// water and one point: 98, 358, 2505.)
+constexpr long long kPotTwo = 327680;
 int pot_points(long long points) { return points >= kPotTwo ? 2 : 1; }
 
 __device__ inline double reff(double r, double r0)
