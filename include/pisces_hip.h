@@ -103,7 +103,11 @@ int pisces_tuning_gram(int *variant, int *rows);
  * of length L[3] (bohr), centred at the origin; computes the 1-D grids and
  * kinetic matrices (sine_dvr, src/sine_dvr.cpp:45-131) and uploads them.
  * Replaces DVR::SetupDVR for DVRType 0 (src/DVR.cpp:64-161, :524-651).
- * device: HIP device ordinal. */
+ * device: HIP device ordinal.
+ * Solves, potential builds and gradients keep the device buffers they needed
+ * with the context, grown to the largest call, until it is destroyed: a solve its
+ * subspace, a gradient about 60 MB and one vector, a potential build its tables
+ * (also pinned on the host) and up to 17 MB for the induced dipoles. */
 int pisces_create(pisces_ctx **ctx, const int n[3], const double L[3], int device);
 /* The same with the DVR type of DVR::SetupDVR (src/DVR.h:56-91, `type`):
  * 0 the sine DVR (as pisces_create); 1 the harmonic-oscillator DVR (ho_dvr,

@@ -1234,9 +1234,8 @@ __device__ __forceinline__ void orth_factor(const double *__restrict__ hg, int h
     }
 }
 
-// S is written one column at a time (rows 0 .. of the basis it then had), so
-// only its upper triangle is current: S(a, b) = S[min + lds * max]
-
+// S is written one column at a time (rows 0 .. of the basis it then had), so only
+// its upper triangle is read
 __global__ void __launch_bounds__(kOT) orth2_kernel(const Orth2Task *__restrict__ tasks)
 {
     constexpr int K = kBdMaxK, M = kBdMaxM;

@@ -45,9 +45,10 @@ void jd_finish(double *C, const double *J, long long ldc, long long N, int k,
 void cholinv(const double *d_G, int k, double *d_W, int *d_info, double rel_tol, hipStream_t s);
 void diag_h(const double *V, const double *Tx, const double *Ty, const double *Tz, int nx,
             int ny, int nz, double *D, hipStream_t s);
-// One-root Davidson iteration (one_root.hip): B, Z hold m <= 63 columns (ld N);
-// the dot products of each kernel go to a buffer of one_part_doubles(N).
-constexpr int kOneLd = 66;
+// One-root Davidson iteration (one_root.hip): B, Z hold m <= kOneMaxM columns (ld
+// N); the dot products of each kernel, at most m + 2, go to a buffer of
+// one_part_doubles(N) in rows of kOneLd.
+constexpr int kOneMaxM = 64, kOneLd = kOneMaxM + 2;
 int one_rows(long long N);
 inline size_t one_part_doubles(long long N) { return (size_t)(one_rows(N) + 1) * kOneLd; }
 // C = (Z y - theta B y) / (theta - D); dots: B^T C (m), ||Z y - theta B y||^2,
@@ -55,10 +56,10 @@ inline size_t one_part_doubles(long long N) { return (size_t)(one_rows(N) + 1) *
 void one_ritz(const double *B, const double *Z, const double *D, long long N, int m, const double *y,
               double theta, double *C, double *U, double *ZV, double *part, hipStream_t s);
 // b = C made orthogonal to B (two Gram-Schmidt passes, the first from part_h's
-// B^T C) and normalised, or 0; C is overwritten
+// B^T C) and normalised, or 0; C is overwritten.  m < kOneMaxM: b is column m
 void one_orth(const double *B, long long N, int m, double *C, double *b, double *part_h, double *part_n,
               hipStream_t s);
-// dots: A^T x (m <= 64 columns) and ||x||^2
+// dots: A^T x (m columns) and ||x||^2
 void one_dots(const double *A, long long N, int m, const double *x, double *part, hipStream_t s);
 // out[0 .. n2): sums j0 .. of part2, then n sums from i0 on of part (out: host memory)
 void one_finish(const double *part, long long N, int i0, int n, const double *part2, int j0, int n2,

@@ -67,8 +67,9 @@ __device__ __forceinline__ void sum_rows(const double *__restrict__ part, int ro
 }
 
 struct OneCoef {
-    double y[64], theta;
+    double y[kOneMaxM], theta;
 };
+static_assert(kOneMaxM == 64, "sum_rows: a lane of a wave per sum");
 
 // The RPT rows of a thread; rows past N read row 0 and count as zeros.
 template <int RPT> struct Rows {
@@ -263,8 +264,9 @@ static const double *one_reduce(double *part, int &rows, int n, hipStream_t s)
 void one_ritz(const double *B, const double *Z, const double *D, long long N, int m, const double *y,
               double theta, double *C, double *U, double *ZV, double *part, hipStream_t s)
 {
+    PC_REQUIRE(m >= 1 && m <= kOneMaxM, PISCES_ERR_ARG, "one-root subspace size");
     OneCoef co;
-    for (int a = 0; a < 64; ++a) co.y[a] = a < m ? y[a] : 0.0;
+    for (int a = 0; a < kOneMaxM; ++a) co.y[a] = a < m ? y[a] : 0.0;
     co.theta = theta;
     const dim3 g(one_rows(N)), t(kT);
     if (one_rpt(N) == 1) {
@@ -280,6 +282,7 @@ void one_ritz(const double *B, const double *Z, const double *D, long long N, in
 void one_orth(const double *B, long long N, int m, double *C, double *b, double *part_h, double *part_n,
               hipStream_t s)
 {
+    PC_REQUIRE(m >= 1 && m < kOneMaxM, PISCES_ERR_ARG, "one-root subspace size");
     const dim3 g(one_rows(N)), t(kT);
     int r1 = one_rows(N), r2 = one_rows(N);
     const double *h = one_reduce(part_h, r1, m, s);
@@ -293,6 +296,7 @@ void one_orth(const double *B, long long N, int m, double *C, double *b, double 
 
 void one_dots(const double *A, long long N, int m, const double *x, double *part, hipStream_t s)
 {
+    PC_REQUIRE(m >= 1 && m <= kOneMaxM, PISCES_ERR_ARG, "one-root subspace size");
     const dim3 g(one_rows(N)), t(kT);
     if (one_rpt(N) == 1) hipLaunchKernelGGL((dots1_kernel<1>), g, t, 0, s, A, N, m, x, part);
     else hipLaunchKernelGGL((dots1_kernel<4>), g, t, 0, s, A, N, m, x, part);

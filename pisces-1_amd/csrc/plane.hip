@@ -3,13 +3,14 @@
 // the FP64 and FP32 forms (plane_f.hip).
 //
 // Both operators are sums or products of dense 1-D matrices applied along the
-// axes of the x-fastest grid (g = i + nx*(j + ny*k)).  A workgroup (4 waves)
-// stages one 2-D plane of one vector in LDS -- rows c, columns i, both padded
-// to multiples of 32 -- and contracts it along one or both of its axes:
+// axes of the x-fastest grid (g = i + nx*(j + ny*k)).  A workgroup stages one
+// 2-D plane of one vector in LDS -- rows c, columns i, both padded to multiples of
+// 32 -- and contracts it along one or both of its axes:
 //   along c:  D(c, i) += sum_k Mc[c][k] P[k][i]   (A = Mc from HBM/L2, B = plane)
 //   along i:  D(c, i) += sum_k P[c][k] Mi[k][i]   (A = plane, B = Mi)
-// on 16 x 16 output tiles, wave w taking tile rows w, w+4, ... and two
-// column tiles at a time (two independent accumulator chains).
+// on 16 x 16 output tiles.  For planes of at most 16 NT points an axis it has NT CS
+// waves: each takes one tile row and, of its columns, one of CS equal parts, two
+// column tiles at a time in the contraction along c (two accumulator chains).
 //
 // Instruction operand layouts (lane l, l16 = l % 16, lq = l / 16):
 //   f64 16x16x4 : A[l16][lq], B[lq][l16], D element r = D[lq + 4r][l16]
@@ -922,12 +923,12 @@ bool one_launch_available()
 }
 
 // The one-launch forms are opt-in (PISCES_HX_FUSED=1, PISCES_FDM_FUSED=1): at
-// 64^3 x 64 vectors they take 0.29 ms (H*X) and 0.43 ms (preconditioner)
-// against 0.086 and 0.129 ms for the multi-launch forms (0.49 and 0.67 ms with
-// one ticket per counter increment).  A ticket's plane takes ~14 us from draw
-// to counted store, and an XCD keeps 64 - 128 of them in flight, where the
-// multi-launch grids keep thousands of planes going; these kernels are bound
-// by that latency, not by the HBM traffic the L2 reuse saves.
+// 64^3 x 64 vectors they take 0.296 ms (H*X) and 0.442 ms (preconditioner)
+// against 0.081 and 0.121 ms for the multi-launch forms.  An XCD keeps 64 tickets
+// (workgroups) in flight, so a ticket of its 1024 (1536) takes about 18 us from
+// draw to counted store, where the multi-launch grids keep thousands of planes
+// going; these kernels are bound by that latency, not by the HBM traffic the L2
+// reuse saves.
 bool hx_fused_enabled()
 {
     static const bool on = [] {

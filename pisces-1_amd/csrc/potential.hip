@@ -215,8 +215,8 @@ potential_grid_batched_kernel(PotParams P, const PotTask *__restrict__ tasks)
 // 256 threads, ten barriers a step) -> now: 24 waters 427 -> 91, 45 waters
 // 1834 -> 313.
 //
-// Two forms: 640 threads (three waves a SIMD, so that 12 pairs fit the registers)
-// up to 640 sites, 1024 threads beyond.
+// Two forms: 640 threads (three waves a SIMD, so that nine pairs fit the
+// registers; twelve spilled) up to 640 sites, 1024 threads (six pairs) beyond.
 template <int NT> struct Scf {
     static constexpr int HELD = NT == 640 ? 9 : 6;      // pairs of a thread in registers
     static constexpr int SLOT_BYTES = NT * 2 * (int)sizeof(double);

@@ -12,7 +12,8 @@
 // orthogonalisation of the corrections is block classical Gram-Schmidt done
 // twice plus a Cholesky QR of the new block (the reference: modified
 // Gram-Schmidt twice, vector by vector), and the small eigenproblem is solved
-// by Jacobi rotations instead of LAPACK dsyev.
+// by Jacobi rotations instead of LAPACK dsyev (one root with the Davidson
+// correction: by tridiagonal QL, in an iteration of its own, solve_one).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
