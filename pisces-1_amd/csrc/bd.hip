@@ -1532,9 +1532,11 @@ bool gram_narrow(int mb)
 
 int gram_task_rows(long long N, bool narrow)
 {
-    if (narrow) return kGRowsNarrow;
-    int rows = g_gram.rows;
-    while (rows / 2 >= kGRowsMin && (rows / 2) % 256 == 0 && (N + rows - 1) / rows < kGramFill) rows /= 2;
+    auto chunks = [&](int rows) { return (N + rows - 1) / rows; };
+    int rows = narrow ? kGRowsNarrow : g_gram.rows;
+    while (rows / 2 >= kGRowsMin && (rows / 2) % 256 == 0 &&
+           (narrow ? chunks(rows / 2) <= kGramNarrowFill : chunks(rows) < kGramFill))
+        rows /= 2;
     return rows;
 }
 

@@ -197,11 +197,15 @@ bool gram_narrow(int mb);
 // down to kGRowsMin: one 64^3 instance at 4096 rows made 64 workgroups, and its
 // launches left three CUs of four idle (matrix-core kernel 70.2 us; 256
 // workgroups of 1024 rows 30.0 us).  Narrow tasks have cpb workgroups a chunk and
-// keep kGRowsNarrow.  ms at rows of wide / narrow tasks 4096 / 4096, 1024 / 4096,
+// halve kGRowsNarrow only as far as kGramNarrowFill chunks.  ms at rows of wide / narrow tasks 4096 / 4096, 1024 / 4096,
 // 1024 / 1024: the block solve of one (H2O)24 64^3 instance 30.4, 23.8, 23.8, of
 // one (H2O)16 48^3 14.7, 10.6, 10.6; the served batch of 32 (FP32 columns) 55.2,
-// 54.6, 58.8.
-constexpr int kGramFill = 512, kGRowsMin = 1024;
+// 54.6, 58.8.  Small grids served, us a step with narrow tasks at 4096 rows / halved
+// up to 32 chunks: one 32^3 212 / 202, 20 of 32^3 361 / 355, 8 of 40^3 (FP64) 382 /
+// 351, 20 of 40^3 431 / 423; up to 64 chunks the last takes 1.03 times longer than
+// up to 32.  (Two FP64 61^3 instances: 325 at 4096 rows, 314 at 1024; eight of 64^3:
+// 33.7 and 34.1 ms a batch.)
+constexpr int kGramFill = 512, kGramNarrowFill = 32, kGRowsMin = 1024;
 // chunks per entry up to which the small factor kernels sum them themselves
 // (eight loads by eight lanes); with more the reduction kernel does, 4.7 us
 constexpr int kGramPartMax = 64;
